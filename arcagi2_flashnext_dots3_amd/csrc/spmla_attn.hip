@@ -40,12 +40,11 @@ constexpr int HGW = NW * HB;          // heads per workgroup
 constexpr int TR = 32;                // rows per tile
 constexpr int KMAX = 2048;            // rows per (token, split): their ids are staged in LDS
 constexpr float TAU = 6.0f;
-// Launches without the in-kernel split merge go to the head-group kernel (spmla_attn_hg.hip: 32 heads per
-// workgroup, each wave streams its own rows, no barrier in the loop, no split merge) while they have at most this
-// many (token, split, 32-head group) work items -- decode batches -- and to fwd_kernel above it (prefill chunks:
+// Launches go to the head-group kernel (spmla_attn_hg.hip: 32 heads per workgroup, each wave streams its own rows, no
+// barrier in the loop; splits merged in the kernel always run there) while they have at most this many (token, split, 32-head group) work items -- decode batches -- and to fwd_kernel above it (prefill chunks:
 // there each row's staging and V^T conversion serve all 128 heads of a token, which pays once the launch fills the
 // GPU with whole tokens). Measured at H = 128, K = 2048: T = 64 (256 items) 69-70 us against 82-84 us for
-// fwd_kernel with 4 splits; T = 256 / 1024: 278 / 909 us against 251 / 796 us for fwd_kernel.
+// fwd_kernel with 4 splits merged; T = 256 / 1024: 278 / 909 us against 251 / 796 us for fwd_kernel.
 constexpr long long HG_TOKENS_MAX = 512;
 
 // LDS map (bytes)
@@ -174,17 +173,7 @@ struct Params {
   // optional prior partial merged into the bf16 output (S == 1): normalized fp32 o and natural-log lse
   const float* prior_o; long long po_st, po_sh;
   const float* prior_lse; long long pl_st;
-  // split merge inside the kernel (S > 1 with the bf16 output): per (token, head group) arrival counters (zero
-  // between launches), per split and head the lse and the partial's exponent, and the f16 partials in the lanes'
-  // order ([split][token][head group][wave][mt][a][lane][4]); null otherwise
-  int* ws_cnt; float* ws_lse; float* ws_exp; uint16_t* ws_o;
 };
-
-// Workspace of the in-kernel split merge (bytes, each part 256-byte aligned).
-__host__ __device__ inline long long ws_align(long long b) { return (b + 255) / 256 * 256; }
-inline long long ws_cnt_bytes(int T, int HG) { return ws_align(4ll * T * HG); }
-inline long long ws_lse_bytes(int T, int HG, int S) { return ws_align(4ll * S * T * HG * HGW); }
-inline long long ws_o_bytes(int T, int HG, int S) { return 2ll * S * T * HG * HGW * D_LAT; }
 
 // Copies of tile jj for wave w: the codes of scale group w of the tile's 32 rows (copy i fills chunks 2 i and 2 i + 1:
 // lane l copies chunk 2 i + l / 32 of row spos(l % 32) to position l % 32), rows 8 w .. 8 w + 7 of the rope tile (lane l
@@ -251,7 +240,7 @@ __device__ inline f16x8 codes8_f16(uint32_t a, uint32_t b) {
 // free); heads >= H are not written.
 constexpr int OROW = 1040;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-static_assert(NW * HB * OROW <= L_IDS, "output staging fits below the flag word");
+static_assert(NW * HB * OROW <= L_TOTAL, "output staging fits the LDS");
 __device__ inline void put_block(SPMLA_LDS uint8_t* reg, int lane, int mt, const float (&v)[16]) {
   const int l32 = lane & 31, hh = lane >> 5;
 #pragma unroll
@@ -269,71 +258,6 @@ __device__ inline void flush_rows(const Params& p, SPMLA_LDS uint8_t* reg, int t
     if (al16) *(u32x4*)dst = v;
     else { *(uint2*)dst = make_uint2(v[0], v[1]); *(uint2*)(dst + 4) = make_uint2(v[2], v[3]); }
   }
-}
-
-// The in-kernel split merge for NS splits, run by the last split to arrive at (token t, head group hg): o = sum_u
-// f[u] * partial_u with f[u] = e^(lse_u - M) kv_scale 2^exp_u / Z (the f16 partials of every split, this one's
-// included), one output block at a time with the next block's loads in flight; lse = M + ln Z.
-template <int NS>
-__device__ inline void merge_splits(const Params& p, SPMLA_LDS uint8_t* reg, int t, int hg, int hbase, int w,
-                                    int lane) {
-  const int l32 = lane & 31, hh = lane >> 5;
-  float lu[NS], f[NS];
-  uint64_t* pu[NS];
-  float lmax = -__builtin_inff();
-#pragma unroll
-  for (int u = 0; u < NS; ++u) {
-    const long long bu = ((long long)u * p.T + t) * p.HG + hg;
-    lu[u] = __builtin_bit_cast(float, __hip_atomic_load((uint32_t*)p.ws_lse + bu * HGW + w * HB + l32,
-                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    f[u] = (float)(int)__hip_atomic_load((uint32_t*)p.ws_exp + bu * HGW + w * HB + l32, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-    pu[u] = (uint64_t*)(p.ws_o + (bu * NW + w) * (16 * 4 * 64 * 4)) + lane;
-    lmax = fmaxf(lmax, lu[u]);
-  }
-  float z = 0.f;
-#pragma unroll
-  for (int u = 0; u < NS; ++u) {
-    lu[u] = lmax > -__builtin_inff() ? expf(lu[u] - lmax) : 0.f;     // exp(-inf) = 0
-    z += lu[u];
-  }
-  const float zi = z > 0.f ? p.kv_scale / z : 0.f;
-#pragma unroll
-  for (int u = 0; u < NS; ++u) f[u] = lu[u] * zi * __builtin_ldexpf(1.f, (int)f[u]);
-  const int h = hbase + l32;
-  if (h < p.H && hh == 0) p.lse[(long long)t * p.lse_st + h] = lmax > -__builtin_inff() ? lmax + logf(z) : lmax;
-  uint64_t x[2][NS][4];
-#pragma unroll
-  for (int u = 0; u < NS; ++u)
-#pragma unroll
-    for (int a = 0; a < 4; ++a) x[0][u][a] = __hip_atomic_load(pu[u] + a * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-  for (int mt = 0; mt < 16; ++mt) {
-    if (mt + 1 < 16) {
-#pragma unroll
-      for (int u = 0; u < NS; ++u)
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-          x[(mt + 1) & 1][u][a] =
-              __hip_atomic_load(pu[u] + ((mt + 1) * 4 + a) * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    float v[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) v[e] = 0.f;
-#pragma unroll
-    for (int u = 0; u < NS; ++u)
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const f16x2_t lo = __builtin_bit_cast(f16x2_t, (uint32_t)x[mt & 1][u][a]);
-        const f16x2_t hi = __builtin_bit_cast(f16x2_t, (uint32_t)(x[mt & 1][u][a] >> 32));
-        v[4 * a] = __builtin_fmaf((float)lo[0], f[u], v[4 * a]);
-        v[4 * a + 1] = __builtin_fmaf((float)lo[1], f[u], v[4 * a + 1]);
-        v[4 * a + 2] = __builtin_fmaf((float)hi[0], f[u], v[4 * a + 2]);
-        v[4 * a + 3] = __builtin_fmaf((float)hi[1], f[u], v[4 * a + 3]);
-      }
-    put_block(reg, lane, mt, v);
-  }
-  flush_rows(p, reg, t, hbase, lane);
 }
 
 __global__ void __launch_bounds__(256, 1) fwd_kernel(Params p) {
@@ -728,56 +652,6 @@ __global__ void __launch_bounds__(256, 1) fwd_kernel(Params p) {
   l_run += half_swap(l_run);
   const float L = l_run;
   float lse_v = L > 0.f ? (m_run + (float)eps + log2f(L)) * 0.69314718055994531f : -__builtin_inff();
-  if (p.ws_o) {                            // ---- split merge in the kernel (all waves reach the barriers)
-    const long long blk = ((long long)s * p.T + t) * p.HG + hg;   // this split's partial
-    if (wact) {
-      // partial o / 2^(eps + 3) in f16: every row scale is <= 2^(9 + eps), so |o| < 448 * 2^(9 + eps) < 2^(18 + eps)
-      const float f = L > 0.f ? __builtin_ldexpf(1.f, -(eps + 3)) / L : 0.f;
-      // agent-scope stores (written through to the device's coherence point: the merging split may run on another
-      // XCD, whose L2 does not see this one's) -- no L2 write-back fence needed
-      uint64_t* po = (uint64_t*)(p.ws_o + (blk * NW + w) * (16 * 4 * 64 * 4)) + lane;
-#pragma unroll
-      for (int mt = 0; mt < 16; ++mt) {
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const uint64_t v = (uint64_t)pk_f16(O[mt][4 * a] * f, O[mt][4 * a + 1] * f) |
-                             ((uint64_t)pk_f16(O[mt][4 * a + 2] * f, O[mt][4 * a + 3] * f) << 32);
-          __hip_atomic_store(po + (mt * 4 + a) * 64, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (hh == 0) {
-        __hip_atomic_store((uint32_t*)p.ws_lse + blk * HGW + w * HB + l32, __builtin_bit_cast(uint32_t, lse_v),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store((uint32_t*)p.ws_exp + blk * HGW + w * HB + l32, (uint32_t)(eps + 3), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0);         // every store of the partial has completed before it is counted
-    __syncthreads();
-    SPMLA_LDS int* flag = (SPMLA_LDS int*)(lds + L_IDS);
-    if (tid == 0) {
-      int* cnt = p.ws_cnt + (long long)t * p.HG + hg;
-      const int old = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const bool last = old == p.S - 1;
-      if (last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
-      *flag = last;
-    }
-    __syncthreads();
-    if (!*flag) return;                    // another split merges this token's heads
-    if (!wact) return;                     // (the merge reads the partials with agent-scope loads)
-    SPMLA_LDS uint8_t* reg = lds + w * HB * OROW;
-    switch (p.S) {
-      case 2: merge_splits<2>(p, reg, t, hg, hbase, w, lane); break;
-      case 3: merge_splits<3>(p, reg, t, hg, hbase, w, lane); break;
-      case 4: merge_splits<4>(p, reg, t, hg, hbase, w, lane); break;
-      case 5: merge_splits<5>(p, reg, t, hg, hbase, w, lane); break;
-      case 6: merge_splits<6>(p, reg, t, hg, hbase, w, lane); break;
-      case 7: merge_splits<7>(p, reg, t, hg, hbase, w, lane); break;
-      default: merge_splits<8>(p, reg, t, hg, hbase, w, lane); break;
-    }
-    return;
-  }
   if (!wact) return;
   float inv = L > 0.f ? p.kv_scale / L : 0.f;
   float wp = 0.f;                           // weight of the prior partial (merge of two normalized partials)
@@ -906,7 +780,8 @@ int launch_tokens(const void* q, long long q_st, long long q_sh, const void* poo
                   long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                   void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
                   float* lsepart, const float* prior_o, long long po_st, long long po_sh, const float* prior_lse,
-                  long long pl_st, void* stream, bool r576);
+                  long long pl_st, void* ws, void* stream, bool r576);
+long long ws_bytes(int T, int H, int S);
 }  // namespace pk
 }  // namespace spmla
 
@@ -923,23 +798,21 @@ static int attn_launch(const void* q, long long q_st, long long q_sh, const void
   const bool f32part = opart != nullptr;   // fp32 partials (any S) instead of the bf16 output
   const bool fused = !f32part && S > 1;    // bf16 output of S splits merged in the kernel (workspace ws)
   if (f32part ? !lsepart : (!out || !lse)) return SPMLA_EARG;
-  const int HG = (H + attn::HGW - 1) / attn::HGW;
   if (fused) {
     if (!ws || prior_o) return SPMLA_EARG;
     if (S > 8) return SPMLA_ELIMIT;
     if ((uintptr_t)ws & 255) return SPMLA_EALIGN;
-    if (ws_bytes < attn::ws_cnt_bytes(T, HG) + 2 * attn::ws_lse_bytes(T, HG, S) + attn::ws_o_bytes(T, HG, S))
-      return SPMLA_EARG;
+    if (ws_bytes < pk::ws_bytes(T, H, S)) return SPMLA_EARG;
   }
   if (((uintptr_t)q & 15) || (q_st & 7) || (q_sh & 7) || ((uintptr_t)pool & 15)) return SPMLA_EALIGN;
   if (out && (((uintptr_t)out & 7) || (o_st & 3) || (o_sh & 3))) return SPMLA_EALIGN;
   if (f32part && ((uintptr_t)opart & 15)) return SPMLA_EALIGN;
   const bool kfit = ((K + S - 1) / S + attn::TR - 1) / attn::TR * attn::TR <= attn::KMAX;
-  if (!fused && (!kfit || (long long)T * S * ((H + 31) / 32) <= attn::HG_TOKENS_MAX))
+  if (fused && !kfit) return SPMLA_ELIMIT;
+  if (fused || !kfit || (long long)T * S * ((H + 31) / 32) <= attn::HG_TOKENS_MAX)
     return pk::launch_tokens(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st,
-                             o_sh, lse, lse_st, opart, lsepart, prior_o, po_st, po_sh, prior_lse, pl_st, stream,
-                             false);
-  if (!kfit) return SPMLA_ELIMIT;
+                             o_sh, lse, lse_st, opart, lsepart, prior_o, po_st, po_sh, prior_lse, pl_st,
+                             fused ? ws : nullptr, stream, false);
   attn::Params p;
   p.q = (const uint16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.pool = (const uint8_t*)pool; p.R = R;
@@ -950,17 +823,6 @@ static int attn_launch(const void* q, long long q_st, long long q_sh, const void
   p.out = (uint16_t*)out; p.o_st = o_st; p.o_sh = o_sh; p.lse = lse; p.lse_st = lse_st;
   p.opart = f32part ? opart : nullptr; p.lsepart = lsepart;
   p.prior_o = prior_o; p.po_st = po_st; p.po_sh = po_sh; p.prior_lse = prior_lse; p.pl_st = pl_st;
-  p.ws_cnt = nullptr; p.ws_lse = nullptr; p.ws_exp = nullptr; p.ws_o = nullptr;
-  if (fused) {
-    uint8_t* b = (uint8_t*)ws;
-    p.ws_cnt = (int*)b;
-    b += attn::ws_cnt_bytes(T, HG);
-    p.ws_lse = (float*)b;
-    b += attn::ws_lse_bytes(T, HG, S);
-    p.ws_exp = (float*)b;
-    b += attn::ws_lse_bytes(T, HG, S);
-    p.ws_o = (uint16_t*)b;
-  }
   const long long nwork = (long long)T * S * p.HG;
   if (nwork > (1ll << 30)) return SPMLA_ELIMIT;
   const int grid = (int)((nwork + 7) / 8 * 8);
@@ -981,9 +843,7 @@ int spmla_attn_splitk(const void* q, long long q_st, long long q_sh, const void*
 
 long long spmla_attn_ws_bytes(int T, int H, int S) {
   if (T < 0 || H <= 0 || S <= 0) return -1;
-  if (S == 1) return 0;
-  const int HG = (H + attn::HGW - 1) / attn::HGW;
-  return attn::ws_cnt_bytes(T, HG) + 2 * attn::ws_lse_bytes(T, HG, S) + attn::ws_o_bytes(T, HG, S);
+  return S == 1 ? 0 : pk::ws_bytes(T, H, S);
 }
 
 int spmla_attn(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
@@ -994,21 +854,43 @@ int spmla_attn(const void* q, long long q_st, long long q_sh, const void* pool, 
                      lse_st, nullptr, nullptr, nullptr, 0, 0, nullptr, 0, S > 1 ? ws : nullptr, ws_bytes, stream);
 }
 
-int spmla_attn576(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
+static int attn576_launch(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
                   long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                   void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
-                  float* lsepart, void* stream) {
+                  float* lsepart, void* ws, long long ws_bytes, void* stream) {
   if (T < 0 || H <= 0 || K < 0 || S <= 0 || R < 0) return SPMLA_EARG;
   if (T == 0) return SPMLA_OK;
   if (!q || !idx || (R > 0 && !pool)) return SPMLA_EARG;
   const bool f32part = opart != nullptr;
-  if (f32part ? !lsepart : (S != 1 || !out || !lse)) return SPMLA_EARG;
+  const bool fused = !f32part && S > 1;
+  if (f32part ? !lsepart : (!out || !lse || (fused && !ws))) return SPMLA_EARG;
+  if (fused) {
+    if (S > 8) return SPMLA_ELIMIT;
+    if ((uintptr_t)ws & 255) return SPMLA_EALIGN;
+    if (ws_bytes < pk::ws_bytes(T, H, S)) return SPMLA_EARG;
+  }
   if (((uintptr_t)q & 15) || (q_st & 7) || (q_sh & 7) || ((uintptr_t)pool & 15)) return SPMLA_EALIGN;
   if (out && (((uintptr_t)out & 7) || (o_st & 3) || (o_sh & 3))) return SPMLA_EALIGN;
   if (f32part && ((uintptr_t)opart & 15)) return SPMLA_EALIGN;
   return pk::launch_tokens(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st,
-                           o_sh, lse, lse_st, f32part ? opart : nullptr, lsepart, nullptr, 0, 0, nullptr, 0, stream,
-                           true);
+                           o_sh, lse, lse_st, f32part ? opart : nullptr, lsepart, nullptr, 0, 0, nullptr, 0,
+                           fused ? ws : nullptr, stream, true);
+}
+
+int spmla_attn576(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
+                  long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
+                  void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
+                  float* lsepart, void* stream) {
+  return attn576_launch(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st, o_sh,
+                        lse, lse_st, opart, lsepart, nullptr, 0, stream);
+}
+
+int spmla_attn576_ws(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
+                     long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
+                     void* out, long long o_st, long long o_sh, float* lse, long long lse_st, void* ws,
+                     long long ws_bytes, void* stream) {
+  return attn576_launch(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st, o_sh,
+                        lse, lse_st, nullptr, nullptr, ws, ws_bytes, stream);
 }
 
 int spmla_attn_merge(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,

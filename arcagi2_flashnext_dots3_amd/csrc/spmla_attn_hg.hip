@@ -7,6 +7,11 @@
 //     item = request, columns = tokens x heads; a column's softmax keeps only the rows its token selected (per-row
 //     token masks, ballots). Reference: dotsnote/engine/arcstats_pkg/arcstats/csrc/offload_attn.cu:700-1153
 //     (pk_attn_kernel).
+//   * attn_kernel<false, *, true>, the decode kernel whose S splits of a token's rows merge in the kernel (small
+//     batches: K = 2048, 128 heads, 1 / 8 / 16 / 32 tokens 23.6 / 26.5 / 29.0 / 39.0 us in graphs, against 53 / 54 / 55
+//     / 51 us for 128-head workgroups with f16 partials at up to 8 splits, or unsplit at 32 tokens). A launch that
+//     leaves compute units idle is bound by the serial chain of a wave (12.7 us of prologue and merge, 2.2 us per
+//     tile), so the rows go to more workgroups;
 //   * attn_kernel<false, true>, the same decode over Row576 rows (spmla_attn576: 512 + 64 e4m3 codes, one
 //     per-tensor kv_scale): no per-group scales, so the latent MFMAs run as one chain into S (no scale combine), P'
 //     is P itself in f16 for every group, and the rope codes are widened to bf16 (exact) in registers.
@@ -140,12 +145,90 @@ struct Params {
   // token t0 + (c >> (5 - tsh)) (t0 = cu[t] or t * ql) and head hg * (32 >> tsh) + c % (32 >> tsh); a column's
   // softmax keeps the rows its token selected. T = total tokens (output rows), NR = requests.
   const uint8_t* mk; const int* cu; int ql, tsh, NR;
+  // split merge in the kernel (attn_kernel<false, *, true>): arrival counters, one byte per 32-head group (four groups of
+  // a token to a word, zero between launches), and per split the lse [32 heads] and the normalized fp32 partial in
+  // the lanes' order [16 output blocks][4][64 lanes][4]
+  uint32_t* ws_cnt; float* ws_lse; float* ws_o;
 };
+
+// Workspace of the split merge (bytes): counters (4 per token and 128 heads), lse, partials. Each part 256-byte aligned.
+constexpr int ws_groups(int H) { return (H + HG - 1) / HG; }
+inline long long ws_cnt_bytes(int T, int H) { return (4ll * T * ((H + 127) / 128) + 255) / 256 * 256; }
+inline long long ws_lse_bytes(int T, int H, int S) { return (4ll * S * T * ws_groups(H) * HG + 255) / 256 * 256; }
+long long ws_bytes(int T, int H, int S) {
+  return ws_cnt_bytes(T, H) + ws_lse_bytes(T, H, S) + 4ll * S * T * ws_groups(H) * HG * D_LAT;
+}
+
+// A partial of the split merge ([16 output blocks][4][64 lanes][4] fp32, 64 KiB) as a buffer, read and written with
+// agent scope (sc1): written through to the device's coherence point and read from there, since the merging workgroup
+// may run on another XCD, whose L2 does not see this one's. 16 bytes an access (a 64-bit atomic moves 8).
+constexpr int SC1 = 16;
+constexpr int PART = 16 * 4 * 64 * 4;               // floats
+__device__ inline __amdgpu_buffer_rsrc_t part_rsrc(const Params& p, int u, int t, int hg) {
+  const uint64_t a = (uint64_t)(uintptr_t)(p.ws_o + (((long long)u * p.T + t) * p.HGN + hg) * PART);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)hi << 32) | lo), (short)0, PART * 4, 0x00020000);
+}
+
+// The split merge of (token t, head group hg), run by the 4 waves of the last split to arrive: o = sum_u w_u o_u,
+// w_u = e^(lse_u - M) / Z, lse = M + ln Z over the S splits in order (the same bits whichever split comes last). NS:
+// S rounded up; the loads past S repeat the last split's with weight 0. Wave w takes output blocks 4 w .. 4 w + 3.
+// Bound by the round trip to the coherence point: the lse loads and DEP pieces of every split are in flight together.
+template <int NS>
+__device__ inline void merge_splits(const Params& p, int t, int hg, int w, int lane) {
+  const int half = lane >> 5, l32 = lane & 31, h = hg * HG + l32;
+  float f[NS];
+  constexpr int DEP = NS == 8 ? 6 : 12;               // 1 KiB pieces of every split in flight per wave
+  f32x4 x[DEP][NS];
+  __amdgpu_buffer_rsrc_t r[NS];
+#pragma unroll
+  for (int u = 0; u < NS; ++u) r[u] = part_rsrc(p, min(u, p.S - 1), t, hg);
+  auto load = [&](int i) {                            // piece i = 4 b + qd: output block 4 w + b, columns 8 qd + 4 half ..
+#pragma unroll
+    for (int u = 0; u < NS; ++u)
+      x[i % DEP][u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+          r[u], ((16 * w + i) * 64 + lane) * 16, 0, SC1));
+  };
+#pragma unroll
+  for (int u = 0; u < NS; ++u)
+    f[u] = __builtin_bit_cast(float, __hip_atomic_load(
+        (uint32_t*)p.ws_lse + (((long long)min(u, p.S - 1) * p.T + t) * p.HGN + hg) * HG + l32, __ATOMIC_RELAXED,
+        __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+  for (int i = 0; i < DEP; ++i) load(i);
+  float lmax = -__builtin_inff();
+#pragma unroll
+  for (int u = 0; u < NS; ++u) {
+    if (u >= p.S) f[u] = -__builtin_inff();
+    lmax = fmaxf(lmax, f[u]);
+  }
+  float z = 0.f;
+#pragma unroll
+  for (int u = 0; u < NS; ++u) {
+    f[u] = lmax > -__builtin_inff() ? expf(f[u] - lmax) : 0.f;     // exp(-inf) = 0
+    z += f[u];
+  }
+  const float zi = z > 0.f ? 1.f / z : 0.f;
+  if (w == 0 && half == 0 && h < p.H) p.lse[(long long)t * p.lse_st + h] = z > 0.f ? lmax + logf(z) : -__builtin_inff();
+  uint16_t* orow = p.out + (long long)t * p.o_st + (long long)(h < p.H ? h : 0) * p.o_sh;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < NS; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = __builtin_fmaf(x[i % DEP][u][e], f[u], a[e]);
+    if (i + DEP < 16) load(i + DEP);
+    if (h < p.H)
+      *(uint2*)(orow + 128 * w + 8 * i + 4 * half) =
+          make_uint2(pk_bf16(a[0] * zi, a[1] * zi), pk_bf16(a[2] * zi, a[3] * zi));
+  }
+}
 
 // Source of invalid and padding rows: zero codes, zero scales, zero rope (their P is 0, and 0 * 0 stays 0 in PV).
 __device__ __attribute__((aligned(16))) uint8_t zero_row[ROW656];
 
-template <bool PK, bool R5 = false>
+template <bool PK, bool R5 = false, bool SP = false>
 __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
   constexpr int RB = R5 ? ROW576 : ROW656;      // row bytes
   constexpr int NRP = R5 ? 2 : 4;               // 16-byte rope pieces per lane: e4m3 (32 B) or bf16 (64 B)
@@ -175,11 +258,14 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: scalar control flow
   const int half = lane >> 5, l32 = lane & 31;
 
-  // ---- row range of this split
-  const int kc = ((p.K + p.S - 1) / p.S + TR - 1) / TR * TR;
+  // ---- row range of this split. The splits merged in the kernel share the token's own count (a short list spreads
+  // over all of them); partials handed out are cut at the same places for every token.
+  int kn = p.K, klim = p.K;
+  if (p.kcount) { const int c = p.kcount[t]; klim = klim < c ? klim : c; }
+  if (SP) kn = klim > 0 ? klim : 0;
+  const int kc = ((kn + p.S - 1) / p.S + TR - 1) / TR * TR;
   const int kb = s * kc;
-  int ke = kb + kc < p.K ? kb + kc : p.K;
-  if (p.kcount) { const int c = p.kcount[t]; ke = ke < c ? ke : c; }
+  const int ke = kb + kc < klim ? kb + kc : klim;
   const int nrow = ke > kb ? ke - kb : 0;
   const int ntile = p.R > 0 ? (nrow + TR - 1) / TR : 0;     // no rows to read: o = 0, lse = -inf
 
@@ -609,7 +695,10 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(x[e], fv[v], acc[e]);
         }
-        if (hoval) {
+        if constexpr (SP) {
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc), part_rsrc(p, s, t, hg),
+                                                 ((mt * 4 + qd) * 64 + lane) * 16, 0, SC1);
+        } else if (hoval) {
           const int col = 32 * mt + 8 * qd + 4 * half;      // C-layout rows of values 4qd .. 4qd + 3
           if (p.prior_o) {
             const f32x4 x = *(const f32x4*)(p.prior_o + (long long)t * p.po_st + (long long)ho * p.po_sh + col);
@@ -627,6 +716,28 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
       }
     }
   }
+  if constexpr (SP) {
+    if (w == 0 && half == 0)
+      __hip_atomic_store((uint32_t*)p.ws_lse + (((long long)s * p.T + t) * p.HGN + hg) * HG + l32,
+                         __builtin_bit_cast(uint32_t, lse_v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);         // every store of the partial has completed before it is counted
+    __syncthreads();                       // (and every wave has read the merge's weights: s_ml is free)
+    SPMLA_LDS int* flag = (SPMLA_LDS int*)s_ml;
+    if (tid == 0) {
+      uint32_t* cnt = p.ws_cnt + (long long)t * ((p.H + 127) / 128) + (hg >> 2);
+      const int sh = 8 * (hg & 3);
+      const uint32_t old = __hip_atomic_fetch_add(cnt, 1u << sh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const bool last = (int)((old >> sh) & 255u) == p.S - 1;
+      if (last) __hip_atomic_fetch_sub(cnt, (uint32_t)p.S << sh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *flag = last;
+    }
+    __syncthreads();
+    if (!*flag) return;                    // another split merges this group
+    if (p.S <= 2) merge_splits<2>(p, t, hg, w, lane);
+    else if (p.S <= 4) merge_splits<4>(p, t, hg, w, lane);
+    else merge_splits<8>(p, t, hg, w, lane);
+    return;
+  }
   if (w == 0 && half == 0 && hoval) {
     if (p.opart == nullptr) p.lse[(long long)to * p.lse_st + ho] = lse_v;
     else p.lsepart[((long long)s * p.T + to) * p.H + ho] = lse_v;
@@ -641,7 +752,7 @@ int launch_tokens(const void* q, long long q_st, long long q_sh, const void* poo
                   long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                   void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
                   float* lsepart, const float* prior_o, long long po_st, long long po_sh, const float* prior_lse,
-                  long long pl_st, void* stream, bool r576) {
+                  long long pl_st, void* ws, void* stream, bool r576) {
   Params p;
   p.q = (const uint16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.pool = (const uint8_t*)pool; p.R = R;
@@ -653,18 +764,23 @@ int launch_tokens(const void* q, long long q_st, long long q_sh, const void* poo
   p.opart = opart; p.lsepart = lsepart;
   p.prior_o = prior_o; p.po_st = po_st; p.po_sh = po_sh; p.prior_lse = prior_lse; p.pl_st = pl_st;
   p.mk = nullptr; p.cu = nullptr; p.ql = 1; p.tsh = 0; p.NR = T;
+  p.ws_cnt = (uint32_t*)ws;
+  p.ws_lse = ws ? (float*)((uint8_t*)ws + ws_cnt_bytes(T, H)) : nullptr;
+  p.ws_o = ws ? (float*)((uint8_t*)p.ws_lse + ws_lse_bytes(T, H, S)) : nullptr;
   const long long nwork = (long long)T * S * p.HGN;
   if (nwork > (1ll << 30)) return SPMLA_ELIMIT;
   const int grid = (int)((nwork + 7) / 8 * 8);
-  if (r576) {
-    static DynLds lds_attr5;
-    if (const int e = lds_attr5.ensure((const void*)attn_kernel<false, true>, L_TOTAL)) return e;
-    hipLaunchKernelGGL((attn_kernel<false, true>), dim3(grid), dim3(256), L_TOTAL, (hipStream_t)stream, p);
-  } else {
-    static DynLds lds_attr;
-    if (const int e = lds_attr.ensure((const void*)attn_kernel<false>, L_TOTAL)) return e;
-    hipLaunchKernelGGL(attn_kernel<false>, dim3(grid), dim3(256), L_TOTAL, (hipStream_t)stream, p);
-  }
+  static DynLds lds_attr[4];
+  const int v = (r576 ? 2 : 0) | (ws ? 1 : 0);
+  const void* fn = v == 0 ? (const void*)attn_kernel<false> : v == 1 ? (const void*)attn_kernel<false, false, true>
+                 : v == 2 ? (const void*)attn_kernel<false, true> : (const void*)attn_kernel<false, true, true>;
+  if (const int e = lds_attr[v].ensure(fn, L_TOTAL)) return e;
+  const dim3 g(grid), b(256);
+  const hipStream_t st = (hipStream_t)stream;
+  if (v == 0) hipLaunchKernelGGL(attn_kernel<false>, g, b, L_TOTAL, st, p);
+  else if (v == 1) hipLaunchKernelGGL((attn_kernel<false, false, true>), g, b, L_TOTAL, st, p);
+  else if (v == 2) hipLaunchKernelGGL((attn_kernel<false, true>), g, b, L_TOTAL, st, p);
+  else hipLaunchKernelGGL((attn_kernel<false, true, true>), g, b, L_TOTAL, st, p);
   return (int)hipGetLastError();
 }
 
@@ -701,6 +817,7 @@ int spmla_attn_packed(const void* q, long long q_st, long long q_sh, const void*
   p.opart = f32part ? opart : nullptr; p.lsepart = lsepart;
   p.prior_o = nullptr; p.po_st = p.po_sh = 0; p.prior_lse = nullptr; p.pl_st = 0;
   p.mk = (const uint8_t*)mk; p.cu = cu; p.ql = ql; p.NR = nreq;
+  p.ws_cnt = nullptr; p.ws_lse = nullptr; p.ws_o = nullptr;
   const long long nwork = (long long)nreq * S * p.HGN;
   if (nwork > (1ll << 30)) return SPMLA_ELIMIT;
   const int grid = (int)((nwork + 7) / 8 * 8);

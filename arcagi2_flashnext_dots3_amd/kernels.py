@@ -4,6 +4,8 @@ Each wrapper mirrors the Python side of the reference kernel it replaces (offloa
 offload_cuda.split_partials, fast_topk.local/merge, ShardStore.write/logits, LayerOffload.gather), raises
 RuntimeError on a failed launch and never falls back to a CPU path.
 """
+import functools
+
 import torch
 
 from . import _lib
@@ -211,9 +213,9 @@ def _workspace(kind, device, nbytes, zero=False):
 
 
 def fused_max_tokens(H, cus=256):
-    """The most tokens for which auto_split picks the in-kernel split merge (H heads): below it attend needs a
+    """The most tokens for which auto_split picks the in-kernel split merge (H heads): up to it attend needs a
     workspace."""
-    return max(0, -(-cus * 3 // (8 * ((H + 31) // 32))) - 1)
+    return cus // (2 * ((H + 31) // 32))
 
 
 def reserve_workspace(device, H, T=None, split=8):
@@ -222,6 +224,24 @@ def reserve_workspace(device, H, T=None, split=8):
     T = fused_max_tokens(H) if T is None else T
     if T > 0:
         _workspace("attn", device, int(_lib.lib().spmla_attn_ws_bytes(T, H, split)), zero=True)
+
+
+def _attn_workspace(device, T, H, split, private=False):
+    """A workspace for a merged launch with its leading counter bytes zero (queued on the current stream): the cached
+    one, or, with private under graph capture, a temporary of the graph itself, so that graphs may replay beside each
+    other and beside eager calls."""
+    nb, cnt = attn_ws_bytes(T, H, split), _attn_counter_bytes(T, H)
+    if private and torch.cuda.is_current_stream_capturing():
+        ws, key = torch.empty(nb, dtype=torch.uint8, device=device), None
+    else:
+        ws, key = _workspace("attn", device, nb, zero=True)
+    if key is None:                       # captured: replays come in any order, so every replay clears its counters
+        ws[:cnt].zero_()
+    else:
+        if cnt > _WS_CNT[key]:            # counter bytes the previous launch used as scratch: cleared by a fill kernel
+            ws[_WS_CNT[key]:cnt].zero_()
+        _WS_CNT[key] = cnt
+    return ws
 
 
 def _attn_counter_bytes(T, H):
@@ -633,33 +653,31 @@ def attention_ok(q, idx):
 ATTN_SPLIT_ROWS = 2048      # rows of one (token, split) in spmla_attn's split merge, rounded up to 32-row tiles
 
 
-def auto_split(T, H, K, cus=256):
-    """Row splits per token. 1 when the unsplit launch has at least cus * 3 / 8 workgroups of 32 heads (the
-    head-group kernel: a workgroup of 32 heads over all K rows takes as long as one of 128 heads over K / 4 rows, so
-    a partly filled unsplit launch still beats a split one with its merge); else the in-kernel split merge over
-    128-head workgroups, doubled while that launch has fewer workgroups than compute units and every split keeps
-    at least 8 tiles of 32 rows (at most 8 splits). 1 as well when a split would hold more than ATTN_SPLIT_ROWS
-    rows (the split kernel's limit; the head-group kernel takes any K)."""
-    if T * ((H + 31) // 32) * 8 >= cus * 3:
-        return 1
-    n = T * ((H + 127) // 128)
-    s = 1
-    while s < 8 and n * s < cus and K >= 2 * s * 256:
-        s *= 2
-    if -(-(-(-K // s)) // 32) * 32 > ATTN_SPLIT_ROWS:
-        return 1
-    return s
+def _split_cost(n, K, s, cus):
+    """Model of a launch of n * s workgroups over K / s rows each (us): rounds of one workgroup per compute unit, each a
+    fixed part and the longest wave's 32-row tiles; the merge of the splits on top. Fitted to graphed launches at
+    K = 512 .. 2048 (128 heads, K = 2048, T = 1 / 8 / 16 / 32: 1 split 48 / 50 / 50 / 51 us, 2 splits 34 / 36 / 36 / 39,
+    4 splits 25 / 27 / 29 / 54, 8 splits 24 / 26 / 49 / 85)."""
+    tiles = -(-(-(-K // s)) // 32)
+    return -(-n * s // cus) * (12.7 + 2.2 * -(-tiles // 4)) + (3.0 + 0.6 * s if s > 1 else 0.0)
 
 
+@functools.lru_cache(maxsize=4096)
 def auto_split576(T, H, K, cus=256):
-    """Row splits per token of a Row576 launch (one kernel, 32 heads per workgroup; split partials in fp32, merged by
-    spmla_lse_merge): doubled while the launch has fewer than cus * 3 / 8 workgroups and every split keeps at least
-    8 tiles of 32 rows (at most 8 splits)."""
+    """Row splits per token (merged in the kernel, at most 8). 1 when the unsplit launch has more than half as many
+    workgroups of 32 heads as there are compute units: a second round would cost what the shorter lists save. Else the
+    split of least _split_cost."""
     n = T * ((H + 31) // 32)
-    s = 1
-    while s < 8 and n * s * 8 < cus * 3 and K >= 2 * s * 256:
-        s *= 2
-    return s
+    if 2 * n > cus or n == 0:
+        return 1
+    return min(range(1, 9), key=lambda s: (_split_cost(n, K, s, cus), s))
+
+
+def auto_split(T, H, K, cus=256):
+    """auto_split576 for Row656 pools: 1 as well when a split would hold more than ATTN_SPLIT_ROWS rows (the limit of
+    spmla_attn; the unsplit kernel takes any K)."""
+    s = auto_split576(T, H, K, cus)
+    return 1 if -(-(-(-K // s)) // 32) * 32 > ATTN_SPLIT_ROWS else s
 
 
 def attn_ws_bytes(T, H, split):
@@ -671,11 +689,12 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
            row_bytes=None):
     """q [T, H, 576] bf16, pool [R, 656] uint8 Row656 rows (or a mapped host address with R given), idx [T, K]
     int32 rows -> (out [T, H, 512] bf16, lse [T, H] fp32). Row576 rows (pool [..., 576], or row_bytes=576: the
-    per-tensor fp8 cache, every code times kv_scale) go to spmla_attn576, whose splits merge through fp32 partials
-    (split None: auto_split576). For Row656, split > 1 (at most 8) cuts K into partials that the
-    kernel merges (spmla_attn; ws: a uint8 workspace of attn_ws_bytes whose leading counter bytes are zero -- the
-    kernel leaves them so --, else a cached one per stream; under HIP graph capture either ws or a workspace reserved
-    by an earlier eager call, see reserve_workspace); None: auto_split."""
+    per-tensor fp8 cache, every code times kv_scale) go to spmla_attn576 / spmla_attn576_ws (split None: auto_split576).
+    split > 1 (at most 8) cuts K into partials that the kernel merges in a workspace: a cached one per stream, under
+    HIP graph capture one of the graph's own. For Row656 (spmla_attn; split None: auto_split) ws may be given, a uint8
+    workspace of attn_ws_bytes whose leading counter bytes are zero -- the kernel leaves them so --, and captured
+    launches of fewer than 96 workgroups (token, 32 heads) take either ws or a workspace reserved by an earlier eager
+    call, see reserve_workspace."""
     T, H, _ = q.shape
     K = idx.shape[1]
     rb = int(row_bytes) if row_bytes is not None else (int(pool.shape[-1]) if torch.is_tensor(pool) else ROW656)
@@ -697,12 +716,11 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
                       idx.stride(0), K, _ptr(kcount), T, H, float(sm_scale), float(kv_scale), 1, out.data_ptr(),
                       out.stride(0), out.stride(1), lse.data_ptr(), lse.stride(0), None, None, st)
             return out, lse
-        opart = torch.empty(split, T, H, D_LAT, dtype=torch.float32, device=q.device)
-        lpart = torch.empty(split, T, H, dtype=torch.float32, device=q.device)
-        _lib.call("spmla_attn576", q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(), idx.stride(0),
-                  K, _ptr(kcount), T, H, float(sm_scale), float(kv_scale), split, None, 0, 0, None, 0,
-                  opart.data_ptr(), lpart.data_ptr(), st)
-        return lse_merge(opart, lpart, out=out, lse=lse)
+        ws = _attn_workspace(q.device, T, H, split, private=True)
+        _lib.call("spmla_attn576_ws", q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(), idx.stride(0),
+                  K, _ptr(kcount), T, H, float(sm_scale), float(kv_scale), split, out.data_ptr(), out.stride(0),
+                  out.stride(1), lse.data_ptr(), lse.stride(0), ws.data_ptr(), ws.numel(), st)
+        return out, lse
     if split == 1:
         _lib.call("spmla_attn_splitk", q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(),
                   idx.stride(0), K, _ptr(kcount), T, H, float(sm_scale), float(kv_scale), 1, out.data_ptr(),
@@ -711,14 +729,8 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
     _need(1 <= split <= 8, "attend: split must be 1 .. 8")
     nb = int(_lib.lib().spmla_attn_ws_bytes(T, H, split))
     if ws is None:
-        ws, key = _workspace("attn", q.device, nb, zero=True)
-        cnt = _attn_counter_bytes(T, H)
-        if key is None:                   # captured: replays come in any order, so every replay clears its counters
-            ws[:cnt].zero_()
-        else:
-            if cnt > _WS_CNT[key]:        # counter bytes the previous launch used as scratch: cleared by a fill kernel
-                ws[_WS_CNT[key]:cnt].zero_()
-            _WS_CNT[key] = cnt
+        # from 96 workgroups on (3/8 of the compute units) the unsplit launch needs none: a capture brings its own
+        ws = _attn_workspace(q.device, T, H, split, private=T * ((H + 31) // 32) >= 96)
     _need(ws.dtype == torch.uint8 and ws.numel() >= nb, "attend: workspace too small")
     _lib.call("spmla_attn", q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(), idx.stride(0), K,
               _ptr(kcount), T, H, float(sm_scale), float(kv_scale), split, out.data_ptr(), out.stride(0),

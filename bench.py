@@ -191,15 +191,15 @@ def run_config2(a, dev):
     ms = _timed(replay, reps, max(1, a.warmup // n)) / n
     eager_ms = _timed(step, a.steps, a.warmup)          # right after, at the same settled clocks
     gbs = ALG_BYTES / (ms * 1e-3) / 1e9
-    # unsplit decode launches run the head-group kernel, split ones the 128-head kernel with its in-kernel merge
-    kname = "spmla::pk::attn_kernel<false, false>" if split == 1 else "spmla::attn::fwd_kernel"
+    # unsplit decode launches run the head-group kernel, split ones its instance with the in-kernel merge
+    kname = f"spmla::pk::attn_kernel<false, false, {'false' if split == 1 else 'true'}>"
     roof = {"bound": "hbm", "achieved": round(gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
             "kernel": kname, "alg_bytes_per_launch": ALG_BYTES,
             "mfma_tflops": round(ALG_FLOPS / (ms * 1e-3) / 1e12, 2),
             "mfma_frac_bf16_peak": round(ALG_FLOPS / (ms * 1e-3) / 1e12 / BF16_PEAK_TFLOPS, 4)}
     if not a.no_traffic:     # HBM bytes per launch, counted in this run (rocprofv3 --pmc over probe children)
-        tr = measure_traffic(r"attn_kernel<false, false>" if split == 1 else "fwd_kernel",
+        tr = measure_traffic(kname.split("::")[-1],
                              ["--config", "2", "--probe", "--idx-sets", str(a.idx_sets)])
         roof["traffic"] = tr.get("bytes_per_launch")
         roof["traffic_detail"] = tr

@@ -320,9 +320,9 @@ int spmla_attn576(const void* q, long long q_st, long long q_sh, const void* poo
 /* Bytes of the workspace spmla_attn needs for T tokens, H heads and S splits (0 for S = 1; -1 for bad sizes). */
 long long spmla_attn_ws_bytes(int T, int H, int S);
 
-/* spmla_attn_splitk with the bf16 out + lse for any S in 1 .. 8: the S splits of a (token, group of 128 heads) merge
- * in the kernel -- each writes its normalized partial (f16, with a power-of-two exponent per head that keeps it in
- * range) and lse to ws, and the last split to finish merges all of them (weights e^(lse_s - M) / Z) into out / lse.
+/* spmla_attn_splitk with the bf16 out + lse for any S in 1 .. 8: the S splits of a (token, group of 32 heads), which
+ * share the token's min(K, kcount) entries, merge in the kernel -- each writes its normalized fp32 partial and lse to
+ * ws, and the last split to finish merges all of them in order (weights e^(lse_s - M) / Z) into out / lse.
  * ws: spmla_attn_ws_bytes(T, H, S) bytes, 256-byte aligned. Its first C = 4 * T * ceil(H / 128) bytes (rounded up
  * to a multiple of 256) are the launch's counters and must be zero when it starts; the kernel leaves them zero, and
  * the bytes past them are scratch. So a workspace zero-filled once serves launches that run one after another,
@@ -336,6 +336,12 @@ int spmla_attn(const void* q, long long q_st, long long q_sh, const void* pool, 
                long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                void* out, long long o_st, long long o_sh, float* lse, long long lse_st, void* ws, long long ws_bytes,
                void* stream);
+
+/* spmla_attn over Row576 rows (spmla_attn576's arguments, S splits merged in the kernel, the same workspace; any K). */
+int spmla_attn576_ws(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
+                     long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
+                     void* out, long long o_st, long long o_sh, float* lse, long long lse_st, void* ws,
+                     long long ws_bytes, void* stream);
 
 /* spmla_attn_splitk (S = 1) whose result is merged with a prior partial of the same tokens and heads before the bf16
  * write: prior_o [T][H][512] fp32 normalized (strides po_st, po_sh; 16-byte aligned), prior_lse [T][H] (stride

@@ -141,3 +141,55 @@ def test_plugin_row576_paged_prefill_scale(dev):
     o_ref, l_ref = ref.attention(q[tokens].float().cpu().numpy(), rows, local, 192 ** -0.5, ks, fmt=576)
     o = out[tokens].float().cpu().numpy()
     assert attn_excess(o, o_ref) <= 0
+
+
+@pytest.mark.parametrize("split", [2, 3, 5, 8])
+def test_attn576_splits_merged_in_the_kernel(dev, split):
+    """S splits of five head groups (the counters of a token cross a word) merged in the kernel: ragged counts that
+    leave splits or whole tokens without rows, the same bits on a second launch, and vs the oracle."""
+    T, H, R, K = 3, 160, 3000, 1000
+    pool = make_pool_576(R, seed=17, kv_scale=0.5)
+    q = make_q(T, H, seed=18)
+    idx = distinct_idx(T, K, R, seed=19)
+    idx[1, 40:90] = -1
+    kcount = torch.tensor([1000, 65, 0], dtype=torch.int32)
+    sm = 192 ** -0.5
+    print(f"[576] merged splits {split}", flush=True)
+    o, l = _attend(dev, q, pool, idx, sm, 0.5, split, kcount)
+    o_ref, l_ref = ref.attention(q.float().numpy(), pool, idx.numpy(), sm, 0.5, kcount=kcount.numpy(), fmt=576)
+    _check(o, l, o_ref, l_ref, f"Row576 split {split}")
+    o2, l2 = _attend(dev, q, pool, idx, sm, 0.5, split, kcount)
+    assert np.array_equal(o, o2) and np.array_equal(l, l2)
+
+
+@pytest.mark.parametrize("row,T", [(656, 24), (576, 24), (576, 2)])
+def test_captured_merge_without_a_reserved_workspace(dev, row, T, monkeypatch):
+    """Launches that need no workspace reserved before a capture bring their own: two graphs replayed alternately, with
+    eager calls between them, give the eager bits every time."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    H, K, R, sm = 128, 2048, 4096, 192 ** -0.5
+    pool = torch.randint(0, 120, (R, row), dtype=torch.uint8, generator=torch.Generator().manual_seed(3)).to(dev)
+    if row == 656:
+        pool[:, 512:528] = torch.full((4,), 0.01).view(torch.uint8).to(dev)
+        pool[:, 528:] = torch.ones(64, dtype=torch.bfloat16).view(torch.uint8).to(dev)
+    qs = [make_q(T, H, seed=20 + i).to(dev) for i in range(2)]
+    ids = [distinct_idx(T, K, R, seed=30 + i).to(dev) for i in range(2)]
+    print(f"[capture] row {row} T={T} split {kernels.auto_split576(T, H, K)}", flush=True)
+    assert kernels.auto_split576(T, H, K) > 1
+    eager = [kernels.attend(q, pool, i, sm) for q, i in zip(qs, ids)]
+    torch.cuda.synchronize()
+    monkeypatch.setattr(kernels, "_WS", {})
+    graphs, outs = [], []
+    for q, i in zip(qs, ids):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            outs.append(kernels.attend(q, pool, i, sm))
+        graphs.append(g)
+    for _ in range(3):
+        for n in (0, 1):
+            outs[n][0].fill_(7.0)
+            graphs[n].replay()
+            o, l = kernels.attend(qs[1 - n], pool, ids[1 - n], sm)
+            torch.cuda.synchronize()
+            assert torch.equal(outs[n][0], eager[n][0]) and torch.equal(outs[n][1], eager[n][1])
+            assert torch.equal(o, eager[1 - n][0]) and torch.equal(l, eager[1 - n][1])
