@@ -16,10 +16,11 @@
 //   (-0 < +0, NaN largest); equal keys -> lower column first; output positions sorted by (value desc, column asc),
 //   -1 where the value is +-inf and in slots >= n. fp32 or fp16 logits: an fp16 key is the same order key of the
 //   16-bit pattern placed in the top half of the 32-bit key (low half zero), so one radix code serves both.
-//   gfx950: one 1024-thread workgroup per row, the row's keys in VGPRs (32 per thread, all loads in flight):
-//   11/11/10-bit radix levels with an LDS histogram; keys above the boundary bin are appended at slots from a block
-//   scan of per-thread counts (wave scans on DPP); once the boundary bin holds at most the candidate cap the remaining
-//   levels run on those candidates alone; ties on the final key take the lowest columns. The K winners are
+//   gfx950: rows of up to 32768 columns, and up to 8 such chunks of a row, are selected and sorted by bins of equal
+//   width (topk_row_kernel, topk_chunk_kernel). Longer rows, and the two stages of the rank-sharded selection, go
+//   through 11/11/10-bit radix levels with an LDS histogram; keys above the boundary bin are appended at slots from a
+//   block scan of per-thread counts (wave scans on DPP); once the boundary bin holds at most the candidate cap the
+//   remaining levels run on those candidates alone; ties on the final key take the lowest columns. The K winners are
 //   bitonic-sorted in LDS (only the stages whose pairs cross waves take a workgroup barrier); on the several-
 //   workgroup path, whose lists arrive in column order, fp16 winners are ordered by a stable radix sort instead.
 #include "spmla_common.h"
@@ -59,9 +60,7 @@ struct LogitParams {
   const int* lo;                             // optional per-row first valid position (flat layout: cu_seqlen_ks)
   const float* kscale; long long k_st;       // flat layout: key j codes at store + j * k_st, scale kscale[j]
   int tpg;                                   // 32-key tiles per workgroup (the launcher's lg_grid)
-  // optional level-0 top-k histograms (P == 1): workgroup (row, g) counts the top-k keys of its columns j <
-  // min(ctx, Lc) into hist + row * hist_rs bytes + g * 2048 bins (its columns are top-k chunk g)
-  uint32_t* hist; long long hist_rs;
+  int all;                                   // 1 (P == 1): columns below min(ctx, Lc) are written whatever noinf says
 };
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -98,7 +97,6 @@ template <bool POW2, int LY, bool F16OUT = false>
 __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
   constexpr bool SHUF = LY == LY_SHUF, FLAT = LY == LY_FLAT;
   constexpr int D = LG_D;
-  __shared__ uint32_t hh[1024];                             // level-0 histogram (p.hist): 2048 16-bit counts
   __shared__ float sbuf[LG_STAGE];                          // staged logits of the range's columns
   __shared__ uint32_t smask[LG_STAGE / 32];                 // per tile: the columns to write
   __shared__ int claim;                                     // next unclaimed tile of the range
@@ -119,20 +117,13 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
   const int te = min(tb + p.tpg, (p.Lc + 31) >> 5);
   const long long nvalid = ctx > p.rank ? ((long long)ctx - p.rank + p.P - 1) / p.P : 0;   // keys below ctx
   const int tv = p.lim == 0 ? tb : (int)min((long long)te, max((long long)tb, (nvalid + 31) >> 5));
-  if (!p.noinf)                                                         // keys of the range past ctx
-    for (int j = 32 * tv + (int)threadIdx.x; j < 32 * te && j < p.Lc; j += LG_NWV * 64) put(j, -__builtin_inff());
-  // the top-k's histogram covers columns below min(ctx, Lc) (P == 1: all in tiles below tv, none in the fill)
-  uint32_t* hrow_out = p.hist ? (uint32_t*)((uint8_t*)p.hist + (long long)row * p.hist_rs) + blockIdx.y * 2048 : nullptr;
-  if (tv <= tb) {                                           // uniform over the workgroup: no barrier below
-    if (hrow_out)
-      for (int b = (int)threadIdx.x; b < 2048; b += LG_NWV * 64) hrow_out[b] = 0u;
-    return;
-  }
+  const int nh = p.all ? min(ctx, p.Lc) : 0;                // columns the caller's top-k reads
+  if (!p.noinf || p.all)                                                // keys of the range past ctx
+    for (int j = 32 * tv + (int)threadIdx.x; j < 32 * te && j < (p.noinf ? nh : p.Lc); j += LG_NWV * 64)
+      put(j, -__builtin_inff());
+  if (tv <= tb) return;                                     // uniform over the workgroup: no barrier below
   if (threadIdx.x == 0) claim = tb + 2 * LG_D * LG_NWV;     // steps 0 .. 2 LG_D - 1 take tiles tb + k NW + w
-  if (hrow_out)
-    for (int b = (int)threadIdx.x; b < 1024; b += LG_NWV * 64) hh[b] = 0u;
   __syncthreads();
-  const int nh = hrow_out ? min(ctx, p.Lc) : 0;             // columns the histogram counts
   const int* btr = FLAT ? nullptr : p.bt + (long long)p.req[row] * p.bt_st;
   const int lo = p.lo ? p.lo[row] : 0;
   // n / d, n % d: shifts when every divisor is a power of two (POW2), else 32-bit division
@@ -240,21 +231,13 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
     const int j = 32 * id + l32;
     const float lg = p.clamp ? fminf(part * sc, 60000.f) : part * sc;
     const float v = ok ? lg : -__builtin_inff();
-    const bool counted = half == 0 && j < nh;               // a top-k column: always written
-    const bool wr = half == 0 && j < p.Lc && (ok || !p.noinf || counted);
+    const bool wr = half == 0 && j < p.Lc && (ok || !p.noinf || j < nh);
     if (stage) {
       if (half == 0) sbuf[32 * (id - tb) + l32] = v;
       const uint64_t m = __ballot(wr);
       if (lane == 0) smask[id - tb] = (uint32_t)m;
     } else if (wr) {
       put(j, v);
-    }
-    if (counted) {                                          // the key of the value as stored
-      uint32_t key;
-      if constexpr (F16OUT) key = okey16(__builtin_bit_cast(uint16_t, (_Float16)v));
-      else key = okey(v);
-      const uint32_t bin = key >> 21;
-      atomicAdd(&hh[bin >> 1], 1u << (16 * (bin & 1u)));
     }
   };
 
@@ -295,7 +278,7 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
       btv[s] = load_bt(ids[s]);
     }
   }
-  if (stage || hrow_out) __syncthreads();   // every wave has computed (and counted) its tiles
+  if (stage) __syncthreads();                // every wave has computed its tiles
   if (stage) {                               // 4 columns per thread: one 16-byte (fp16: 8-byte) store when all go out
     const int ncol = 32 * (tv - tb);
     const bool vec = ((uintptr_t)p.out & (F16OUT ? 7u : 15u)) == 0 && (p.out_st & 3) == 0;   // j % 4 == 0 below
@@ -317,8 +300,6 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
       }
     }
   }
-  if (hrow_out)
-    for (int b = (int)threadIdx.x; b < 2048; b += LG_NWV * 64) hrow_out[b] = (hh[b >> 1] >> (16 * (b & 1))) & 0xffffu;
 }
 
 // ------------------------------------------------------------------------------------------------ top-k
@@ -942,12 +923,364 @@ __global__ void __launch_bounds__(TK_NT) topk_kernel(TopkParams p) {
   tk_emit_sorted(src, nsel, p.K, p.out + (long long)row * p.out_st, L);
 }
 
+// ---- bucket selection: rows of at most 32768 columns, and chunks of longer rows ------------------------------
+// One 1024-thread workgroup holds up to 32768 keys in VGPRs and selects and sorts in one go: the values' range is cut
+// into 4096 equal bins (a float subtract and multiply round monotonically, so a larger value never gets a lower bin);
+// an LDS histogram and one scan give every bin's first slot in descending order and the bin of the K-th key; the keys
+// of that bin and above go to their bin's slots (an LDS atomic each), and an entry's final slot is its bin's first plus
+// the number of larger entries (key, then lower column) in its bin. Bins of equal width are nearly evenly filled by
+// indexer logits (a few entries each at the K-th key, where the 11-bit radix digits of the key put a fifth of the row
+// into one bin), so there is no second level and no sort of the winners. A row is a chain of barriers, LDS atomics and
+// one read of the row; in graphs, against a radix level over several workgroups, a second on its bin and a finishing
+// sort: 4 rows of 16000 columns 9.6 us (32.7), 64 of 32768 15.0 us (39.0), 2048 of 16384 55.6 us (356).
+// A row whose bins from the K-th key's on hold more than BK_LIM entries somewhere (heavy ties, far outliers, no finite
+// value) goes through a radix select over (key, column) instead.
+constexpr int BK_BINS = 4096;
+constexpr int BK_LIM = 256;                  // entries of a bin that are ranked by counting
+constexpr int BK_LIST = TK_KMAX + BK_LIM;    // entries from the K-th key's bin on
+constexpr int BK_COLS = 32768;               // columns of one workgroup
+static_assert(BK_BINS == 4 * TK_NT, "a thread owns 4 bins");
+
+struct BkLds {
+  __attribute__((aligned(16))) uint32_t off[BK_BINS];   // counts, then first slots, then ends
+  unsigned long long list[BK_LIST];
+  __attribute__((aligned(16))) uint32_t wsum[16];
+  __attribute__((aligned(16))) uint32_t red[32];        // per wave: smallest, largest finite key
+  uint32_t sh[8];
+};
+
+__device__ inline float unkey(uint32_t k) { return u2f((k & 0x80000000u) ? k & 0x7fffffffu : ~k); }   // okey's inverse
+__device__ inline int bk_bin(float v, float vmin, float scale) {
+  const float t = fminf(fmaxf((v - vmin) * scale, 0.f), (float)(BK_BINS - 1));   // -inf: 0; +inf: the last bin
+  return v != v ? BK_BINS - 1 : (int)t;                                            // NaN is the largest key
+}
+struct BkRange { float vmin, scale; int bin; uint32_t n; };   // bin of the K-th key, entries from it on
+
+// Bins of the keys v (bit i of vm: v[i] is one), K of them wanted (0 < K <= their number): L.off = every bin's first slot.
+// False (uniform) when the radix select has to do it.
+template <int EPT>
+__device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uint32_t K, BkRange& r) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const bool fin = ((vm >> i) & 1u) && __builtin_fabsf(v[i]) < __builtin_inff();
+    mn = fin ? fminf(mn, v[i]) : mn;
+    mx = fin ? fmaxf(mx, v[i]) : mx;
+  }
+  const uint32_t kn = wave_minmax<false>(okey(mn)), kx = wave_minmax<true>(okey(mx));
+  if (lane == 0) { L.red[wv] = kn; L.red[16 + wv] = kx; }
+  ((u32x4*)L.off)[tid] = u32x4{0u, 0u, 0u, 0u};
+  if (tid < 8) L.sh[tid] = 0u;
+  __syncthreads();
+  uint32_t an = 0xffffffffu, ax = 0u;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const u32x4 a = ((const u32x4*)L.red)[q], b = ((const u32x4*)L.red)[4 + q];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { an = min(an, a[e]); ax = max(ax, b[e]); }
+  }
+  r.vmin = unkey(an);
+  r.scale = ((float)BK_BINS - 0.01f) / (unkey(ax) - r.vmin);
+  if (!(r.scale > 0.f && r.scale < __builtin_inff())) return false;   // no finite value, one value, or an overflow
+#pragma unroll
+  for (int i = 0; i < EPT; ++i)
+    if ((vm >> i) & 1u) atomicAdd(&L.off[bk_bin(v[i], r.vmin, r.scale)], 1u);
+  __syncthreads();
+  u32x4* own = (u32x4*)L.off + (TK_NT - 1 - tid);      // bins 4095 - 4 t (element 3) down to 4092 - 4 t
+  u32x4 h = *own;
+  uint32_t tot;
+  uint32_t run = block_excl_scan(h[0] + h[1] + h[2] + h[3], L.wsum, &tot);
+  uint32_t big = 0;
+#pragma unroll
+  for (int e = 3; e >= 0; --e) {
+    const uint32_t c = h[e];
+    if (run < K) big = max(big, c);
+    if (run < K && run + c >= K) { L.sh[1] = (uint32_t)(BK_BINS - 4 - 4 * tid + e); L.sh[2] = run + c; }
+    h[e] = run;
+    run += c;
+  }
+  *own = h;
+  big = wave_minmax<true>(big);
+  if (lane == 0) atomicMax(&L.sh[0], big);
+  __syncthreads();
+  r.bin = (int)L.sh[1];
+  r.n = L.sh[2];
+  return L.sh[0] <= (uint32_t)BK_LIM;
+}
+
+// The K best of the entries src.ent(j), j < n ((key, ~column) packed, 0: none), into L.list in no order: radix select
+// over the 64 bits (all entries differ), then an append.
+template <class Src>
+__device__ inline void bk_radix(BkLds& L, const Src& src, int n, uint32_t K) {
+  const int tid = threadIdx.x;
+  unsigned long long prefix = 0, mask = 0;
+  uint32_t need = K;
+  for (int level = 0; level < 6; ++level) {
+    const int shift = level == 0 ? 53 : level == 1 ? 42 : level == 2 ? 32 : level == 3 ? 21 : level == 4 ? 10 : 0;
+    const unsigned long long dm = level == 2 || level == 5 ? 0x3ffu : 0x7ffu;
+    __syncthreads();
+    L.off[tid] = 0u;
+    L.off[tid + TK_NT] = 0u;
+    __syncthreads();
+    for (int j = tid; j < n; j += TK_NT) {
+      const unsigned long long e = src.ent(j);
+      if (e && (e & mask) == prefix) atomicAdd(&L.off[(e >> shift) & dm], 1u);
+    }
+    __syncthreads();
+    const int b0 = 2047 - 2 * tid;
+    const uint32_t h0 = L.off[b0], h1 = L.off[b0 - 1];
+    uint32_t tot;
+    const uint32_t before = block_excl_scan(h0 + h1, L.wsum, &tot);
+    if (before < need && before + h0 >= need) { L.sh[1] = (uint32_t)b0; L.sh[2] = before; L.sh[3] = h0; }
+    if (before + h0 < need && before + h0 + h1 >= need) { L.sh[1] = (uint32_t)b0 - 1; L.sh[2] = before + h0; L.sh[3] = h1; }
+    __syncthreads();
+    prefix |= (unsigned long long)L.sh[1] << shift;
+    mask |= dm << shift;
+    need -= L.sh[2];
+    if (L.sh[3] == need) break;                        // uniform: the bin is taken whole
+  }
+  __syncthreads();
+  if (tid == 0) L.sh[4] = 0u;
+  __syncthreads();
+  for (int j = tid; j < n; j += TK_NT) {
+    const unsigned long long e = src.ent(j);
+    if (e && (e & mask) >= prefix) {
+      const uint32_t s = atomicAdd(&L.sh[4], 1u);
+      if (s < (uint32_t)BK_LIST) L.list[s] = e;
+    }
+  }
+  __syncthreads();
+}
+
+// Columns c0 .. c1 - 1 of a logits row (at most EPT * 1024): v[4 g + e] = column c0 + 4 (tid + 1024 g) + e as fp32, and
+// the mask of the columns that exist. Through a buffer that ends at c1 (reads past it give 0), so no load is under a
+// branch; 4 columns a load on aligned rows (the last, partial four by single loads).
+template <bool F16, int EPT>
+__device__ inline uint32_t bk_load(const void* row, int c0, int c1, float (&v)[EPT]) {
+  constexpr int ES = F16 ? 2 : 4;
+  const int tid = threadIdx.x, n = c1 - c0;
+  const uint64_t a = (uint64_t)(uintptr_t)row + (uint64_t)c0 * ES;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(uintptr_t)(((uint64_t)hi << 32) | lo), (short)0, n * ES, 0x00020000);
+  auto one = [&](int j) -> float {
+    if constexpr (F16) return (float)__builtin_bit_cast(_Float16, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, 2 * j, 0, 0));
+    else return u2f(__builtin_amdgcn_raw_buffer_load_b32(rs, 4 * j, 0, 0));
+  };
+  uint32_t vm = 0;
+  if ((lo & (4 * ES - 1)) == 0u) {
+#pragma unroll
+    for (int g = 0; g < EPT / 4; ++g) {
+      const int j = 4 * (tid + TK_NT * g);
+      const int at = j + 4 <= n ? j * ES : n * ES;         // past the end: zeros
+      if constexpr (F16) {
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+        const f16x4 x = __builtin_bit_cast(f16x4, (u32x2)__builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * g + e] = (float)x[e];
+      } else {
+        const f32x4 x = __builtin_bit_cast(f32x4, (u32x4)__builtin_amdgcn_raw_buffer_load_b128(rs, at, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * g + e] = x[e];
+      }
+    }
+    const int q = n >> 2;                                  // the partial four, if any, is group q / 1024 of thread q % 1024
+    if ((n & 3) && tid == (q & (TK_NT - 1))) {
+#pragma unroll
+      for (int g = 0; g < EPT / 4; ++g)
+        if (g == q >> 10) {
+#pragma unroll
+          for (int e = 0; e < 3; ++e) v[4 * g + e] = one(4 * q + e);
+        }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) v[i] = one(4 * (tid + TK_NT * (i >> 2)) + (i & 3));
+  }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) vm |= (uint32_t)(4 * (tid + TK_NT * (i >> 2)) + (i & 3) < n) << i;
+  return vm;
+}
+
+template <bool F16>
+struct RowEnts {     // columns c0 .. of a logits row as (key, ~column)
+  const void* x; int c0;
+  __device__ unsigned long long ent(int j) const {
+    float v;
+    if constexpr (F16) v = (float)((const _Float16*)x)[c0 + j];
+    else v = ((const float*)x)[c0 + j];
+    return tk_pack(okey(v), c0 + j);
+  }
+};
+
+// The entries of L.list from the K-th key's bin on, in final order, to o[0, K) (column, -1 for +-inf), and -1 to kout.
+__device__ inline void bk_emit(BkLds& L, const BkRange& r, uint32_t K, int kout, int* o) {
+  for (uint32_t i = threadIdx.x; i < r.n; i += TK_NT) {
+    const unsigned long long e = L.list[i];
+    const int b = bk_bin(unkey((uint32_t)(e >> 32)), r.vmin, r.scale);
+    const uint32_t end = L.off[b];                        // the appends moved a bin's first slot to its end
+    uint32_t at = b + 1 < BK_BINS ? L.off[b + 1] : 0u, first = at;
+    for (uint32_t j = first; j < end; ++j) at += (uint32_t)(L.list[j] > e);
+    if (at < K) o[at] = inf_key<false>((uint32_t)(e >> 32)) ? -1 : (int)~(uint32_t)e;
+  }
+  for (int s = (int)K + (int)threadIdx.x; s < kout; s += TK_NT) o[s] = -1;
+}
+__device__ inline void bk_emit_sorted(BkLds& L, uint32_t K, int kout, int* o) {   // after bk_radix
+  tk_sort_desc(L.list, (int)K);
+  for (int s = threadIdx.x; s < kout; s += TK_NT) {
+    int c = -1;
+    if (s < (int)K) {
+      const unsigned long long e = L.list[s];
+      if (!inf_key<false>((uint32_t)(e >> 32))) c = (int)~(uint32_t)e;
+    }
+    o[s] = c;
+  }
+}
+
+// Rows of at most EPT * 1024 columns, one workgroup each. Two workgroups share a compute unit up to 16 keys a thread.
+template <bool F16, int EPT>
+__global__ void __launch_bounds__(TK_NT, EPT <= 16 ? 8 : 4) topk_row_kernel(TopkParams p) {
+  __shared__ BkLds L;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  int n = p.ctx[row];
+  n = n < 0 ? 0 : (n > p.Lc ? p.Lc : n);
+  int* o = p.out + (long long)row * p.out_st;
+  const uint32_t K = (uint32_t)min(n, p.K);
+  if (K == 0) {                                           // uniform
+    for (int s = tid; s < p.K; s += TK_NT) o[s] = -1;
+    return;
+  }
+  const void* x = lrow<F16>(p.lg, row, p.lg_st);
+  float v[EPT];
+  const uint32_t vm = bk_load<F16, EPT>(x, 0, n, v);
+  BkRange r;
+  if (!bk_bins<EPT>(L, v, vm, K, r)) {
+    bk_radix(L, RowEnts<F16>{x, 0}, n, K);
+    bk_emit_sorted(L, K, p.K, o);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const int b = bk_bin(v[i], r.vmin, r.scale);
+    if (((vm >> i) & 1u) && b >= r.bin) L.list[atomicAdd(&L.off[b], 1u)] = tk_pack(okey(v[i]), 4 * (tid + TK_NT * (i >> 2)) + (i & 3));
+  }
+  __syncthreads();
+  bk_emit(L, r, K, p.K, o);
+}
+
+// Longer rows: a workgroup per chunk of at most 32768 columns writes its entries that can be among the row's K (its
+// own K best and the rest of their last bin) to a list in the workspace, then one workgroup per row selects and sorts
+// over the lists. 64 rows of 131072 columns 26.7 us against 50.6 for the radix passes, 1024 of 65536 132 against 560.
+struct BkWs {                                             // workspace of a row: G list lengths, then G lists
+  static constexpr int GMAX = 8;
+  static constexpr long long LISTS = 64;                  // bytes before the lists
+  static constexpr long long NEED = LISTS + (long long)GMAX * BK_LIST * 8;
+};
+struct TopkChunkParams {
+  const void* lg; long long lg_st;
+  const int* ctx; int rows, Lc, K;
+  int* out; long long out_st;
+  uint8_t* ws; long long row_bytes; int G, CL;            // chunks per row, columns per chunk
+};
+
+template <bool F16>
+__global__ void __launch_bounds__(TK_NT) topk_chunk_kernel(TopkChunkParams p) {
+  constexpr int EPT = BK_COLS / TK_NT;
+  __shared__ BkLds L;
+  const int row = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
+  int n = p.ctx[row];
+  n = n < 0 ? 0 : (n > p.Lc ? p.Lc : n);
+  uint8_t* wr = p.ws + (long long)row * p.row_bytes;
+  unsigned long long* list = (unsigned long long*)(wr + BkWs::LISTS) + (long long)g * BK_LIST;
+  const int c0 = min(g * p.CL, n), c1 = min(c0 + p.CL, n);
+  const uint32_t K = (uint32_t)min(c1 - c0, p.K);
+  if (K == 0) {
+    if (tid == 0) ((uint32_t*)wr)[g] = 0u;
+    return;
+  }
+  const void* x = lrow<F16>(p.lg, row, p.lg_st);
+  float v[EPT];
+  const uint32_t vm = bk_load<F16, EPT>(x, c0, c1, v);
+  BkRange r;
+  if (!bk_bins<EPT>(L, v, vm, K, r)) {
+    bk_radix(L, RowEnts<F16>{x, c0}, c1 - c0, K);
+    for (uint32_t i = tid; i < K; i += TK_NT) list[i] = L.list[i];
+    if (tid == 0) ((uint32_t*)wr)[g] = K;
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const int b = bk_bin(v[i], r.vmin, r.scale);
+    if (((vm >> i) & 1u) && b >= r.bin) list[atomicAdd(&L.off[b], 1u)] = tk_pack(okey(v[i]), c0 + 4 * (tid + TK_NT * (i >> 2)) + (i & 3));
+  }
+  if (tid == 0) ((uint32_t*)wr)[g] = r.n;
+}
+
+struct ListEnts {     // the lists of a row one after another, BK_LIST places each (0: no entry)
+  const uint8_t* wr;
+  __device__ unsigned long long ent(int j) const {
+    const int g = j / BK_LIST;
+    return (uint32_t)(j - g * BK_LIST) < ((const uint32_t*)wr)[g] ? ((const unsigned long long*)(wr + BkWs::LISTS))[j] : 0ull;
+  }
+};
+
+template <int G>                                          // lists per row, rounded up
+__global__ void __launch_bounds__(TK_NT) topk_lists_kernel(TopkChunkParams p) {
+  constexpr int EPT = (G * BK_LIST + TK_NT - 1) / TK_NT;
+  __shared__ BkLds L;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  int n = p.ctx[row];
+  n = n < 0 ? 0 : (n > p.Lc ? p.Lc : n);
+  int* o = p.out + (long long)row * p.out_st;
+  const uint32_t K = (uint32_t)min(n, p.K);
+  if (K == 0) {
+    for (int s = tid; s < p.K; s += TK_NT) o[s] = -1;
+    return;
+  }
+  const ListEnts src{p.ws + (long long)row * p.row_bytes};
+  const int m = p.G * BK_LIST;
+  unsigned long long e[EPT];
+  float v[EPT];
+  uint32_t vm = 0, cnt[EPT];
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {                         // every place is read, the unused ones dropped
+    const int j = min(tid + TK_NT * i, m - 1);
+    e[i] = ((const unsigned long long*)(src.wr + BkWs::LISTS))[j];
+    cnt[i] = ((const uint32_t*)src.wr)[j / BK_LIST];
+  }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const int j = tid + TK_NT * i;
+    if (j >= m || (uint32_t)(j % BK_LIST) >= cnt[i]) e[i] = 0ull;
+  }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    vm |= (uint32_t)(e[i] != 0ull) << i;
+    v[i] = unkey((uint32_t)(e[i] >> 32));
+  }
+  BkRange r;
+  if (!bk_bins<EPT>(L, v, vm, K, r)) {
+    bk_radix(L, src, m, K);
+    bk_emit_sorted(L, K, p.K, o);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const int b = bk_bin(v[i], r.vmin, r.scale);
+    if (((vm >> i) & 1u) && b >= r.bin) L.list[atomicAdd(&L.off[b], 1u)] = e[i];
+  }
+  __syncthreads();
+  bk_emit(L, r, K, p.K, o);
+}
+
 // ---- top-k over several workgroups per row (workspace variant) -------------------------------------------
 // Two radix levels run across G workgroups per row (chunks of at most CL columns):
 //   hist:    the histogram of the level-0 11-bit digit over each chunk's keys;
 //   collect: every workgroup sums the G histograms of the level and finds the boundary bin b of the row's
 //            remaining need; it writes its chunk's keys above b (and in b when that completes the need) to the row's
-//            winner list, and the keys in b to the candidate list when the bin holds at most p.cap keys. A chunk's
+//            winner list, and the keys in b to the candidate list when the bin holds at most TK_CAP1 keys. A chunk's
 //            entries start at the offset the histograms of the chunks before it give; inside the chunk each wave
 //            takes its slots from a block scan per pass over 8 consecutive columns per thread, so every list is
 //            in column order (the finishing pass's stable radix sort of fp16 keys relies on it). Otherwise the
@@ -994,7 +1327,6 @@ struct TopkWsParams {
   int* out; long long out_st;
   uint8_t* ws; TopkWs w;
   unsigned long long* ovf;                        // optional overflow lists, G * CL entries per row (or null)
-  int cap;                                        // boundary bins of at most cap keys go to the finishing pass
   int level;
 };
 
@@ -1080,7 +1412,7 @@ __global__ void __launch_bounds__(TK_NT) topk_collect_kernel(TopkWsParams p) {
   __syncthreads();
   const uint32_t b = sh[1], above = sh[2], binc = sh[3];
   const bool whole = above + binc == need;
-  const bool fits = !whole && binc <= (uint32_t)p.cap;
+  const bool fits = !whole && binc <= (uint32_t)TK_CAP1;
   // this chunk's offsets: winners of the chunks before g (bins above b, and b itself when whole); candidates in b
   const uint32_t mine = ((uint32_t)b0 > b || (whole && (uint32_t)b0 == b) ? q0 : 0u) +
                         ((uint32_t)b1 > b || (whole && (uint32_t)b1 == b) ? q1 : 0u);
@@ -1202,7 +1534,7 @@ __global__ void __launch_bounds__(TK_NT) topk_collect_kernel(TopkWsParams p) {
   }
 }
 
-template <bool F16, int CAPK>                      // CAPK: the launch's candidate cap (p.cap)
+template <bool F16>
 __global__ void __launch_bounds__(TK_NT) topk_finish_kernel(TopkWsParams p) {
   __shared__ TopkLds L;
   const int row = blockIdx.x, tid = threadIdx.x;
@@ -1216,7 +1548,7 @@ __global__ void __launch_bounds__(TK_NT) topk_finish_kernel(TopkWsParams p) {
     nsel = tk_select(src, p.K, L);                  // few columns, or ties too heavy for the lists
   } else {
     // the header's counts, kept inside the lists (they are, whenever the histograms were this row's)
-    const int nsb = min(max(st.sb, 0), p.K), nbc = min(max(st.binc, 0), CAPK);
+    const int nsb = min(max(st.sb, 0), p.K), nbc = min(max(st.binc, 0), TK_CAP1);
     const uint32_t nneed = (uint32_t)min(max(st.need, 0), p.K - nsb);
     const unsigned long long* sel = p.w.sel(p.ws, row);
     for (int i = tid; i < nsb; i += TK_NT) L.sel[i] = sel[i];
@@ -1226,7 +1558,7 @@ __global__ void __launch_bounds__(TK_NT) topk_finish_kernel(TopkWsParams p) {
     }
     __syncthreads();
     if (st.state == TKW_CANDS)
-      tk_resolve_cands<CAPK / TK_NT>(L, nbc, st.lvl, (uint32_t)st.prefix, (uint32_t)st.mask, nneed, (uint32_t)nsb, n);
+      tk_resolve_cands<TK_CAP1 / TK_NT>(L, nbc, st.lvl, (uint32_t)st.prefix, (uint32_t)st.mask, nneed, (uint32_t)nsb, n);
     if constexpr (F16) {
       // fp16 keys: at most two radix passes (the keys' low half is zero), faster than the bitonic network here;
       // fp32 keys need three or four, slower than it (measured on the bench's indexer logits)
@@ -1357,18 +1689,39 @@ int scratch_ptr(void** out) {
 
 namespace spmla {
 namespace idx {
-// the passes of spmla_topk_ws on fp32 (F16 false) or fp16 logits
+// rows of at most BK_COLS columns: one workgroup each, 8 / 16 / 32 keys a thread (fewer registers and loads)
+static void topk_rows(const TopkParams& p, int dtype, hipStream_t st) {
+  const int v = (p.Lc <= 8 * TK_NT ? 0 : p.Lc <= 16 * TK_NT ? 2 : 4) + (dtype == 1 ? 1 : 0);
+  const dim3 g(p.rows), b(TK_NT);
+  switch (v) {
+    case 0: hipLaunchKernelGGL((topk_row_kernel<false, 8>), g, b, 0, st, p); break;
+    case 1: hipLaunchKernelGGL((topk_row_kernel<true, 8>), g, b, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((topk_row_kernel<false, 16>), g, b, 0, st, p); break;
+    case 3: hipLaunchKernelGGL((topk_row_kernel<true, 16>), g, b, 0, st, p); break;
+    case 4: hipLaunchKernelGGL((topk_row_kernel<false, 32>), g, b, 0, st, p); break;
+    default: hipLaunchKernelGGL((topk_row_kernel<true, 32>), g, b, 0, st, p); break;
+  }
+}
+static void topk_chunks(const TopkChunkParams& p, int dtype, hipStream_t st) {
+  const dim3 g(p.rows, p.G), b(TK_NT);
+  if (dtype == 1) hipLaunchKernelGGL(topk_chunk_kernel<true>, g, b, 0, st, p);
+  else hipLaunchKernelGGL(topk_chunk_kernel<false>, g, b, 0, st, p);
+  if (p.G <= 2) hipLaunchKernelGGL(topk_lists_kernel<2>, dim3(p.rows), b, 0, st, p);
+  else if (p.G <= 4) hipLaunchKernelGGL(topk_lists_kernel<4>, dim3(p.rows), b, 0, st, p);
+  else hipLaunchKernelGGL(topk_lists_kernel<BkWs::GMAX>, dim3(p.rows), b, 0, st, p);
+}
+
+// longer rows: the radix passes on fp32 (F16 false) or fp16 logits
 template <bool F16>
-static void topk_ws_passes(TopkWsParams p, hipStream_t stream, bool hist = true) {
+static void topk_ws_passes(TopkWsParams p, hipStream_t stream) {
   p.level = 0;
-  if (hist) hipLaunchKernelGGL(topk_hist_kernel<F16>, dim3(p.rows, p.w.G), dim3(TK_NT), 0, stream, p);
+  hipLaunchKernelGGL(topk_hist_kernel<F16>, dim3(p.rows, p.w.G), dim3(TK_NT), 0, stream, p);
   for (int level = 0; level < 2; ++level) {        // the level-1 histograms come from the level-0 collect
     p.level = level;
     hipLaunchKernelGGL(topk_collect_kernel<F16>, dim3(p.rows, p.w.G), dim3(TK_NT), 0, stream, p);
   }
   p.level = 2;                                      // header 2: the state after both levels
-  if (p.cap > TK_CAP1) hipLaunchKernelGGL((topk_finish_kernel<F16, TK_CAP>), dim3(p.rows), dim3(TK_NT), 0, stream, p);
-  else hipLaunchKernelGGL((topk_finish_kernel<F16, TK_CAP1>), dim3(p.rows), dim3(TK_NT), 0, stream, p);
+  hipLaunchKernelGGL(topk_finish_kernel<F16>, dim3(p.rows), dim3(TK_NT), 0, stream, p);
 }
 
 }  // namespace idx
@@ -1405,7 +1758,7 @@ static int logits_row(const void* q, long long q_st, long long q_sh, const float
                       const void* store, long long R_local, int rows_per_block, long long block_stride,
                       const int* block_table, long long bt_st, int block_size, const int* req, const int* ctx,
                       int rows, int H, int D, int Lc, int P, int rank, int noinf, void* out, long long out_st,
-                      int out_dtype, void* stream, uint32_t* hist, long long hist_rs, int tpg, int gy) {
+                      int out_dtype, void* stream, int all) {
   if (rows < 0 || Lc < 0 || P <= 0 || rank < 0 || rank >= P || block_size <= 0 || rows_per_block <= 0) return SPMLA_EARG;
   if (out_dtype != 0 && out_dtype != 1) return SPMLA_EARG;
   if (rows == 0 || Lc == 0) return SPMLA_OK;
@@ -1424,12 +1777,8 @@ static int logits_row(const void* q, long long q_st, long long q_sh, const float
   p.lim = R_local * P;
   p.clamp = 1;
   p.lo = nullptr; p.kscale = nullptr; p.k_st = 0;
-  dim3 grid = lg_grid(rows, Lc, p.tpg);
-  if (tpg > 0) {                                            // workgroup g = top-k chunk g < gy (the histogram's)
-    p.tpg = tpg;
-    grid = dim3(rows, (unsigned)gy);
-  }
-  p.hist = hist; p.hist_rs = hist_rs;
+  const dim3 grid = lg_grid(rows, Lc, p.tpg);
+  p.all = all;
   const bool pow2 = p.bs_sh >= 0 && p.rpb_sh >= 0 && p.p_sh >= 0;
   if (out_dtype == 1) {
     if (pow2) hipLaunchKernelGGL((idx::logits_kernel<true, idx::LY_ROW, true>), grid, dim3(idx::LG_NWV * 64), 0, (hipStream_t)stream, p);
@@ -1447,7 +1796,7 @@ int spmla_index_logits(const void* q, long long q_st, long long q_sh, const floa
                        int rows, int H, int D, int Lc, int P, int rank, int noinf, void* out, long long out_st,
                        int out_dtype, void* stream) {
   return logits_row(q, q_st, q_sh, w, w_st, store, R_local, rows_per_block, block_stride, block_table, bt_st,
-                    block_size, req, ctx, rows, H, D, Lc, P, rank, noinf, out, out_st, out_dtype, stream, nullptr, 0, 0, 0);
+                    block_size, req, ctx, rows, H, D, Lc, P, rank, noinf, out, out_st, out_dtype, stream, 0);
 }
 
 int spmla_index_logits_hist(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
@@ -1460,10 +1809,9 @@ int spmla_index_logits_hist(const void* q, long long q_st, long long q_sh, const
   if (rows == 0 || Lc == 0) return SPMLA_OK;
   const idx::TopkWs tw = idx::topk_ws_layout(Lc);
   if (!topk_ws || ((uintptr_t)topk_ws & 15) || ws_bytes < (long long)rows * tw.row_bytes) return SPMLA_EARG;
-  if (tw.CL >= 65536) return SPMLA_ELIMIT;                  // 16-bit counts per chunk: use the separate pass
+  if (tw.CL >= 65536) return SPMLA_ELIMIT;                  // longer rows: use the separate calls
   return logits_row(q, q_st, q_sh, w, w_st, store, R_local, rows_per_block, block_stride, block_table, bt_st,
-                    block_size, req, ctx, rows, H, D, Lc, 1, 0, noinf, out, out_st, out_dtype, stream,
-                    tw.hist((uint8_t*)topk_ws, 0), tw.row_bytes, tw.CL / 32, tw.G);
+                    block_size, req, ctx, rows, H, D, Lc, 1, 0, noinf, out, out_st, out_dtype, stream, 1);
 }
 
 int spmla_paged_mqa_logits(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
@@ -1528,7 +1876,8 @@ int spmla_topk(const void* logits, long long lg_st, const int* ctx, int rows, in
   if (!logits || !ctx || !out) return SPMLA_EARG;
   idx::TopkParams p;
   p.lg = logits; p.lg_st = lg_st; p.ctx = ctx; p.rows = rows; p.Lc = Lc; p.K = K; p.out = out; p.out_st = out_st;
-  if (dtype == 1) hipLaunchKernelGGL(idx::topk_kernel<true>, dim3(rows), dim3(idx::TK_NT), 0, (hipStream_t)stream, p);
+  if (Lc <= idx::BK_COLS) idx::topk_rows(p, dtype, (hipStream_t)stream);
+  else if (dtype == 1) hipLaunchKernelGGL(idx::topk_kernel<true>, dim3(rows), dim3(idx::TK_NT), 0, (hipStream_t)stream, p);
   else hipLaunchKernelGGL(idx::topk_kernel<false>, dim3(rows), dim3(idx::TK_NT), 0, (hipStream_t)stream, p);
   return (int)hipGetLastError();
 }
@@ -1546,36 +1895,38 @@ long long spmla_topk_ws_bytes(int rows, int Lc, int K) {
   return topk_ws_base(rows, Lc) + topk_ws_ovf(rows, Lc);
 }
 
-static int topk_ws_run(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
-                       long long out_st, void* ws, long long ws_bytes, int dtype, void* stream, bool hist) {
+int spmla_topk_ws(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
+                  long long out_st, void* ws, long long ws_bytes, int dtype, void* stream) {
   if (rows < 0 || Lc < 0 || K <= 0 || (dtype != 0 && dtype != 1)) return SPMLA_EARG;
   if (K > idx::TK_KMAX) return SPMLA_ELIMIT;
   if (rows == 0) return SPMLA_OK;
   if (!logits || !ctx || !out || !ws) return SPMLA_EARG;
   const long long base = topk_ws_base(rows, Lc), ovf = topk_ws_ovf(rows, Lc);
   if (((uintptr_t)ws & 15) || ws_bytes < base) return SPMLA_EARG;
+  if (Lc <= idx::BK_COLS) {                         // a row fits one workgroup's registers
+    idx::topk_rows(idx::TopkParams{logits, lg_st, ctx, rows, Lc, K, out, out_st}, dtype, (hipStream_t)stream);
+    return (int)hipGetLastError();
+  }
+  if (Lc <= idx::BkWs::GMAX * idx::BK_COLS) {       // up to 8 chunks, whose lists one workgroup's registers hold
+    const int G = (Lc + idx::BK_COLS - 1) / idx::BK_COLS;
+    idx::topk_chunks(idx::TopkChunkParams{logits, lg_st, ctx, rows, Lc, K, out, out_st, (uint8_t*)ws,
+                                          idx::topk_ws_layout(Lc).row_bytes, G, ((Lc + G - 1) / G + 1023) / 1024 * 1024},
+                     dtype, (hipStream_t)stream);
+    return (int)hipGetLastError();
+  }
   idx::TopkWsParams p;
   p.lg = logits; p.lg_st = lg_st; p.ctx = ctx; p.rows = rows; p.Lc = Lc; p.K = K; p.out = out; p.out_st = out_st;
   p.ws = (uint8_t*)ws; p.w = idx::topk_ws_layout(Lc);
   // with room for the overflow lists, a level that narrows hands its bin's keys to the next level in a list
   p.ovf = ovf > 0 && ws_bytes >= base + ovf ? (unsigned long long*)((uint8_t*)ws + base) : nullptr;
-  // fp32 rows of at most 32768 columns: the finishing pass takes boundary bins of up to 8192 keys, so the level-1
-  // collect has no row to refine on indexer logits (their level-0 bins hold up to ~21% of such a row); longer rows
-  // keep 4096 (their bins pass 8192 anyway, and longer candidate lists only slow the finishing pass)
-  p.cap = dtype == 0 && Lc <= 32768 ? idx::TK_CAP : idx::TK_CAP1;
-  if (dtype == 1) idx::topk_ws_passes<true>(p, (hipStream_t)stream, hist);
-  else idx::topk_ws_passes<false>(p, (hipStream_t)stream, hist);
+  if (dtype == 1) idx::topk_ws_passes<true>(p, (hipStream_t)stream);
+  else idx::topk_ws_passes<false>(p, (hipStream_t)stream);
   return (int)hipGetLastError();
-}
-
-int spmla_topk_ws(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
-                  long long out_st, void* ws, long long ws_bytes, int dtype, void* stream) {
-  return topk_ws_run(logits, lg_st, ctx, rows, Lc, K, out, out_st, ws, ws_bytes, dtype, stream, true);
 }
 
 int spmla_topk_ws_prehist(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
                           long long out_st, void* ws, long long ws_bytes, int dtype, void* stream) {
-  return topk_ws_run(logits, lg_st, ctx, rows, Lc, K, out, out_st, ws, ws_bytes, dtype, stream, false);
+  return spmla_topk_ws(logits, lg_st, ctx, rows, Lc, K, out, out_st, ws, ws_bytes, dtype, stream);
 }
 
 long long spmla_topk_scratch_bytes(void) { return idx::TOPK_SCRATCH_BYTES; }

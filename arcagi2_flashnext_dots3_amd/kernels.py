@@ -274,8 +274,7 @@ def topk(logits, ctx, K, out=None, single_pass=False, ws=None):
 
 
 def topk_prehist(logits, ctx, K, ws, out=None):
-    """topk over logits whose first-level histograms spmla_index_logits_hist already wrote into ws (same rows, Lc, K,
-    ctx and dtype; spmla_topk_ws_prehist): the histogram pass is skipped, the result is topk's."""
+    """topk over the logits of logits_hist (same rows, Lc, K, ctx, dtype and workspace; spmla_topk_ws_prehist)."""
     rows, Lc = logits.shape
     _need(logits.dtype in _LG_DT and logits.stride(1) == 1, "fp32 / fp16 logits with contiguous rows")
     _need(ctx.dtype == torch.int32 and ctx.is_contiguous(), "ctx int32")
@@ -289,9 +288,9 @@ def topk_prehist(logits, ctx, K, ws, out=None):
 
 
 def logits_hist(q, w, base, R, rpb, bstride, block_table, block_size, req, ctx, Lc, K, lg, ws, noinf=False):
-    """spmla_index_logits_hist (P = 1): the logits into lg [rows, >= Lc] (fp32 / fp16) and the first-level top-k
-    histograms into ws. Returns False without a launch when the fused path does not apply (a top-k chunk of 65536 or
-    more columns); the caller then runs the logits and topk separately."""
+    """spmla_index_logits_hist (P = 1): the logits into lg [rows, >= Lc] (fp32 / fp16), every column below
+    min(ctx, Lc) written. Returns False without a launch above 258048 columns; the caller then runs the logits and topk
+    separately."""
     rows = q.shape[0]
     rc = _lib.lib().spmla_index_logits_hist(
         q.data_ptr(), q.stride(0), q.stride(1), w.data_ptr(), w.stride(0), base.data_ptr(), R, rpb, bstride,
@@ -307,9 +306,8 @@ def logits_hist(q, w, base, R, rpb, bstride, block_table, block_size, req, ctx, 
 
 def logits_topk(q, w, store, block_table, block_size, req, ctx, Lc, K, lg=None, out=None, noinf=False,
                 dtype=torch.float32, ws=None):
-    """index_logits (P = 1) then topk of its [rows, Lc] logits, with the top-k's first histogram pass done in the
-    logits epilogue (logits_hist + topk_prehist) when it applies, else the two separate calls; same logits and
-    positions either way. Returns (logits, positions)."""
+    """index_logits (P = 1) then topk of its [rows, Lc] logits (logits_hist + topk_prehist, above 258048 columns
+    index_logits + topk; same logits and positions either way). Returns (logits, positions)."""
     rows, H, D = q.shape
     _need(q.dtype == torch.bfloat16 and q.stride(2) == 1, "q bf16 with contiguous head dim")
     _need(w.dtype == torch.float32 and w.stride(1) == 1, "w fp32")

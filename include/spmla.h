@@ -71,38 +71,33 @@ int spmla_topk(const void* logits, long long lg_st, const int* ctx, int rows, in
                long long out_st, int dtype, void* stream);
 
 /* Bytes of workspace spmla_topk_ws uses for rows x Lc (0 for invalid sizes): the per-row state, lists and histograms,
- * then the overflow lists (8 bytes per column) through which a narrowing level hands its boundary bin's keys to the
- * next level instead of that level reading the row again. */
+ * then the overflow lists (8 bytes per column) through which a narrowing level of rows above 262144 columns hands its
+ * boundary bin's keys to the next level instead of that level reading the row again. */
 long long spmla_topk_ws_bytes(int rows, int Lc, int K);
 
-/* spmla_topk with the same result, spread over several workgroups per row: a histogram pass and a collect pass over
- * chunks of 8192 or more columns (at most 4 chunks per row), then one workgroup per row that resolves the boundary bin
- * and sorts. ws: device memory of spmla_topk_ws_bytes(rows, Lc, K) bytes (a smaller one without the overflow lists is
- * accepted: the second level then reads the row again), 16-byte aligned, any contents (every pass writes what the
- * next reads); calls that share a workspace must not overlap. Same replacement as
- * spmla_topk (fast_topk.local + merge at P = 1, dotsnote/engine/arcstats_pkg/arcstats/fast_topk.py:52-78;
- * csrc/topk_select.cu:251-286; shard_indexer.py:194-221). */
+/* spmla_topk with the same result, long rows spread over several workgroups: rows of at most 32768 columns take
+ * spmla_topk's one workgroup, up to 262144 columns a workgroup per chunk of at most 32768 columns and one that selects
+ * among their lists, above that a histogram pass and two collect passes over 4 chunks and a finishing workgroup.
+ * ws: device memory of spmla_topk_ws_bytes(rows, Lc, K) bytes (a smaller one without the overflow lists is accepted),
+ * 16-byte aligned, any contents (every pass writes what the next reads); calls that share a workspace must not
+ * overlap. Same replacement as spmla_topk (fast_topk.local + merge at P = 1, dotsnote/engine/arcstats_pkg/arcstats/
+ * fast_topk.py:52-78; csrc/topk_select.cu:251-286; shard_indexer.py:194-221). */
 int spmla_topk_ws(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
                   long long out_st, void* ws, long long ws_bytes, int dtype, void* stream);
 
-/* spmla_index_logits (P = 1, rank 0) that also writes the first radix level of spmla_topk_ws into the top-k's
- * workspace ws (spmla_topk_ws_bytes(rows, Lc, K) bytes, 16-byte aligned): the logits workgroups cover the top-k's
- * column chunks and count the keys of the values they store in columns j < min(ctx[row], Lc), so the pass that would
- * re-read the logits for that histogram is not needed (spmla_topk_ws_prehist). Columns j < min(ctx, Lc) whose key
- * has no block-table entry are written -inf even with noinf != 0 (they are top-k columns). SPMLA_ELIMIT when a
- * chunk reaches 65536 columns (16-bit counts; Lc above 4 x 64512): use spmla_index_logits and spmla_topk_ws. The
- * reference computes the logits and then selects in separate calls (shard_indexer.py:63-91 then fast_topk.py:52-78 /
- * csrc/topk_select.cu:75-201 at P = 1, shard_indexer.py:194-221); the pair of entry points below is the same
- * computation with the selection's first pass done in the logits epilogue. */
+/* spmla_index_logits (P = 1, rank 0) for a top-k over the same rows, Lc and ctx that follows with workspace topk_ws
+ * (spmla_topk_ws_bytes(rows, Lc, K) bytes, 16-byte aligned): columns j < min(ctx[row], Lc) whose key has no block-table
+ * entry are written -inf even with noinf != 0 (they are top-k columns). The workspace is left as it is (the selection
+ * needs no histogram of the logits). SPMLA_ELIMIT for Lc above 4 x 64512: use spmla_index_logits and spmla_topk_ws.
+ * The reference computes the logits and then selects in separate calls (shard_indexer.py:63-91 then
+ * fast_topk.py:52-78 / csrc/topk_select.cu:75-201 at P = 1, shard_indexer.py:194-221). */
 int spmla_index_logits_hist(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
                             const void* store, long long R_local, int rows_per_block, long long block_stride,
                             const int* block_table, long long bt_st, int block_size, const int* req, const int* ctx,
                             int rows, int H, int D, int Lc, int noinf, void* out, long long out_st, int out_dtype,
                             void* topk_ws, long long ws_bytes, int K, void* stream);
 
-/* spmla_topk_ws whose workspace already holds the first-level histograms of these logits (written by
- * spmla_index_logits_hist with the same rows, Lc, K, ctx and dtype, and no other use of the workspace in between):
- * the histogram pass is skipped; same result as spmla_topk_ws. */
+/* spmla_topk_ws over the logits of spmla_index_logits_hist; same result. */
 int spmla_topk_ws_prehist(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
                           long long out_st, void* ws, long long ws_bytes, int dtype, void* stream);
 

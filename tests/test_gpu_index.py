@@ -375,3 +375,47 @@ def test_logits_f16_then_topk(dev):
                               bs, req.to(dev), ctx.to(dev), L, dtype=torch.float16)
     sel = kernels.topk(lg, ctx.to(dev), 2048).cpu().numpy()
     assert np.array_equal(sel, ref.topk(lg.cpu().numpy().astype(np.float32), ctx.numpy(), 2048))
+
+
+def _bucket_rows(L, seed):
+    """Rows that stress a selection by equal-width bins of the values: indexer-like, both signs, one far outlier, one
+    value in the whole row, three values, an exponential spread over 60 binades, -inf in front (a flat key range),
+    NaN and both infinities, subnormals, a boundary value held by 300 columns."""
+    g = np.random.RandomState(seed)
+    x = (40 + 4 * g.randn(10, L)).astype(np.float32)
+    x[1] = g.randn(L)
+    x[2, L // 3] = 1e30
+    x[3] = 2.5
+    x[4] = g.randint(0, 3, L)
+    x[5] = np.exp2(g.uniform(-30, 30, L)) * np.where(g.rand(L) < 0.5, -1, 1)
+    x[6, : L // 2] = -np.inf
+    x[7, ::7] = np.nan
+    x[7, 3::11] = np.inf
+    x[7, 5::13] = -np.inf
+    x[8] = g.randn(L) * 1e-39
+    x[9, g.permutation(L)[: min(300, L)]] = np.partition(x[9], -min(200, L))[-min(200, L)]
+    return x
+
+
+@pytest.mark.parametrize("L", [1, 5, 2047, 2049, 8191, 8193, 16384, 16387, 32768, 32769, 65537, 100003, 262144, 262147])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_topk_bucket_selection(dev, L, dtype):
+    """Edges of the top-k's routes (8 / 16 / 32 keys per thread, two and more chunks, the radix passes of longer rows)
+    over rows that fill its bins evenly, badly or not at all, with ragged row lengths and rows whose start is not
+    16-byte aligned: bit-exact against the oracle."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    src = torch.from_numpy(_bucket_rows(L, L % 1000))
+    lg = torch.where(torch.isinf(src) | torch.isnan(src), src.to(dtype), src.clamp(-60000, 60000).to(dtype)) \
+        if dtype == torch.float16 else src
+    lg = lg.numpy()
+    ctx = np.array([max(0, L - 3 * r) if r % 2 else L for r in range(lg.shape[0])], dtype=np.int32)
+    ctx[1] = min(L, 700)
+    for K in sorted({1, 300, 2048}):
+        print(f"[bucket] L={L} K={K} {dtype}", flush=True)
+        exp, dctx = ref.topk(lg, ctx, K), torch.from_numpy(ctx).to(dev)
+        for single in (False, True):
+            got = kernels.topk(torch.from_numpy(lg).to(dev), dctx, K, single_pass=single).cpu().numpy()
+            assert np.array_equal(got, exp), f"rows {np.where((got != exp).any(1))[0]} (single_pass={single})"
+        wide = torch.full((lg.shape[0], L + 5), 9.0, dtype=dtype, device=dev)      # rows at odd strides and offsets
+        wide[:, 3:3 + L] = torch.from_numpy(lg).to(dev)
+        assert np.array_equal(kernels.topk(wide[:, 3:3 + L], dctx, K).cpu().numpy(), exp)
