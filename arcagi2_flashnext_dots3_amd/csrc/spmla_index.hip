@@ -302,6 +302,194 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
   }
 }
 
+// ---- prefill logits over gathered keys (many query rows over the same keys) --------------------------------------
+// The kernel above reads and converts every key for every query row (2048 rows of 16384 keys: 786 us, a third of them
+// matrix-core time). Here a workgroup keeps 512 keys as bf16 MFMA operands in registers, 64 a wave (2
+// waves per SIMD), and runs up to 64 query rows past them: a row's 64 heads (16 KiB) and weights go through a 3-deep
+// LDS ring by LDS DMA, every wave reads them as the A operand (chunk c of head h at c ^ (h & 7): no bank conflicts) and
+// does 32 MFMAs a row, two head blocks by two key blocks; the ReLU and weighting of one product run under the
+// MFMAs of the next. Same products and sums in the same order as above. Rows whose range misses the 512 keys are only
+// filled. Bound by the matrix cores (32 x 32 cycles a row and wave) and, at 60%, the LDS reads; measured: 2048 rows of 16384
+// keys (15360 valid on average) 417 us.
+constexpr int FL_NWV = 8, FL_KEYS = 64 * FL_NWV;   // waves, keys of a workgroup
+constexpr int FL_RING = 3;
+constexpr int FL_ROWB = 64 * 256 + 256;            // a query row in LDS: 64 heads x 128 bf16, then 64 fp32 weights
+
+struct FlatParams {
+  const uint16_t* q; long long q_st, q_sh;
+  const float* w; long long w_st;
+  const uint8_t* k; long long k_st; const float* kscale;
+  const int* lo; const int* hi;                    // per row: first valid key, end of the valid keys
+  int M, N, rw;                                    // rows, keys, rows per workgroup (at most 64)
+  float* out; long long out_st;
+};
+
+__global__ void __launch_bounds__(FL_NWV * 64, 2) flat_logits_kernel(FlatParams p) {
+  __shared__ __attribute__((aligned(16))) uint8_t ring[FL_RING * FL_ROWB];
+  SPMLA_LDS uint8_t* lds = (SPMLA_LDS uint8_t*)ring;
+  const int ntile = (p.N + FL_KEYS - 1) / FL_KEYS, nchunk = (p.M + p.rw - 1) / p.rw;
+  const int f = remap_xcd(blockIdx.x, ntile * nchunk);      // an XCD's workgroups take the same rows past all keys
+  if (f < 0) return;
+  const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int m0 = f / ntile * p.rw, n0 = f % ntile * FL_KEYS;
+  const int key = n0 + 64 * wv + lane;                      // this lane's output column
+  // rows of the chunk: lane r holds row m0 + r's range
+  const int mr = m0 + lane;
+  const bool rok = lane < p.rw && mr < p.M;
+  const int lo_l = rok ? p.lo[mr] : 0, hi_l = rok ? p.hi[mr] : 0;
+  const bool act = rok && max(lo_l, n0) < min(hi_l, min(n0 + FL_KEYS, p.N));
+  uint64_t todo = __ballot(act), fill = __ballot(rok && !act);
+  auto put = [&](int r, float v) {                          // column `key` of row m0 + r (beyond N, r < 0: dropped)
+    const uint64_t a = (uint64_t)(uintptr_t)(p.out + (long long)(m0 + max(r, 0)) * p.out_st);
+    const uint32_t alo = __builtin_amdgcn_readfirstlane((uint32_t)a), ahi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(uintptr_t)(((uint64_t)ahi << 32) | alo), (short)0, r < 0 ? 0 : 4 * p.N, 0x00020000);
+    __builtin_amdgcn_raw_buffer_store_b32(f2u(v), rs, 4 * key, 0, 0);
+  };
+  for (; fill; fill &= fill - 1) put(__builtin_ctzll(fill), -__builtin_inff());
+  if (!todo) return;                                        // uniform over the workgroup
+
+  // copies of query row m0 + r into ring slot s: 64 heads, 2 KiB a wave, then 8 weights a wave (3 instructions)
+  auto issue = [&](int r, int s) {
+    SPMLA_LDS uint8_t* d = lds + s * FL_ROWB;
+    const uint16_t* qr = p.q + (long long)(m0 + r) * p.q_st;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int h = 4 * (2 * wv + i) + (lane >> 4);
+      dma16(qr + (long long)h * p.q_sh + 8 * ((lane & 15) ^ (h & 7)), d + (2 * wv + i) * 1024);
+    }
+    if (lane < 8) dma4(p.w + (long long)(m0 + r) * p.w_st + 8 * wv + lane, d + 64 * 256 + 32 * wv);
+  };
+  // row sequence: the set bits of todo, then the last one again (its copies are repeated, not used)
+  uint64_t ahead = todo;
+  int last = 0;
+  auto next_row = [&]() -> int {
+    if (ahead) { last = __builtin_ctzll(ahead); ahead &= ahead - 1; }
+    return last;
+  };
+#pragma unroll
+  for (int s = 0; s < FL_RING; ++s) issue(next_row(), s);
+
+  // this wave's keys: block b = keys n0 + 64 wv + 32 b + l32, dims in the order of the A operand's fragments
+  bf16x8 kf[2][8];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int kn = min(n0 + 64 * wv + 32 * b + l32, p.N - 1);
+    const uint8_t* src = p.k + (long long)kn * p.k_st + 16 * half;
+    u32x4 c[4];
+#pragma unroll
+    for (int kp = 0; kp < 4; ++kp) {
+      const u32x4u v = *(const u32x4u*)(src + 32 * kp);
+      c[kp] = u32x4{v[0], v[1], v[2], v[3]};
+    }
+#pragma unroll
+    for (int kp = 0; kp < 4; ++kp) {
+      i32x4 a0, a1;
+      a0[0] = (int)fp8lo_bf16x2(c[kp][0]); a0[1] = (int)fp8hi_bf16x2(c[kp][0]);
+      a0[2] = (int)fp8lo_bf16x2(c[kp][1]); a0[3] = (int)fp8hi_bf16x2(c[kp][1]);
+      a1[0] = (int)fp8lo_bf16x2(c[kp][2]); a1[1] = (int)fp8hi_bf16x2(c[kp][2]);
+      a1[2] = (int)fp8lo_bf16x2(c[kp][3]); a1[3] = (int)fp8hi_bf16x2(c[kp][3]);
+      kf[b][2 * kp] = __builtin_bit_cast(bf16x8, a0);
+      kf[b][2 * kp + 1] = __builtin_bit_cast(bf16x8, a1);
+    }
+  }
+  const float sc = p.kscale[min(key, p.N - 1)];
+
+  // A fragment ks = 2 kp + e of head block m: chunk 4 kp + 2 half + e of head 32 m + l32
+  auto load_a = [&](int s, int m, bf16x8 (&a)[8]) {
+    SPMLA_LDS uint8_t* d = lds + s * FL_ROWB + (32 * m + l32) * 256;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+      a[ks] = __builtin_bit_cast(bf16x8, *(SPMLA_LDS u32x4*)(d + 16 * ((4 * (ks >> 1) + 2 * half + (ks & 1)) ^ (l32 & 7))));
+  };
+  auto load_w = [&](int s, int m, f32x4 (&x)[4]) {          // weights of the C layout's rows 8 q + 4 half ..
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[q] = *(SPMLA_LDS f32x4*)(lds + s * FL_ROWB + 64 * 256 + (32 * m + 8 * q + 4 * half) * 4);
+  };
+  auto product = [&](const bf16x8 (&a)[8], const bf16x8 (&k)[8]) -> f32x16 {
+    f32x16 acc = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks], k[ks], acc, 0, 0, 0);
+    return acc;
+  };
+  auto weigh = [&](const f32x16& acc, const f32x4 (&x)[4]) -> float {   // sum of w * relu (an integer max: see above)
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float v = acc[i];
+      s = __builtin_fmaf(x[i >> 2][i & 3], __builtin_bit_cast(float, max(__builtin_bit_cast(int, v), 0)), s);
+    }
+    return s;
+  };
+  // one MFMA, then a slice of the previous product's 32 VALU instructions, eight times
+  auto interleave = [&]() {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+    }
+  };
+
+  wait_vm<0>();
+  lds_barrier();
+  bf16x8 a0[8], a1[8];
+  f32x4 w0[4], w1[4];
+  load_a(0, 0, a0);
+  load_w(0, 0, w0);
+  f32x16 x = f32x16{}, y = f32x16{};
+  float pa0 = 0.f, pa1 = 0.f, pb0 = 0.f;
+  int prow = -1, slot = 0;
+  auto finish = [&](float pb1) {                            // row prow's logits of the lane's key
+    const float s0 = pa0 + pb0, s1 = pa1 + pb1;
+    const auto t = __builtin_amdgcn_permlane32_swap(f2u(s0), f2u(s1), false, false);
+    const float v = (u2f(t[0]) + u2f(t[1])) * sc;           // lanes 0 .. 31: block 0's keys, the others block 1's
+    const int lo = __builtin_amdgcn_readlane(lo_l, max(prow, 0)), hi = __builtin_amdgcn_readlane(hi_l, max(prow, 0));
+    put(prow, key >= lo && key < hi ? v : -__builtin_inff());
+  };
+#pragma unroll 1
+  for (; todo; todo &= todo - 1) {
+    const int r = __builtin_ctzll(todo);
+    const int ns = slot == FL_RING - 1 ? 0 : slot + 1;
+    load_a(slot, 1, a1);
+    x = product(a0, kf[0]);
+    float pb1 = weigh(y, w1);                               // the previous row's last product
+    interleave();
+    asm volatile("" : "+v"(pb1));                           // (keeps the slices here)
+    __builtin_amdgcn_sched_barrier(0);
+    finish(pb1);                                            // (the first time round: dropped)
+    load_w(slot, 1, w1);
+    __builtin_amdgcn_sched_barrier(0);
+    y = product(a0, kf[1]);
+    pa0 = weigh(x, w0);
+    interleave();
+    asm volatile("" : "+v"(pa0));
+    __builtin_amdgcn_sched_barrier(0);
+    x = product(a1, kf[0]);
+    pa1 = weigh(y, w0);
+    interleave();
+    asm volatile("" : "+v"(pa1));
+    __builtin_amdgcn_sched_barrier(0);
+    // the next row's copies have landed (issued two rows ago: after them one row's copies and two stores) and this row
+    // is read by every wave: its slot takes the row after the next two
+    wait_vm<5>();
+    lds_barrier();
+    issue(next_row(), slot);
+    load_a(ns, 0, a0);
+    load_w(ns, 0, w0);
+    __builtin_amdgcn_sched_barrier(0);
+    y = product(a1, kf[1]);
+    pb0 = weigh(x, w1);
+    interleave();
+    asm volatile("" : "+v"(pb0));
+    __builtin_amdgcn_sched_barrier(0);
+    prow = r;
+    slot = ns;
+  }
+  finish(weigh(y, w1));
+  wait_vm<0>();                                             // no copy in flight when the LDS is given back
+}
+
 // ------------------------------------------------------------------------------------------------ top-k
 constexpr int TK_NT = 1024;
 constexpr int TK_KMAX = 2048;
@@ -1752,6 +1940,23 @@ inline dim3 lg_grid(int rows, int cols, int& tpg) {
 }
 
 
+// Rows per workgroup of flat_logits_kernel (0: the row-at-a-time kernel, which spreads a few rows over all compute
+// units). A workgroup takes 4.2 us for its keys and 1.33 us a row, one workgroup per compute unit at a time: the count
+// with the shortest rounds. Against the row-at-a-time kernel, including ~12 us of host time a call (us): 2048 x 16384 417
+// / 786, 256 x 16384 56 / 72, 64 x 16384 18 / 25, 16 x 65536 18 / 26, 64 x 4096 12 / 15, 2048 x 1024 32 / 76.
+inline int flat_rows(int M, int N) {
+  if (M < 8 || N > (1 << 28)) return 0;                     // (32-bit byte offsets in a row)
+  const long long tiles = (N + idx::FL_KEYS - 1) / idx::FL_KEYS;
+  int best = 0;
+  double cost = 0;
+  for (int rw = 64; rw >= 2; rw /= 2) {
+    const long long wgs = tiles * ((M + rw - 1) / rw);
+    const double c = (double)((wgs + lg_cus() - 1) / lg_cus()) * (4.2 + 1.33 * rw);
+    if (!best || c < cost) { best = rw; cost = c; }
+  }
+  return best;
+}
+
 extern "C" {
 
 static int logits_row(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
@@ -1854,6 +2059,14 @@ int spmla_mqa_logits(const void* q, long long q_st, long long q_sh, const float*
   if (((uintptr_t)q & 15) || (q_st & 7) || (q_sh & 7) || ((uintptr_t)k & 3) || (k_st & 3) || k_st < 128 ||
       ((uintptr_t)kscale & 3))
     return SPMLA_EALIGN;
+  if (const int rw = flat_rows(M, N)) {
+    const idx::FlatParams p{(const uint16_t*)q, q_st, q_sh, w, w_st, (const uint8_t*)k, k_st, kscale, ks, ke, M, N, rw,
+                            out, out_st};
+    const long long n = (long long)((N + idx::FL_KEYS - 1) / idx::FL_KEYS) * ((M + rw - 1) / rw);
+    hipLaunchKernelGGL(idx::flat_logits_kernel, dim3((unsigned)((n + 7) / 8 * 8)), dim3(idx::FL_NWV * 64), 0,
+                       (hipStream_t)stream, p);
+    return (int)hipGetLastError();
+  }
   idx::LogitParams p{};
   p.q = (const uint16_t*)q; p.q_st = q_st; p.q_sh = q_sh; p.w = w; p.w_st = w_st;
   p.store = (const uint8_t*)k; p.R_local = N; p.rpb = 1; p.blk_stride = 0;

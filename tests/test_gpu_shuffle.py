@@ -111,3 +111,40 @@ def test_mqa_logits_flat(dev):
     err = np.abs(got[fin] - exp[fin]) / np.maximum(1.0, np.abs(exp[fin]))
     print(f"[mqa logits] max rel err {err.max():.3e}", flush=True)
     assert err.max() <= 2e-5
+
+
+@pytest.mark.parametrize("M,N", [(8, 1), (9, 511), (33, 512), (130, 513), (300, 1537), (67, 9000)])
+def test_mqa_logits_many_rows(dev, M, N):
+    """The many-row kernel (512 keys a workgroup, up to 64 rows past them) against the row-at-a-time kernel, which
+    serves launches of fewer than 8 rows: bit for bit, over ranges that are empty, single keys, end inside a tile, miss a
+    workgroup's keys or reach past N, signed weights, strided queries and 132-byte key rows; and against the oracle."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    g = torch.Generator().manual_seed(M + N)
+    k = torch.randn(N, 128, generator=g).to(torch.bfloat16)
+    rows = np.zeros((N, 132), dtype=np.uint8)
+    ref.index_key_write(bf16_bits(k), np.arange(N), rows)
+    kd = torch.from_numpy(rows).to(dev)
+    scales = torch.from_numpy(rows[:, 128:].copy().view(np.float32)[:, 0].copy()).to(dev)
+    q = torch.randn(M, 64, 136, generator=g).to(torch.bfloat16).to(dev)[:, :, :128]
+    w = torch.randn(M, 64, generator=g).to(dev)
+    ks = torch.randint(0, N, (M,), generator=g).to(torch.int32)
+    ke = (ks + torch.randint(0, N, (M,), generator=g)).to(torch.int32)
+    ks[0], ke[0] = 0, N + 5
+    ks[1], ke[1] = N - 1, N
+    ke[2] = ks[2]
+    ks[3], ke[3] = 0, 1
+    print(f"[mqa logits] M={M} N={N}", flush=True)
+    got = kernels.mqa_logits(q, (kd[:, :128], scales), w, ks.to(dev), ke.to(dev))
+    one = torch.cat([kernels.mqa_logits(q[m:m + 7], (kd[:, :128], scales), w[m:m + 7], ks[m:m + 7].to(dev),
+                                        ke[m:m + 7].to(dev)) for m in range(0, M, 7)])
+    torch.cuda.synchronize()
+    assert torch.equal(got, one)
+    t = list(range(0, M, 29))
+    exp = ref.mqa_logits(q[t].float().cpu().numpy(), rows[:, :128], scales.cpu().numpy(), w[t].cpu().numpy(), ks[t].numpy(),
+                         ke[t].numpy())
+    fin = np.isfinite(exp)
+    assert np.array_equal(fin, np.isfinite(got[t].cpu().numpy()))
+    # 2e-5 of sum |w| times the standard deviation of q . k (sqrt(128)): the bar of the one-signed logits above, relative
+    # to the terms, since signed weights cancel
+    scale = np.broadcast_to(np.abs(w[t].cpu().numpy()).sum(1)[:, None] * 128 ** 0.5, exp.shape)
+    assert np.all(np.abs(got[t].cpu().numpy()[fin] - exp[fin]) <= 2e-5 * scale[fin])
