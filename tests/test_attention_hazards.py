@@ -1,0 +1,76 @@
+"""The attention kernel's inline-asm MFMA and DPP statements rely on the order of the compiled code instead of wait
+states, which the compiler does not add for asm: in the assembly of fwd_kernel no MFMA operand and no DPP source is
+written by the VALU in the two instructions before, and no VGPR result of an MFMA is read or overwritten before three
+more MFMAs were issued."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from arcagi2_flashnext_dots3_amd import build
+
+REG = re.compile(r"([av])(?:\[(\d+):(\d+)\]|(\d+))$")
+
+
+def _regs(tok):
+    m = REG.match(tok)
+    if not m:
+        return set()
+    lo, hi = (m[4], m[4]) if m[4] else (m[2], m[3])
+    return {(m[1], i) for i in range(int(lo), int(hi) + 1)}
+
+
+def hazards(lines):
+    """[(line, text)] of the violations in one kernel's assembly."""
+    bad, hist, mfma = [], [], []
+    for n, l in enumerate(lines):
+        l = l.split(";")[0].strip()
+        if not l or l.startswith(".") or l.endswith(":"):
+            continue
+        op, _, rest = l.partition(" ")
+        toks = [t.strip().split(" ")[0] for t in re.split(r",\s*(?![^\[]*\])", rest)]
+        dst = _regs(toks[0])
+        stores = op.startswith(("ds_write", "global_store", "scratch_store"))
+        src = set().union(*map(_regs, toks if stores else toks[1:]))
+        need = set().union(*map(_regs, toks[1:3])) if "mfma" in op else _regs(toks[1]) if "_dpp" in op else set()
+        states = 0
+        for o, d, imm in reversed(hist[-4:]):
+            states += int(imm, 0) if o == "s_nop" else 0
+            if o.startswith("v_") and "mfma" not in o and d & need and states < 2:
+                bad.append((n, l))
+            states += 1
+        if "mfma" in op:
+            mfma.append(dst)
+        else:
+            touched = {r for r in src | (dst if op.startswith("v_") else set()) if r[0] == "v"}
+            if any(touched & d for d in mfma[-3:]):
+                bad.append((n, l))
+        hist.append((op, set() if stores else dst, toks[0]))
+    return bad
+
+
+def test_scanner_finds_planted_hazards():
+    ok = ["v_add_f32_e32 v1, v2, v3", "s_nop 1", "v_mul_f32_dpp v4, v1, v5 quad_perm:[0,0,0,0]"]
+    assert not hazards(ok)
+    assert hazards([ok[0], ok[2]])
+    m = "v_mfma_f32_32x32x16_bf16 v[16:31], v[0:3], v[4:7], 0"
+    assert hazards(["v_mov_b32_e32 v5, v9", "s_nop 0", m])
+    a = "v_mfma_f32_32x32x16_f16 a[0:15], v[40:43], v[44:47], a[0:15]"
+    assert hazards([m, a, a, "ds_write_b128 v9, v[16:19] offset:64"])
+    assert not hazards([m, a, a, a, "ds_write_b128 v9, v[16:19] offset:64"])
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no hipcc")
+def test_compiled_order_of_asm_statements(tmp_path):
+    out = tmp_path / "attn.s"
+    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, "spmla_attn.hip"),
+                    "-o", str(out)], check=True, capture_output=True)
+    text = out.read_text().split("\n")
+    starts = [i for i, l in enumerate(text) if re.match(r"_ZN5spmla4attn10fwd_kernelILb[01]EEE\S*:", l)]
+    assert len(starts) == 2
+    for s in starts:
+        end = next(i for i in range(s, len(text)) if ".Lfunc_end" in text[i])
+        body = text[s:end]
+        assert sum("v_mfma_f32_32x32x16_bf16" in l for l in body) >= 36
+        assert not hazards(body)
