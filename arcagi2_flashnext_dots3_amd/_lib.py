@@ -63,6 +63,7 @@ SIGNATURES = {
     "spmla_index_key_write_shuffle": [P, LL, P, I, P, LL, I, LL, I, P],
     "spmla_mqa_logits": [P, LL, LL, P, LL, P, LL, P, I, P, P, I, I, I, P, LL, P],
     "spmla_paged_mqa_logits": [P, LL, LL, P, LL, P, LL, I, LL, P, LL, P, P, I, I, I, I, I, P, LL, P],
+    "spmla_paged_mqa_logits_seq": [P, LL, LL, P, LL, P, LL, I, LL, P, LL, P, I, I, I, I, I, I, I, P, LL, P],
     "spmla_version": [],
     "spmla_host_e4m3_encode": [P, P, LL],
 }

@@ -52,6 +52,9 @@ struct LogitParams {
   const uint8_t* store; long long R_local; int rpb; long long blk_stride;
   const int* bt; long long bt_st; int bs;    // block table [req][...], block size (positions per block)
   const int* req; const int* ctx;            // per row
+  // per > 0 (req null): rows per request, row r belongs to request r / per; tail: ctx is per request and row r sees
+  // per - 1 - r % per keys less
+  int per, tail;
   int rows, Lc, P, rank, noinf;
   void* out; long long out_st;              // fp32, or fp16 (F16OUT); stride in elements
   int bs_sh, rpb_sh, p_sh;                   // log2 of bs, rpb, P when a power of two, else -1
@@ -105,7 +108,8 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
   const int lane = threadIdx.x & 63;
   const bool stage = 32LL * p.tpg <= LG_STAGE;              // uniform
   const int half = lane >> 5, l32 = lane & 31;
-  const int ctx = p.ctx[row];
+  const int rq = FLAT ? 0 : p.per ? row / p.per : p.req[row];
+  const int ctx = p.tail ? p.ctx[rq] - (p.per - 1 - (row - rq * p.per)) : p.ctx[row];
   float* orow = (float*)p.out + (long long)row * p.out_st;            // fp32 output row
   _Float16* hrow = (_Float16*)p.out + (long long)row * p.out_st;      // fp16 output row
   auto put = [&](int j, float v) {
@@ -124,7 +128,7 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
   if (tv <= tb) return;                                     // uniform over the workgroup: no barrier below
   if (threadIdx.x == 0) claim = tb + 2 * LG_D * LG_NWV;     // steps 0 .. 2 LG_D - 1 take tiles tb + k NW + w
   __syncthreads();
-  const int* btr = FLAT ? nullptr : p.bt + (long long)p.req[row] * p.bt_st;
+  const int* btr = FLAT ? nullptr : p.bt + (long long)rq * p.bt_st;
   const int lo = p.lo ? p.lo[row] : 0;
   // n / d, n % d: shifts when every divisor is a power of two (POW2), else 32-bit division
   auto dv = [&](uint32_t n, uint32_t d, int sh) -> uint32_t { return POW2 ? n >> sh : n / d; };
@@ -2019,15 +2023,16 @@ int spmla_index_logits_hist(const void* q, long long q_st, long long q_sh, const
                     block_size, req, ctx, rows, H, D, Lc, 1, 0, noinf, out, out_st, out_dtype, stream, 1);
 }
 
-int spmla_paged_mqa_logits(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
-                           const void* cache, long long num_blocks, int block_size, long long block_stride,
-                           const int* block_table, long long bt_st, const int* req, const int* ctx, int rows, int H,
-                           int D, int Lc, int noinf, float* out, long long out_st, void* stream) {
+// per, tail: see LogitParams
+static int paged_launch(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
+                        const void* cache, long long num_blocks, int block_size, long long block_stride,
+                        const int* block_table, long long bt_st, const int* req, const int* ctx, int per, int tail,
+                        int rows, int H, int D, int Lc, int noinf, float* out, long long out_st, void* stream) {
   if (rows < 0 || Lc < 0 || block_size <= 0 || (block_size & 15) || num_blocks < 0) return SPMLA_EARG;
   if (rows == 0 || Lc == 0) return SPMLA_OK;
   if (H != 64 || D != 128) return SPMLA_ELIMIT;
   if (num_blocks > (long long)INT_MAX / block_size) return SPMLA_ELIMIT;
-  if (!q || !w || !cache || !block_table || !req || !ctx || !out) return SPMLA_EARG;
+  if (!q || !w || !cache || !block_table || !(req || per) || !ctx || !out) return SPMLA_EARG;
   if (((uintptr_t)q & 15) || (q_st & 7) || (q_sh & 7) || ((uintptr_t)cache & 3) || (block_stride & 3) ||
       block_stride < (long long)block_size * 132)
     return SPMLA_EALIGN;
@@ -2035,6 +2040,7 @@ int spmla_paged_mqa_logits(const void* q, long long q_st, long long q_sh, const 
   p.q = (const uint16_t*)q; p.q_st = q_st; p.q_sh = q_sh; p.w = w; p.w_st = w_st;
   p.store = (const uint8_t*)cache; p.R_local = num_blocks * block_size; p.rpb = block_size;
   p.blk_stride = block_stride; p.bt = block_table; p.bt_st = bt_st; p.bs = block_size; p.req = req; p.ctx = ctx;
+  p.per = per; p.tail = tail;
   p.rows = rows; p.Lc = Lc; p.P = 1; p.rank = 0; p.noinf = noinf; p.out = out; p.out_st = out_st;
   auto log2_or = [](long long v) { return (v & (v - 1)) == 0 ? __builtin_ctzll((unsigned long long)v) : -1; };
   p.bs_sh = log2_or(block_size); p.rpb_sh = p.bs_sh; p.p_sh = 0;
@@ -2047,6 +2053,23 @@ int spmla_paged_mqa_logits(const void* q, long long q_st, long long q_sh, const 
   else
     hipLaunchKernelGGL((idx::logits_kernel<false, idx::LY_SHUF>), grid, dim3(idx::LG_NWV * 64), 0, (hipStream_t)stream, p);
   return (int)hipGetLastError();
+}
+
+int spmla_paged_mqa_logits(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
+                           const void* cache, long long num_blocks, int block_size, long long block_stride,
+                           const int* block_table, long long bt_st, const int* req, const int* ctx, int rows, int H,
+                           int D, int Lc, int noinf, float* out, long long out_st, void* stream) {
+  return paged_launch(q, q_st, q_sh, w, w_st, cache, num_blocks, block_size, block_stride, block_table, bt_st, req, ctx,
+                      0, 0, rows, H, D, Lc, noinf, out, out_st, stream);
+}
+
+int spmla_paged_mqa_logits_seq(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
+                               const void* cache, long long num_blocks, int block_size, long long block_stride,
+                               const int* block_table, long long bt_st, const int* seq_lens, int per_row, int next_n,
+                               int rows, int H, int D, int Lc, int noinf, float* out, long long out_st, void* stream) {
+  if (next_n <= 0) return SPMLA_EARG;
+  return paged_launch(q, q_st, q_sh, w, w_st, cache, num_blocks, block_size, block_stride, block_table, bt_st, nullptr,
+                      seq_lens, next_n, per_row == 0, rows, H, D, Lc, noinf, out, out_st, stream);
 }
 
 int spmla_mqa_logits(const void* q, long long q_st, long long q_sh, const float* w, long long w_st, const void* k,

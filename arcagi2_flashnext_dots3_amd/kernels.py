@@ -117,13 +117,14 @@ def paged_mqa_logits(q, kv_cache, weights, seq_lens, block_table, max_model_len,
     _need(weights.dtype == torch.float32 and weights.stride(1) == 1, "weights fp32")
     _need(block_table.dtype == torch.int32, "int32 block table")
     nb, bs, bstride = _shuffle_cache(kv_cache)
-    req, ctx = paged_ctx(seq_lens, nn)
+    seq = seq_lens.to(torch.int32).contiguous()
     rows = B * nn
     if out is None:
         out = torch.empty(rows, max(max_model_len, 1), dtype=torch.float32, device=q.device)
-    _lib.call("spmla_paged_mqa_logits", qr.data_ptr(), qr.stride(0), qr.stride(1), weights.data_ptr(),
+    _lib.call("spmla_paged_mqa_logits_seq", qr.data_ptr(), qr.stride(0), qr.stride(1), weights.data_ptr(),
               weights.stride(0), kv_cache.data_ptr(), nb, bs, bstride, block_table.data_ptr(), block_table.stride(0),
-              req.data_ptr(), ctx.data_ptr(), rows, H, D, max_model_len, 0, out.data_ptr(), out.stride(0), _stream(q))
+              seq.data_ptr(), int(seq.dim() == 2), max(nn, 1), rows, H, D, max_model_len, 0, out.data_ptr(),
+              out.stride(0), _stream(q))
     return out
 
 

@@ -393,11 +393,18 @@ int spmla_index_key_write_shuffle(const void* k, long long k_st, const long long
  * relu(q[row][h] . kcode) * kscale for positions j < ctx[row] (key block block_table[req[row]][j / block_size]),
  * -inf beyond (noinf: left unwritten). H = 64, D = 128, q bf16.
  * Replaces paged_mqa_logits_triton / _paged_logits_kernel (dotsnote/engine/arcstats_pkg/arcstats/dsa_sm89.py:41-94),
- * the decode logits of the reference's default indexer path; the host wrapper builds req / ctx for next_n > 1. */
+ * the decode logits of the reference's default indexer path, with the rows' requests and contexts given. */
 int spmla_paged_mqa_logits(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
                            const void* cache, long long num_blocks, int block_size, long long block_stride,
                            const int* block_table, long long bt_st, const int* req, const int* ctx, int rows, int H,
                            int D, int Lc, int noinf, float* out, long long out_st, void* stream);
+
+/* spmla_paged_mqa_logits with the rows' requests and contexts formed in the kernel: row r belongs to request
+ * r / next_n and sees seq_lens[r] keys (per_row), else seq_lens[r / next_n] - (next_n - 1 - r % next_n). */
+int spmla_paged_mqa_logits_seq(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
+                               const void* cache, long long num_blocks, int block_size, long long block_stride,
+                               const int* block_table, long long bt_st, const int* seq_lens, int per_row, int next_n,
+                               int rows, int H, int D, int Lc, int noinf, float* out, long long out_st, void* stream);
 
 /* Prefill indexer logits over gathered keys: out[m][n] = sum_h w[m][h] * relu(q[m][h] . kcode[n]) * kscale[n] for
  * ks[m] <= n < ke[m], -inf for the other n < N (no clamp). Key n's 128 e4m3 codes at k + n * k_st bytes, its fp32

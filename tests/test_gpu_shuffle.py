@@ -148,3 +148,31 @@ def test_mqa_logits_many_rows(dev, M, N):
     # to the terms, since signed weights cancel
     scale = np.broadcast_to(np.abs(w[t].cpu().numpy()).sum(1)[:, None] * 128 ** 0.5, exp.shape)
     assert np.all(np.abs(got[t].cpu().numpy()[fin] - exp[fin]) <= 2e-5 * scale[fin])
+
+
+@pytest.mark.parametrize("B,nn,two_d,dtype", [(3, 2, False, torch.int64), (3, 4, True, torch.int32), (5, 1, False, torch.int32)])
+def test_paged_logits_rows_formed_in_the_kernel(dev, B, nn, two_d, dtype):
+    """spmla_paged_mqa_logits_seq (the wrapper) against spmla_paged_mqa_logits with explicit per-row requests and
+    contexts: the same bits; a context shorter than next_n leaves its first rows without keys."""
+    from arcagi2_flashnext_dots3_amd import _lib, kernels
+    bs, L = 16, 130
+    nbp = (L + bs - 1) // bs
+    g = torch.Generator().manual_seed(B * nn)
+    cache = torch.zeros(B * nbp, bs, 132, dtype=torch.uint8, device=dev)
+    kernels.index_key_write_shuffle(torch.randn(B * nbp * bs, 128, generator=g).to(torch.bfloat16).to(dev),
+                                    torch.arange(B * nbp * bs, device=dev), cache)
+    bt = torch.randperm(B * nbp, generator=g).view(B, nbp).to(torch.int32).to(dev)
+    q = torch.randn(B, nn, 64, 128, generator=g).to(torch.bfloat16).to(dev)
+    w = torch.rand(B * nn, 64, generator=g).to(dev)
+    sl = torch.randint(1, L + 1, (B, nn) if two_d else (B,), generator=g).to(dtype)
+    sl.view(-1)[0] = 1
+    sl = sl.to(dev)
+    print(f"[paged logits] B={B} next_n={nn} 2d={two_d}", flush=True)
+    a = kernels.paged_mqa_logits(q, cache, w, sl, bt, L)
+    req, ctx = kernels.paged_ctx(sl, nn)
+    b = torch.empty_like(a)
+    _lib.call("spmla_paged_mqa_logits", q.data_ptr(), q.stride(1), q.stride(2), w.data_ptr(), w.stride(0),
+              cache.data_ptr(), B * nbp, bs, cache.stride(0), bt.data_ptr(), bt.stride(0), req.data_ptr(), ctx.data_ptr(),
+              B * nn, 64, 128, L, 0, b.data_ptr(), b.stride(0), kernels._stream(q))
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
