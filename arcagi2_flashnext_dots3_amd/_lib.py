@@ -73,6 +73,7 @@ _RESTYPE = {"spmla_version": ctypes.c_char_p, "spmla_host_e4m3_encode": None, "s
 ERRORS = {-2: "bad argument", -3: "misaligned pointer or stride", -5: "size beyond the kernel's limit"}
 
 _L = None
+_FN = {}      # entry point -> callable: _native's, else ctypes'
 
 
 def lib():
@@ -86,13 +87,23 @@ def lib():
             f = getattr(L, name)
             f.argtypes = args
             f.restype = _RESTYPE.get(name, ctypes.c_int)
+        _FN.update({name: getattr(L, name) for name in SIGNATURES})
+        try:
+            from . import _native
+            _FN.update(_native.load(LIB_PATH))
+        except ImportError:      # built without Python's headers
+            pass
         _L = L
     return _L
 
 
 def call(name, *args):
     """Invoke entry point `name`; a nonzero return code raises RuntimeError naming the entry point."""
-    rc = getattr(lib(), name)(*args)
+    f = _FN.get(name) or getattr(lib(), name)
+    try:
+        rc = f(*args)
+    except TypeError:            # not ints, floats and None: ctypes takes it or refuses it
+        rc = getattr(lib(), name)(*args)
     if rc != 0:
         raise RuntimeError(f"{name} failed: {rc} ({ERRORS.get(rc, 'hip error')})")
     return rc

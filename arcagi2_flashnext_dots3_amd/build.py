@@ -2,17 +2,23 @@
 
 Every .hip file under csrc/ is compiled to an object (in parallel) and linked into one shared library next to
 this file; the Python loader (_lib.py) and the tests load that file. Objects go to _build/ (git-ignored).
+csrc/py_call.cpp becomes the extension module _native (the loader's callables; without Python's headers or a C++
+compiler it is left out and the loader calls through ctypes).
 All HIP code is compiled with packed fp32 instructions disabled (-packed-fp32-ops), see the feature flag below.
 """
 import concurrent.futures
 import os
+import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 REPO = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libspmla_gfx950.so")
+NATIVE = os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
+CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
@@ -25,6 +31,19 @@ def _run(cmd):
     if r.returncode != 0:
         raise RuntimeError(f"build failed: {' '.join(cmd)}\n{err}")
     return err
+
+
+def build_native():
+    inc = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(inc, "Python.h")) or shutil.which(CXX.split()[0]) is None:
+        if os.path.exists(NATIVE):
+            os.remove(NATIVE)
+        return None
+    tmp = NATIVE + ".tmp"
+    _run([*CXX.split(), "-O2", "-std=c++17", "-shared", "-fPIC", "-I", inc, "-I", os.path.join(REPO, "include"),
+          os.path.join(CSRC, "py_call.cpp"), "-o", tmp, "-ldl"])
+    os.replace(tmp, NATIVE)
+    return NATIVE
 
 
 def build(verbose=False):
@@ -42,6 +61,7 @@ def build(verbose=False):
     tmp = LIB + ".tmp"
     _run([HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", tmp, *objs])
     os.replace(tmp, LIB)
+    build_native()
     return LIB
 
 

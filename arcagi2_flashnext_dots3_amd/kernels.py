@@ -16,8 +16,20 @@ _ROWB = {0: ROW656, 1: ROW576, 2: ROW400}        # cache_write formats
 LOG2E = 1.4426950408889634
 
 
+# device index -> the current stream's handle (torch.cuda.current_stream builds a Stream object: 1.5 us a call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t):
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
+
+
+def _device_stream(dev):
+    if _raw_stream is not None and dev.type == "cuda" and dev.index is not None:
+        return _raw_stream(dev.index)
+    return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _ptr(t):
@@ -34,12 +46,16 @@ def cache_write(kv_c, k_pe, slots, cache, fmt=0, kv_scale=1.0, block_size=None, 
     """kv_c [n, 512] bf16, k_pe [n, 64] or [n, 1, 64] bf16, slots [n] int64 -> rows of `cache` (uint8, Row656
     (fmt 0), Row576 (fmt 1) or Row400 (fmt 2, the compact e2m2b32 row)). cache is [R, row] or paged
     [blocks, block_size, row] (block stride may be padded)."""
-    kpe = k_pe.reshape(k_pe.shape[0], -1)
+    if k_pe.dim() == 3 and k_pe.shape[1] == 1 and k_pe.shape[0]:
+        kpe, kpe_w = k_pe, k_pe.shape[2]
+    else:
+        kpe = k_pe.reshape(k_pe.shape[0], -1)
+        kpe_w = kpe.shape[1]
     n = min(kv_c.shape[0], slots.shape[0])
     _need(fmt in _ROWB, f"fmt must be one of {sorted(_ROWB)}")
     rowb = _ROWB[fmt]
     _need(kv_c.dtype == torch.bfloat16 and kpe.dtype == torch.bfloat16, "kv_c / k_pe must be bf16")
-    _need(kv_c.shape[1] == D_LAT and kpe.shape[1] == D_ROPE and kv_c.stride(1) == 1 and kpe.stride(1) == 1,
+    _need(kv_c.shape[1] == D_LAT and kpe_w == D_ROPE and kv_c.stride(1) == 1 and kpe.stride(-1) == 1,
           "kv_c [n, 512] / k_pe [n, 64] with contiguous rows")
     _need(cache.dtype == torch.uint8 and cache.shape[-1] == rowb and cache.stride(-1) == 1, "cache rows of uint8")
     _need(slots.dtype == torch.int64, "slots int64")
@@ -202,7 +218,7 @@ def _workspace(kind, device, nbytes, zero=False):
               f"{kind} workspace of {nbytes} bytes needed under HIP graph capture: pass one explicitly, or make an "
               f"eager call of at least this size (reserve_workspace) before capturing")
         return b, None
-    key = (kind, dev, torch.cuda.current_stream(dev).cuda_stream)
+    key = (kind, dev, _device_stream(dev))
     b = _WS.get(key)
     if b is None or b.numel() < nbytes:
         n = max(nbytes, 256, 2 * b.numel() if b is not None else 0)
@@ -224,7 +240,7 @@ def reserve_workspace(device, H, T=None, split=8):
     (default: every size auto_split sends there), so that later HIP graph captures find it. No-op when present."""
     T = fused_max_tokens(H) if T is None else T
     if T > 0:
-        _workspace("attn", device, int(_lib.lib().spmla_attn_ws_bytes(T, H, split)), zero=True)
+        _workspace("attn", device, attn_ws_bytes(T, H, split), zero=True)
 
 
 def _attn_workspace(device, T, H, split, private=False):
@@ -250,6 +266,12 @@ def _attn_counter_bytes(T, H):
     return (4 * T * ((H + 127) // 128) + 255) // 256 * 256
 
 
+@functools.lru_cache(maxsize=4096)
+def topk_ws_bytes(rows, Lc, K):
+    """Bytes of the workspace topk needs (spmla_topk_ws_bytes)."""
+    return int(_lib.lib().spmla_topk_ws_bytes(rows, Lc, K))
+
+
 def topk(logits, ctx, K, out=None, single_pass=False, ws=None):
     """logits [rows, Lc] fp32 or fp16, ctx [rows] int32 -> [rows, K] int32 positions (value desc, position asc; -1
     pad). Several workgroups per row (spmla_topk_ws; ws: a uint8 workspace, else a cached one of
@@ -265,9 +287,8 @@ def topk(logits, ctx, K, out=None, single_pass=False, ws=None):
         _lib.call("spmla_topk", logits.data_ptr(), logits.stride(0), ctx.data_ptr(), rows, Lc, K, out.data_ptr(),
                   out.stride(0), _LG_DT[logits.dtype], _stream(logits))
         return out
-    nb = int(_lib.lib().spmla_topk_ws_bytes(rows, Lc, K))
     if ws is None:
-        ws, _ = _workspace("topk", logits.device, nb)
+        ws, _ = _workspace("topk", logits.device, topk_ws_bytes(rows, Lc, K))
     _lib.call("spmla_topk_ws", logits.data_ptr(), logits.stride(0), ctx.data_ptr(), rows, Lc, K, out.data_ptr(),
               out.stride(0), ws.data_ptr(), ws.numel(), _LG_DT[logits.dtype], _stream(logits))
     return out
@@ -293,7 +314,8 @@ def logits_hist(q, w, base, R, rpb, bstride, block_table, block_size, req, ctx, 
     min(ctx, Lc) written. Returns False without a launch above 258048 columns; the caller then runs the logits and topk
     separately."""
     rows = q.shape[0]
-    rc = _lib.lib().spmla_index_logits_hist(
+    _lib.lib()
+    rc = _lib._FN["spmla_index_logits_hist"](
         q.data_ptr(), q.stride(0), q.stride(1), w.data_ptr(), w.stride(0), base.data_ptr(), R, rpb, bstride,
         block_table.data_ptr(), block_table.stride(0), block_size, req.data_ptr(), ctx.data_ptr(), rows, q.shape[1],
         q.shape[2], Lc, int(bool(noinf)), lg.data_ptr(), lg.stride(0), _LG_DT[lg.dtype], ws.data_ptr(), ws.numel(),
@@ -330,7 +352,7 @@ def logits_topk(q, w, store, block_table, block_size, req, ctx, Lc, K, lg=None, 
         return lg, out
     lgv = lg[:rows, :Lc]
     if ws is None:
-        ws, _ = _workspace("topk", q.device, int(_lib.lib().spmla_topk_ws_bytes(rows, Lc, K)))
+        ws, _ = _workspace("topk", q.device, topk_ws_bytes(rows, Lc, K))
     if logits_hist(q, w, store, R, rpb, bstride, block_table, block_size, req, ctx, Lc, K, lg, ws, noinf):
         topk_prehist(lgv, ctx, K, ws, out=out)
     else:
@@ -642,11 +664,17 @@ def compact_stage(rows, sidx, workspace=None):
 
 
 # ---------------------------------------------------------------------------------------------- attention
+def query_ok(q):
+    """The query's part of attention_ok."""
+    if q.dtype != torch.bfloat16 or q.dim() != 3 or q.shape[2] != D_QK:
+        return False
+    st, sh, sd = q.stride()
+    return sd == 1 and q.data_ptr() % 16 == 0 and st % 8 == 0 and sh % 8 == 0
+
+
 def attention_ok(q, idx):
     """Preconditions of spmla_attn_splitk (the reference's offload_cuda2.ok analogue)."""
-    return (q.dtype == torch.bfloat16 and q.dim() == 3 and q.shape[2] == D_QK and q.stride(2) == 1
-            and q.data_ptr() % 16 == 0 and q.stride(0) % 8 == 0 and q.stride(1) % 8 == 0
-            and idx.dtype == torch.int32 and idx.stride(1) == 1)
+    return query_ok(q) and idx.dtype == torch.int32 and idx.stride(1) == 1
 
 
 ATTN_SPLIT_ROWS = 2048      # rows of one (token, split) in spmla_attn's split merge, rounded up to 32-row tiles
@@ -679,6 +707,7 @@ def auto_split(T, H, K, cus=256):
     return 1 if -(-(-(-K // s)) // 32) * 32 > ATTN_SPLIT_ROWS else s
 
 
+@functools.lru_cache(maxsize=4096)
 def attn_ws_bytes(T, H, split):
     """Bytes of the workspace attend needs for T tokens, H heads and `split` splits (0 for split 1)."""
     return int(_lib.lib().spmla_attn_ws_bytes(T, H, split))
@@ -726,7 +755,7 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
                   out.stride(0), out.stride(1), lse.data_ptr(), lse.stride(0), None, None, st)
         return out, lse
     _need(1 <= split <= 8, "attend: split must be 1 .. 8")
-    nb = int(_lib.lib().spmla_attn_ws_bytes(T, H, split))
+    nb = attn_ws_bytes(T, H, split)
     if ws is None:
         # from 96 workgroups on (3/8 of the compute units) the unsplit launch needs none: a capture brings its own
         ws = _attn_workspace(q.device, T, H, split, private=T * ((H + 31) // 32) >= 96)
@@ -809,10 +838,10 @@ def bmm_fp8(a, codes, scales, scale_k, out):
     _need(codes.dtype in (torch.uint8, torch.float8_e4m3fn) and codes.shape[0] == N and codes.shape[2] == K,
           "codes [N, J, K] e4m3")
     _need(scales.dtype == torch.float32, "scales fp32")
-    _need(out.dtype in (torch.bfloat16, torch.float32) and tuple(out.shape) == (N, B, J), "out [N, B, J]")
-    _lib.call("spmla_bmm_fp8", a.data_ptr(), a.stride(0), a.stride(1), a.stride(2), codes.data_ptr(), codes.stride(0),
-              codes.stride(1), codes.stride(2), scales.data_ptr(), scales.stride(0), scales.stride(1),
-              scales.stride(2), int(bool(scale_k)), out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
+    _need(out.dtype in (torch.bfloat16, torch.float32) and out.shape == (N, B, J), "out [N, B, J]")
+    cs, ss = codes.stride(), scales.stride()
+    _lib.call("spmla_bmm_fp8", a.data_ptr(), *a.stride(), codes.data_ptr(), cs[0], cs[1], cs[2], scales.data_ptr(),
+              ss[0], ss[1], ss[2], int(bool(scale_k)), out.data_ptr(), *out.stride(),
               int(out.dtype == torch.float32), N, B, J, K, _stream(a))
     return out
 
@@ -820,16 +849,17 @@ def bmm_fp8(a, codes, scales, scale_k, out):
 def mla_query(q_nope, q_pe, codes_uk, scales_uk, out=None):
     """The decode query of the sparse attention in one launch: out[t, h, :512] = q_nope[t, h] @ W_UK_T[h] (FP8
     weights, codes [H, 512, 128], scales [H, 128, 4]), out[t, h, 512:] = q_pe[t, h]."""
-    T, H, _ = q_nope.shape
-    _need(q_nope.dtype == torch.bfloat16 and q_nope.shape[2] == 128 and q_nope.stride(2) == 1, "q_nope [T, H, 128]")
-    _need(q_pe.dtype == torch.bfloat16 and tuple(q_pe.shape) == (T, H, 64) and q_pe.stride(2) == 1, "q_pe [T, H, 64]")
-    _need(tuple(codes_uk.shape) == (H, 512, 128) and codes_uk.is_contiguous(), "codes_uk [H, 512, 128]")
-    _need(tuple(scales_uk.shape) == (H, 128, 4) and scales_uk.is_contiguous() and scales_uk.dtype == torch.float32,
+    T, H, d = q_nope.shape
+    n_st, n_sh, n_sd = q_nope.stride()
+    _need(q_nope.dtype == torch.bfloat16 and d == 128 and n_sd == 1, "q_nope [T, H, 128]")
+    _need(q_pe.dtype == torch.bfloat16 and q_pe.shape == (T, H, 64) and q_pe.stride(2) == 1, "q_pe [T, H, 64]")
+    _need(codes_uk.shape == (H, 512, 128) and codes_uk.is_contiguous(), "codes_uk [H, 512, 128]")
+    _need(scales_uk.shape == (H, 128, 4) and scales_uk.is_contiguous() and scales_uk.dtype == torch.float32,
           "scales_uk [H, 128, 4] fp32")
     if out is None:
         out = torch.empty(T, H, D_QK, dtype=torch.bfloat16, device=q_nope.device)
-    _need(out.dtype == torch.bfloat16 and tuple(out.shape) == (T, H, D_QK) and out.stride(2) == 1, "out [T, H, 576]")
-    _lib.call("spmla_mla_query", q_nope.data_ptr(), q_nope.stride(0), q_nope.stride(1), q_pe.data_ptr(),
+    _need(out.dtype == torch.bfloat16 and out.shape == (T, H, D_QK) and out.stride(2) == 1, "out [T, H, 576]")
+    _lib.call("spmla_mla_query", q_nope.data_ptr(), n_st, n_sh, q_pe.data_ptr(),
               q_pe.stride(0), q_pe.stride(1), codes_uk.data_ptr(), scales_uk.data_ptr(), T, H, out.data_ptr(),
               out.stride(0), out.stride(1), _stream(q_nope))
     return out
