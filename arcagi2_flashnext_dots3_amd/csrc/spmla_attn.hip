@@ -30,7 +30,7 @@
 // registers) issues about one instruction per 4 cycles (8-byte ones 4.6, scalar ones 8: measured), 620 (Row656) or 480
 // per tile next to 68 MFMAs; matrix cores are busy 41 - 45 % of the time, LDS 30 %. Hence addresses that are a register
 // plus immediates, no wait states where none are needed, no scalar work per slice.
-// T = 2048, H = 128, K = 2048: Row656 1330 us (880 TFLOP/s), before (heads split over the waves) 1580 us; Row576 1155 us,
+// T = 2048, H = 128, K = 2048: Row656 1304 us (896 TFLOP/s), before (heads split over the waves) 1580 us; Row576 1160 us,
 // before (head-group kernel) 1440 us; back to back for a second the card lowers its clock: 1400 us against 1545, Row576
 // T = 1455 900 us against 1050.
 #include <type_traits>
@@ -159,16 +159,6 @@ __device__ inline float half_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   const uint32_t a = r[0], b = r[1];           // (a bit cast of an element would take element 0)
   return max3(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b), __builtin_bit_cast(float, b));
-}
-
-// LDS DMA of 16 bytes a lane with the instruction's offset OFF, which is added to the global and the LDS address
-template <int OFF>
-__device__ inline void dma16_off(uint64_t g, SPMLA_LDS void* l) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  const uint32_t a = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)l - OFF);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2" ::"v"(g), "s"(a), "n"(OFF) : "memory", "m0");
-#pragma clang diagnostic pop
 }
 
 // O *= a for the 64 AGPR accumulator values of a head block, one register at a time through one VGPR (a plain C++
@@ -354,7 +344,7 @@ __global__ void __launch_bounds__(256, 1) fwd_kernel(Params p) {
     return (x >= 0 ? a : zrow) + (uint32_t)(128 * w + 16 * (ln >> 5));
   };
   auto issue_code = [&](int sl, uint64_t row, auto i) {
-    dma16_off<32 * decltype(i)::value>(row, reg + sl + decltype(i)::value * 1024);
+    dma16_off<32 * decltype(i)::value, 1024 * decltype(i)::value>(row, reg + sl);
   };
   auto issue_rope = [&](int ln, int jj, int sl, uint64_t row) {
     if constexpr (R5) { if (ln < 32) dma16((const void*)(row + (uint64_t)(D_LAT - 112 * w)), reg + sl + 4096); }
@@ -849,13 +839,13 @@ long long ws_bytes(int T, int H, int S);
 extern "C" {
 
 // Whether a launch without the split merge takes fwd_kernel (128 heads per workgroup, one workgroup per compute unit)
-// or the head-group kernel (spmla_attn_hg.hip: 32 heads per workgroup, two per compute unit, any K). fwd_kernel pays for
-// whole groups of 128 heads and for whole rounds of 256 workgroups; a round costs as much as 3.1 times 256 head-group
-// workgroups at K = 2048, 2.5 times at K <= 512. Measured (us, head-group / fwd_kernel), Row656, K = 2048: H = 128:
-// T = 192 158 / 160, 224 218 / 165, 256 230 / 170, 320 256 / 303, 520 439 / 445, 900 726 / 606, 2048 1724 / 1328;
-// T = 2048: H = 32 427 / 1338, 64 844 / 1372, 96 1226 / 1405; T = 700, H = 72: 426 / 436. H = 128: T = 300, K = 512
-// 102 / 100, T = 400, K = 1024 205 / 174, T = 256, K = 64 49 / 27. Row576 lies the same way (H = 128, K = 2048: T = 192
-// 138 / 136, 224 169 / 138, 320 220 / 264, 520 376 / 398, 2048 1442 / 1152).
+// or the head-group kernel (spmla_attn_hg.hip: 32 heads per workgroup, one per compute unit as well, any K). fwd_kernel
+// pays for whole groups of 128 heads and for whole rounds of 256 workgroups; a round costs as much as 3.1 times 256
+// head-group workgroups at K = 2048, 2.5 times at K <= 512 (their prologue and merge weigh more). Measured (us, head-group
+// / fwd_kernel), Row656, K = 2048: H = 128: T = 192 169 / 163, 224 206 / 163, 256 198 / 169, 400 326 / 306, 640 475 / 459,
+// 900 688 / 616, 2048 1559 / 1304; T = 2048: H = 32 417 / 1140, 64 798 / 1186, 96 1199 / 1242; T = 512, H = 160 477 / 598;
+// T = 700, H = 72 406 / 435. H = 128: T = 300, K = 512 100 / 101, T = 400, K = 1024 199 / 172, T = 256, K = 64 45 / 26.
+// Row576 lies the same way (H = 128, K = 2048: T = 192 134 / 140, 224 166 / 146, 400 288 / 279, 2048 1386 / 1168).
 static bool attn_wide(int T, int H, int K, int S) {
   const int rows = ((K + S - 1) / S + attn::TR - 1) / attn::TR * attn::TR;     // of a split
   const long long n32 = (long long)T * S * ((H + 31) / 32), n128 = (long long)T * S * ((H + attn::HGW - 1) / attn::HGW);

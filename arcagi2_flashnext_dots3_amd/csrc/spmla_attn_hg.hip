@@ -8,9 +8,9 @@
 //     token masks, ballots). Reference: dotsnote/engine/arcstats_pkg/arcstats/csrc/offload_attn.cu:700-1153
 //     (pk_attn_kernel).
 //   * attn_kernel<false, *, true>, the decode kernel whose S splits of a token's rows merge in the kernel (small
-//     batches: K = 2048, 128 heads, 1 / 8 / 16 / 32 tokens 23.6 / 26.5 / 29.0 / 39.0 us in graphs, against 53 / 54 / 55
+//     batches: K = 2048, 128 heads, 1 / 8 / 16 / 32 tokens 22.7 / 25.9 / 27.6 / 36.1 us, against 53 / 54 / 55
 //     / 51 us for 128-head workgroups with f16 partials at up to 8 splits, or unsplit at 32 tokens). A launch that
-//     leaves compute units idle is bound by the serial chain of a wave (12.7 us of prologue and merge, 2.2 us per
+//     leaves compute units idle is bound by the serial chain of a wave (12.7 us of prologue and merge, 2.0 us per
 //     tile), so the rows go to more workgroups;
 //   * attn_kernel<false, true>, the same decode over Row576 rows (spmla_attn576: 512 + 64 e4m3 codes, one
 //     per-tensor kv_scale): no per-group scales, so the latent MFMAs run as one chain into S (no scale combine), P'
@@ -26,7 +26,13 @@
 // bf16 and one fp32 scale combine per 128-value group; PV on f16 MFMA with P' = P * scale in fp16 and the codes read
 // transposed with ds_read_b64_tr_b8; lazy rescaling (a column's reference max moves only when a tile exceeds it by
 // more than TAU, so p <= 2^TAU); a power-of-two factor 2^-eps carried by P, O and l keeps P' inside f16's range for
-// any row scale; the 4 waves' (m, l, O) merge through LDS at the end.
+// any row scale; the 4 waves' (m, l, O) merge through LDS at the end. One wave per SIMD: issue bounds the loop (about
+// 4.5 cycles per vector instruction, 8 per scalar one or s_nop 1). So S^T is written in slices, one MFMA and the conversion
+// of the next operand each, without wait states; a group's scale combine runs under the next group; the query rope is
+// read under group 0 and the next tile's first codes under the last PV MFMAs; a tile's copies share one address
+// register. 64 tokens, 128 heads, 2048 rows: 58.5 -> 53.4 us (Row576 51.9 -> 48.3).
+#include <type_traits>
+
 #include "spmla_common.h"
 #include <stdlib.h>
 
@@ -93,22 +99,32 @@ __device__ inline float half_swap(float x) {
 
 // QK MFMAs with the accumulator in VGPRs. The compiler builtin puts every MFMA result in AGPRs when the function
 // uses AGPRs, which here would evict part of the PV accumulator around each QK phase; inline asm pins the QK
-// accumulator (read by the scale FMAs) to VGPRs. Hazards the compiler cannot see inside asm are covered here:
-// "s_nop 1" before the MFMA for VALU-written operands (2 wait states), and after the last MFMA of a chain
-// 16 wait states before any VALU reads the result (8-pass XDL write -> VALU read). Back-to-back MFMAs of one
-// chain have srcC == vdst exactly, which the hardware forwards.
+// accumulator (read by the scale FMAs) to VGPRs; the statements are volatile so that they keep their order. Hazards the
+// compiler cannot see inside asm are kept off by that order, not by wait states (each would take an issue slot): an
+// operand is converted a slice before its MFMA (2 wait states after a VALU write), and a chain's result is read three or
+// more MFMAs, or 11 wait states, after its last one (chain_end). Back-to-back MFMAs of one chain have srcC == vdst exactly
+// (forwarded). tests/test_attention_hazards.py checks the compiled order.
 __device__ inline f32x16 qk_first(bf16x8 a, bf16x8 b) {
   f32x16 d;
-  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b));
   return d;
 }
 __device__ inline f32x16 qk_next(bf16x8 a, bf16x8 b, f32x16 c) {
-  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
   return c;
 }
-__device__ inline f32x16 qk_last(bf16x8 a, bf16x8 b, f32x16 c) {
-  asm("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_nop 7\n\ts_nop 7" : "+v"(c) : "v"(a), "v"(b));
-  return c;
+// after the last MFMA of a chain and N instructions that do not touch c: what is left of 11 wait states
+template <int N>
+__device__ inline void chain_end(f32x16& c) {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop %1" : "+v"(c) : "n"(N < 11 ? 10 - N : 0));
+}
+// the maximum of x over the two lanes l, l ^ 32
+__device__ inline float half_max(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const uint32_t a = r[0], b = r[1];           // (a bit cast of an element would take element 0)
+  return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
 }
 
 // O *= a for the 256 AGPR accumulator values of a lane, one register at a time through one VGPR. Written as
@@ -225,6 +241,9 @@ __device__ inline void merge_splits(const Params& p, int t, int hg, int w, int l
   }
 }
 
+template <int N>
+using ic = std::integral_constant<int, N>;
+
 // Source of invalid and padding rows: zero codes, zero scales, zero rope (their P is 0, and 0 * 0 stays 0 in PV).
 __device__ __attribute__((aligned(16))) uint8_t zero_row[ROW656];
 
@@ -316,20 +335,38 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
   // rope of this lane's row: Row656, dims 16 ks + 8 half .. + 7 of MFMA ks (bf16); Row576, the 32 e4m3 codes of
   // dims 32 half .. 32 half + 31, MFMA ks taking dims 32 half + 8 ks .. + 7 (the query rope is read to match)
   u32x4 rp[NRP];
-  auto load_rope = [&](const uint8_t* src) {
+  auto load_rope = [&](uint64_t src) {                 // (src: the lane's row + 16 half)
+    const uint8_t* b = (const uint8_t*)(uintptr_t)src + (R5 ? D_LAT + 16 * half : ROPE_OFF);
 #pragma unroll
-    for (int ks = 0; ks < NRP; ++ks)
-      rp[ks] = R5 ? *(const u32x4*)(src + D_LAT + 32 * half + 16 * ks)
-                  : *(const u32x4*)(src + ROPE_OFF + ks * 32 + half * 16);
+    for (int ks = 0; ks < NRP; ++ks) rp[ks] = *(const u32x4*)(b + (R5 ? 16 * ks : 32 * ks));
+  };
+  uint64_t zrow = (uint64_t)(uintptr_t)zero_row;
+  asm volatile("" : "+s"(zrow));                       // (its address would be formed again in every tile)
+  auto row_at = [&](int x) -> uint64_t {               // address of row x (-1: the zero row) + 16 half
+    return (x >= 0 ? (uint64_t)(uintptr_t)p.pool + (uint64_t)(uint32_t)x * RB : zrow) + 16u * half;
+  };
+  // the copies of chunks 8 g + 2 i + half, i = 0 .. 3, of a row, and of its scales
+  auto copy_part = [&](uint64_t src, SPMLA_LDS uint8_t* buf, auto g) {
+    constexpr int G4 = 4 * decltype(g)::value;
+    dma16_off<32 * G4, 1024 * G4>(src, buf);
+    dma16_off<32 * G4 + 32, 1024 * G4 + 1024>(src, buf);
+    dma16_off<32 * G4 + 64, 1024 * G4 + 2048>(src, buf);
+    dma16_off<32 * G4 + 96, 1024 * G4 + 3072>(src, buf);
+  };
+  auto copy_scales = [&](uint64_t src, SPMLA_LDS uint8_t* buf) {
+    if constexpr (!R5) {
+      const uint64_t sc = src + (uint64_t)(SC_OFF - 12 * half);
+      dma4_off<0, 0>(sc, buf + T_SCT);
+      dma4_off<8, 256>(sc, buf + T_SCT);
+    }
   };
   if (ntw > 0) {
-    const uint8_t* src = rcur >= 0 ? p.pool + (long long)rcur * RB : zero_row;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dma16(src + (2 * i + half) * 16, mybuf + i * 1024);
-    if constexpr (!R5) {
-      dma4(src + SC_OFF + half * 4, mybuf + T_SCT);
-      dma4(src + SC_OFF + (2 + half) * 4, mybuf + T_SCT + 256);
-    }
+    const uint64_t src = row_at(rcur);
+    copy_part(src, mybuf, ic<0>());
+    copy_part(src, mybuf, ic<1>());
+    copy_part(src, mybuf, ic<2>());
+    copy_part(src, mybuf, ic<3>());
+    copy_scales(src, mybuf);
     load_rope(src);
   }
   // latent query fragments of groups 0, 1 (bf16 B operands), k-pair kp (32 dims = chunks 2kp, 2kp + 1): lane half
@@ -365,19 +402,18 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
   const int G = lane >> 4, gi = (lane & 15) >> 1, gc = lane & 1;
   const int tr_off = ((G & 1) * 32 + 8 * (gi >> 2) + 4 * (G >> 1) + (gi & 3)) * 16 + gc * 8;
 
+  // K codes of latent group 0 of the tile in buf; the next tile's are read during this one's last PV MFMAs
+  u32x4 kr[4];
+  auto kr_read = [&](SPMLA_LDS uint8_t* buf) {
+#pragma unroll
+    for (int kq = 0; kq < 4; ++kq) kr[kq] = *(SPMLA_LDS u32x4*)(buf + (2 * kq + half) * 512 + l32 * 16);
+  };
+  kr_read(mybuf);                               // (no tile: unused bytes)
+
 #pragma unroll 1
-  for (int j = 0; j < ntw; ++j) {
-    wait_vm<0>();                               // tile j copied, its rope loaded
+  for (int j = 0; j < ntw; ++j) {               // tile j copied, its rope loaded
     SPMLA_LDS uint8_t* tb = mybuf + (j & 1) * TILE;
     const int tix = w + NW * j;
-
-    // ---- first LDS reads of the tile: query rope, K group 0, the row ids of this and of the next tile
-    u32x4 qr[4], kr[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      qr[ks] = *(SPMLA_LDS u32x4*)(qrope + l32 * QRS + (R5 ? 32 * half + 8 * ks : 16 * ks + 8 * half) * 2);
-#pragma unroll
-    for (int kq = 0; kq < 4; ++kq) kr[kq] = *(SPMLA_LDS u32x4*)(tb + (2 * kq + half) * 512 + l32 * 16);
     const bool more = j + 1 < ntw;
     // the entries loaded one iteration ago are checked only now, after the wait above: checking them where they
     // are loaded would stall every tile on a global-memory round trip
@@ -386,85 +422,88 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
     if (PK) mnn = j + 2 < ntw ? mk_raw(tix + 2 * NW) : 0u;
     __builtin_amdgcn_sched_barrier(0);
 
-    // ---- rope part of S^T (operands in VGPRs / LDS)
+    // ---- S^T, one slice per MFMA, each followed by a fence: the operand of the next MFMA is converted before this one
+    // is issued, so conversions run under the matrix core and no operand is a fresh VALU result.
+    auto conv = [&](uint32_t w0, uint32_t w1) -> bf16x8 {         // 8 e4m3 codes -> bf16 (exact)
+      return __builtin_bit_cast(bf16x8, u32x4{fp8lo_bf16x2(w0), fp8hi_bf16x2(w0), fp8lo_bf16x2(w1), fp8hi_bf16x2(w1)});
+    };
+    bf16x8 ko[2];                                      // K operands: this and the next MFMA's
+    auto k_conv = [&](const u32x4 (&r)[4], int n) {
+      ko[n & 1] = (n & 1) ? conv(r[n >> 1][2], r[n >> 1][3]) : conv(r[n >> 1][0], r[n >> 1][1]);
+      asm volatile("" : "+v"(ko[n & 1]));              // (the compiler would sink it into the next block)
+    };
+    k_conv(kr, 0);
     f32x16 S;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      bf16x8 a;
-      if constexpr (R5) {                          // 8 e4m3 rope codes -> bf16 (exact)
-        const uint32_t w0 = rp[ks >> 1][2 * (ks & 1)], w1 = rp[ks >> 1][2 * (ks & 1) + 1];
-        i32x4 x;
-        x[0] = (int)fp8lo_bf16x2(w0); x[1] = (int)fp8hi_bf16x2(w0);
-        x[2] = (int)fp8lo_bf16x2(w1); x[3] = (int)fp8hi_bf16x2(w1);
-        a = __builtin_bit_cast(bf16x8, x);
-      } else {
-        a = __builtin_bit_cast(bf16x8, rp[ks]);
-      }
-      const bf16x8 b = __builtin_bit_cast(bf16x8, qr[ks]);
-      // Row576: the chain goes on through the latent groups (no scales to combine)
-      S = ks == 0 ? qk_first(a, b) : ((ks == 3 && !R5) ? qk_last(a, b, S) : qk_next(a, b, S));
-    }
     const unsigned vmask = (unsigned)__ballot(rcur >= 0);  // rows of the tile that exist
     // the next tile's copy is issued in four parts, one per latent group, between that group's MFMAs
-    const uint8_t* nsrc = rnxt >= 0 ? p.pool + (long long)rnxt * RB : zero_row;
+    const uint64_t nsrc = row_at(rnxt);
     SPMLA_LDS uint8_t* nbuf = mybuf + ((j + 1) & 1) * TILE;
 
-    // ---- latent part of S^T: group g = chunks 8g .. 8g + 7; group g + 1's K is read while group g's MFMAs run
+    // ---- latent part of S^T: group g = chunks 8g .. 8g + 7; group g + 1's K is read while group g's MFMAs run, and its
+    // partial is combined with the rows' scales after the third MFMA of group g + 1 (Row576: one chain into S)
+    f32x16 acc[2];
+    f32x4 sg[4];
+    auto sg_read = [&](int g) {
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) sg[qd] = *(SPMLA_LDS f32x4*)(tb + T_SCT + (g * 32 + 8 * qd + 4 * half) * 4);
+    };
+    auto combine = [&](const f32x16& x) {
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[4 * qd + e] = __builtin_fmaf(x[4 * qd + e], sg[qd][e], S[4 * qd + e]);
+    };
+    auto q_read = [&](int n) -> bf16x8 {               // query operand n of groups 2, 3: dims 16 (n & ~1) + 16 half + 8 (n & 1)
+      const SPMLA_LDS uint8_t* qp = qrope + l32 * QRS + 128 + ((n & ~1) * 16 + 16 * half - 2 * QGROUP) * 2 + 16 * (n & 1);
+      return __builtin_bit_cast(bf16x8, *(const SPMLA_LDS u32x4*)qp);
+    };
+    bf16x8 qb[4];                                      // those in flight, read three MFMAs ahead
+    u32x4 qr[4];                                       // query rope
+    bf16x8 ro[2];                                      // Row576: rope operands
+    auto ro_conv = [&](int ks) {
+      ro[ks & 1] = conv(rp[ks >> 1][2 * (ks & 1)], rp[ks >> 1][2 * (ks & 1) + 1]);
+      asm volatile("" : "+v"(ro[ks & 1]));
+    };
+    auto rope = [&]() {                                // rope part of S^T, after latent group 0
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        if (R5 && ks < 3) ro_conv(ks + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const bf16x8 b = __builtin_bit_cast(bf16x8, qr[ks]);
+        if constexpr (R5) S = qk_next(ro[ks & 1], b, S);
+        else S = ks == 0 ? qk_first(__builtin_bit_cast(bf16x8, rp[0]), b) : qk_next(__builtin_bit_cast(bf16x8, rp[ks]), b, S);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       u32x4 kn[4];
-      if (g < 3) {
-#pragma unroll
-        for (int kq = 0; kq < 4; ++kq) kn[kq] = *(SPMLA_LDS u32x4*)(tb + (2 * (4 * g + 4 + kq) + half) * 512 + l32 * 16);
+      if (more) {                                      // part g of the next tile's copy
+        if (g == 0) copy_part(nsrc, nbuf, ic<0>());
+        if (g == 1) copy_part(nsrc, nbuf, ic<1>());
+        if (g == 2) copy_part(nsrc, nbuf, ic<2>());
+        if (g == 3) { copy_part(nsrc, nbuf, ic<3>()); copy_scales(nsrc, nbuf); load_rope(nsrc); }
       }
-      if (more) {                                  // part g of the next tile's copy
 #pragma unroll
-        for (int i = 4 * g; i < 4 * g + 4; ++i) dma16(nsrc + (2 * i + half) * 16, nbuf + i * 1024);
-        if (g == 3) {
-          if constexpr (!R5) {
-            dma4(nsrc + SC_OFF + half * 4, nbuf + T_SCT);
-            dma4(nsrc + SC_OFF + (2 + half) * 4, nbuf + T_SCT + 256);
-          }
-          load_rope(nsrc);
-        }
+      for (int n = 0; n < 8; ++n) {
+        const int q = 8 * g + n;
+        constexpr int KQ[8] = {-1, -1, -1, 0, 1, -1, 2, 3};        // chunk pair of the next group read at MFMA n
+        if (g < 3 && KQ[n] >= 0) kn[KQ[n]] = *(SPMLA_LDS u32x4*)(tb + (2 * (4 * g + 4 + KQ[n]) + half) * 512 + l32 * 16);
+        if (q + 3 >= 16 && q + 3 < 32) qb[(q + 3) & 3] = q_read(q + 3);
+        if (!R5 && ((g > 0 && n == 1) || (g == 3 && n == 5))) sg_read(n == 1 ? g - 1 : 3);
+        if (!R5 && g > 0 && n == 3) combine(acc[(g - 1) & 1]);
+        if (g == 0 && n >= 2 && n < 6)
+          qr[n - 2] = *(SPMLA_LDS u32x4*)(qrope + l32 * QRS + (R5 ? 32 * half + 8 * (n - 2) : 16 * (n - 2) + 8 * half) * 2);
+        if (R5 && g == 0 && n == 7) ro_conv(0);
+        if (n < 7) k_conv(kr, n + 1);
+        else if (g < 3) k_conv(kn, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        const bf16x8 b = g < 2 ? qf[q] : qb[q & 3];
+        if constexpr (R5) S = q == 0 ? qk_first(ko[0], b) : qk_next(ko[n & 1], b, S);
+        else acc[g & 1] = n == 0 ? qk_first(ko[0], b) : qk_next(ko[n & 1], b, acc[g & 1]);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
-      f32x16 acc;
-#pragma unroll
-      for (int kq = 0; kq < 4; ++kq) {
-        const int kp = 4 * g + kq;
-        const u32x4 raw = kr[kq];
-        i32x4 a0, a1;
-        a0[0] = (int)fp8lo_bf16x2(raw[0]); a0[1] = (int)fp8hi_bf16x2(raw[0]);
-        a0[2] = (int)fp8lo_bf16x2(raw[1]); a0[3] = (int)fp8hi_bf16x2(raw[1]);
-        a1[0] = (int)fp8lo_bf16x2(raw[2]); a1[1] = (int)fp8hi_bf16x2(raw[2]);
-        a1[2] = (int)fp8lo_bf16x2(raw[3]); a1[3] = (int)fp8hi_bf16x2(raw[3]);
-        bf16x8 b0, b1;
-        if (g < 2) {
-          b0 = qf[2 * kp];
-          b1 = qf[2 * kp + 1];
-        } else {                                   // dims 16 (2kp + half) + 8e of latent groups 2, 3, from LDS
-          const SPMLA_LDS uint8_t* qp = qrope + l32 * QRS + 128 + ((2 * kp + half) * 16 - 2 * QGROUP) * 2;
-          b0 = __builtin_bit_cast(bf16x8, *(const SPMLA_LDS u32x4*)qp);
-          b1 = __builtin_bit_cast(bf16x8, *(const SPMLA_LDS u32x4*)(qp + 16));
-        }
-        if constexpr (R5) {
-          S = qk_next(__builtin_bit_cast(bf16x8, a0), b0, S);
-          S = (g == 3 && kq == 3) ? qk_last(__builtin_bit_cast(bf16x8, a1), b1, S)
-                                  : qk_next(__builtin_bit_cast(bf16x8, a1), b1, S);
-        } else {
-          acc = kq == 0 ? qk_first(__builtin_bit_cast(bf16x8, a0), b0) : qk_next(__builtin_bit_cast(bf16x8, a0), b0, acc);
-          acc = kq == 3 ? qk_last(__builtin_bit_cast(bf16x8, a1), b1, acc) : qk_next(__builtin_bit_cast(bf16x8, a1), b1, acc);
-        }
-      }
-      if constexpr (!R5) {
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-          const f32x4 sg = *(SPMLA_LDS f32x4*)(tb + T_SCT + (g * 32 + 8 * qd + 4 * half) * 4);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) S[4 * qd + e] = __builtin_fmaf(acc[4 * qd + e], sg[e], S[4 * qd + e]);
-        }
-      }
+      if (g == 0) rope();
       if (g < 3) {
 #pragma unroll
         for (int q4 = 0; q4 < 4; ++q4) kr[q4] = kn[q4];
@@ -484,7 +523,11 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
 #pragma unroll
     for (int f8 = 0; f8 < 8; ++f8)
       tv[f8] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((SPMLA_LDS i32x2*)(tb + (f8 >> 1) * 1024 + (f8 & 1) * 256 + tr_off));
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (R5) chain_end<8>(S);
+    else {
+      chain_end<9>(acc[1]);
+      combine(acc[1]);
+    }
 
     // ---- rows that do not exist: -inf (C-layout row of value i: 8 (i / 4) + 4 half + i % 4)
     unsigned rm = vmask;                                 // rows of the tile this lane's column may use
@@ -508,7 +551,7 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
     float mx = S[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, S[i]);
-    mx = fmaxf(mx, half_swap(mx)) * c;                      // c > 0; -inf stays -inf
+    mx = half_max(mx) * c;                                  // c > 0; -inf stays -inf
     const bool need = mx > m_run + TAU;                      // also true for the first finite tile
     if (__ballot(need)) {
       const float mn = need ? mx : m_run;
@@ -587,6 +630,10 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
         for (int f8 = 0; f8 < 8; ++f8)
           vn[f8] = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
               (SPMLA_LDS i32x2*)(tb + (4 * (g + 1) + (f8 >> 1)) * 1024 + (f8 & 1) * 256 + tr_off));
+      }
+      if (g == 3) {
+        wait_vm<0>();                           // the next tile copied, its rope loaded
+        kr_read(nbuf);
       }
       __builtin_amdgcn_sched_barrier(0);
       f16x8 pbn[2];

@@ -135,6 +135,20 @@ __device__ inline void dma4(const void* g, SPMLA_LDS void* l) {
   const uint32_t a = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)l);
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(a) : "memory", "m0");
 }
+// The same with the instruction's offset OFF, which is added to the global and the LDS address, and an LDS place LD bytes
+// from l (m0 in one scalar instruction): several copies from one address register.
+template <int OFF, int LD>
+__device__ inline void dma16_off(uint64_t g, SPMLA_LDS void* l) {
+  const uint32_t a = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)l);
+  asm volatile("s_add_u32 m0, %1, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off offset:%2"
+               ::"v"(g), "s"(a), "n"(OFF), "n"(LD - OFF) : "memory", "m0", "scc");
+}
+template <int OFF, int LD>
+__device__ inline void dma4_off(uint64_t g, SPMLA_LDS void* l) {
+  const uint32_t a = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)l);
+  asm volatile("s_add_u32 m0, %1, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, off offset:%2"
+               ::"v"(g), "s"(a), "n"(OFF), "n"(LD - OFF) : "memory", "m0", "scc");
+}
 #pragma clang diagnostic pop
 
 // Workgroup barrier for data exchanged through LDS only (no vector-memory drain).

@@ -1,7 +1,7 @@
-"""The attention kernel's inline-asm MFMA and DPP statements rely on the order of the compiled code instead of wait
-states, which the compiler does not add for asm: in the assembly of fwd_kernel no MFMA operand and no DPP source is
+"""The attention kernels' inline-asm MFMA and DPP statements rely on the order of the compiled code instead of wait
+states, which the compiler does not add for asm: in their assembly no MFMA operand and no DPP source is
 written by the VALU in the two instructions before, and no VGPR result of an MFMA is read or overwritten before three
-more MFMAs were issued."""
+more MFMAs were issued or 11 wait states passed."""
 import os
 import re
 import subprocess
@@ -23,7 +23,7 @@ def _regs(tok):
 
 def hazards(lines):
     """[(line, text)] of the violations in one kernel's assembly."""
-    bad, hist, mfma = [], [], []
+    bad, hist, mfma, now = [], [], [], 0          # mfma: (destination, wait states issued before it)
     for n, l in enumerate(lines):
         l = l.split(";")[0].strip()
         if not l or l.startswith(".") or l.endswith(":"):
@@ -41,11 +41,12 @@ def hazards(lines):
                 bad.append((n, l))
             states += 1
         if "mfma" in op:
-            mfma.append(dst)
+            mfma.append((dst, now))
         else:
             touched = {r for r in src | (dst if op.startswith("v_") else set()) if r[0] == "v"}
-            if any(touched & d for d in mfma[-3:]):
+            if any(touched & d and now - at - 1 < 11 for d, at in mfma[-3:]):
                 bad.append((n, l))
+        now += 1 + (int(toks[0], 0) if op == "s_nop" else 0)
         hist.append((op, set() if stores else dst, toks[0]))
     return bad
 
@@ -58,17 +59,20 @@ def test_scanner_finds_planted_hazards():
     assert hazards(["v_mov_b32_e32 v5, v9", "s_nop 0", m])
     a = "v_mfma_f32_32x32x16_f16 a[0:15], v[40:43], v[44:47], a[0:15]"
     assert hazards([m, a, a, "ds_write_b128 v9, v[16:19] offset:64"])
+    assert hazards([m, "s_nop 9", "v_add_f32_e32 v1, v16, v2"]) and not hazards([m, "s_nop 10", "v_add_f32_e32 v1, v16, v2"])
     assert not hazards([m, a, a, a, "ds_write_b128 v9, v[16:19] offset:64"])
 
 
 @pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no hipcc")
-def test_compiled_order_of_asm_statements(tmp_path):
+@pytest.mark.parametrize("src,kernel,count", [("spmla_attn.hip", r"_ZN5spmla4attn10fwd_kernelI\S+:", 2),
+                                              ("spmla_attn_hg.hip", r"_ZN5spmla2pk11attn_kernelI\S+:", 5)])
+def test_compiled_order_of_asm_statements(tmp_path, src, kernel, count):
     out = tmp_path / "attn.s"
-    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, "spmla_attn.hip"),
-                    "-o", str(out)], check=True, capture_output=True)
+    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, src), "-o", str(out)],
+                   check=True, capture_output=True)
     text = out.read_text().split("\n")
-    starts = [i for i, l in enumerate(text) if re.match(r"_ZN5spmla4attn10fwd_kernelILb[01]EEE\S*:", l)]
-    assert len(starts) == 2
+    starts = [i for i, l in enumerate(text) if re.match(kernel, l)]
+    assert len(starts) == count
     for s in starts:
         end = next(i for i in range(s, len(text)) if ".Lfunc_end" in text[i])
         body = text[s:end]
