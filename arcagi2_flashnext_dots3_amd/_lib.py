@@ -52,6 +52,7 @@ SIGNATURES = {
     "spmla_attn576": [P, LL, LL, P, LL, P, LL, I, P, I, I, F, F, I, P, LL, LL, P, LL, P, P, P],
     "spmla_attn": [P, LL, LL, P, LL, P, LL, I, P, I, I, F, F, I, P, LL, LL, P, LL, P, LL, P],
     "spmla_attn576_ws": [P, LL, LL, P, LL, P, LL, I, P, I, I, F, F, I, P, LL, LL, P, LL, P, LL, P],
+    "spmla_attn_paged": [P, LL, LL, P, LL, P, LL, I, P, P, LL, I, I, LL, I, I, F, F, I, I, P, LL, LL, P, LL, P, LL, P],
     "spmla_attn_ws_bytes": [I, I, I],
     "spmla_attn_merge": [P, LL, LL, P, LL, P, LL, I, P, I, I, F, F, P, LL, LL, P, LL, P, LL, LL, P, LL, P],
     "spmla_lse_merge": [P, I, LL, LL, LL, P, LL, LL, I, I, I, P, LL, LL, P, P, LL, P],

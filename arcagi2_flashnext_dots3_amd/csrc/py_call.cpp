@@ -69,7 +69,7 @@ struct Entry<R (*)(A...)> {
   X(spmla_row400_copy) X(spmla_row400_gather_tiers) X(spmla_row400_decode_tiers) X(spmla_tier_split)                \
   X(spmla_wcache_step) X(spmla_wcache_place) X(spmla_wcache_resolve) X(spmla_wcache_fill)                           \
   X(spmla_wcache_invalidate) X(spmla_split_res) X(spmla_wcache_split) X(spmla_compact_stage) X(spmla_attn_splitk)   \
-  X(spmla_attn576) X(spmla_attn) X(spmla_attn576_ws) X(spmla_attn_ws_bytes) X(spmla_attn_merge) X(spmla_lse_merge)  \
+  X(spmla_attn576) X(spmla_attn) X(spmla_attn576_ws) X(spmla_attn_paged) X(spmla_attn_ws_bytes) X(spmla_attn_merge) X(spmla_lse_merge)  \
   X(spmla_bmm_fp8) X(spmla_mla_query) X(spmla_topk_overlap) X(spmla_mtp_union) X(spmla_attn_packed)                 \
   X(spmla_index_key_write_shuffle) X(spmla_mqa_logits) X(spmla_paged_mqa_logits) X(spmla_paged_mqa_logits_seq)
 

@@ -192,6 +192,7 @@ struct Params {
   // optional prior partial merged into the bf16 output (S == 1): normalized fp32 o and natural-log lse
   const float* prior_o; long long po_st, po_sh;
   const float* prior_lse; long long pl_st;
+  Pages pg;                                       // idx holds positions (pg.bt) or rows
 };
 
 // Row scales as DPP operands. z[a] of lane l = scale g of row 8 a + 4 hh + l % 4; value i = 4 a + b of a C-layout
@@ -284,8 +285,18 @@ __global__ void __launch_bounds__(256, 1) fwd_kernel(Params p) {
     const int i = tid + 256 * k;
     int x = -1;
     if (i < nrow) x = idxrow[i];
-    xs[k] = (x >= 0 && (long long)x < p.R) ? x : -1;
+    xs[k] = x;
   }
+  if (p.pg.bt) {
+    const int* btrow = p.pg.bt + (long long)p.pg.req[t] * p.pg.bt_st;
+    int b[KMAX / 256];
+#pragma unroll
+    for (int k = 0; k < KMAX / 256; ++k) b[k] = page_entry(p.pg, btrow, xs[k]);
+#pragma unroll
+    for (int k = 0; k < KMAX / 256; ++k) xs[k] = page_row(p.pg, xs[k], b[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < KMAX / 256; ++k) xs[k] = xs[k] >= 0 && (long long)xs[k] < p.R ? xs[k] : -1;
   bf16x8 qf[4 * NK];                                         // operand r NK + ks; NQL of them move to LDS below
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -831,7 +842,7 @@ int launch_tokens(const void* q, long long q_st, long long q_sh, const void* poo
                   long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                   void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
                   float* lsepart, const float* prior_o, long long po_st, long long po_sh, const float* prior_lse,
-                  long long pl_st, void* ws, void* stream, bool r576);
+                  long long pl_st, void* ws, void* stream, bool r576, const Pages& pg);
 long long ws_bytes(int T, int H, int S);
 }  // namespace pk
 }  // namespace spmla
@@ -856,8 +867,10 @@ static attn::Params wide_params(const void* q, long long q_st, long long q_sh, c
                                 const int* idx, long long idx_st, int K, const int* kcount, int T, int H,
                                 float sm_scale, float kv_scale, int S, void* out, long long o_st, long long o_sh,
                                 float* lse, long long lse_st, float* opart, float* lsepart, const float* prior_o,
-                                long long po_st, long long po_sh, const float* prior_lse, long long pl_st) {
+                                long long po_st, long long po_sh, const float* prior_lse, long long pl_st,
+                                const Pages& pg) {
   attn::Params p;
+  p.pg = pg;
   p.q = (const uint16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.pool = (const uint8_t*)pool; p.R = R;
   p.idx = idx; p.idx_st = idx_st; p.K = K; p.kcount = kcount;
@@ -887,7 +900,7 @@ static int attn_launch(const void* q, long long q_st, long long q_sh, const void
                        long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                        void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
                        float* lsepart, const float* prior_o, long long po_st, long long po_sh, const float* prior_lse,
-                       long long pl_st, void* ws, long long ws_bytes, void* stream) {
+                       long long pl_st, void* ws, long long ws_bytes, void* stream, const Pages& pg = Pages{}) {
   if (T < 0 || H <= 0 || K < 0 || S <= 0 || R < 0) return SPMLA_EARG;
   if (T == 0) return SPMLA_OK;
   if (!q || !idx || (R > 0 && !pool)) return SPMLA_EARG;
@@ -907,9 +920,9 @@ static int attn_launch(const void* q, long long q_st, long long q_sh, const void
   if (fused || !attn_wide(T, H, K, S))
     return pk::launch_tokens(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st,
                              o_sh, lse, lse_st, opart, lsepart, prior_o, po_st, po_sh, prior_lse, pl_st,
-                             fused ? ws : nullptr, stream, false);
+                             fused ? ws : nullptr, stream, false, pg);
   return wide_launch(wide_params(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st,
-                                 o_sh, lse, lse_st, opart, lsepart, prior_o, po_st, po_sh, prior_lse, pl_st), false,
+                                 o_sh, lse, lse_st, opart, lsepart, prior_o, po_st, po_sh, prior_lse, pl_st, pg), false,
                      stream);
 }
 
@@ -938,7 +951,7 @@ int spmla_attn(const void* q, long long q_st, long long q_sh, const void* pool, 
 static int attn576_launch(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
                   long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                   void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
-                  float* lsepart, void* ws, long long ws_bytes, void* stream) {
+                  float* lsepart, void* ws, long long ws_bytes, void* stream, const Pages& pg = Pages{}) {
   if (T < 0 || H <= 0 || K < 0 || S <= 0 || R < 0) return SPMLA_EARG;
   if (T == 0) return SPMLA_OK;
   if (!q || !idx || (R > 0 && !pool)) return SPMLA_EARG;
@@ -955,10 +968,10 @@ static int attn576_launch(const void* q, long long q_st, long long q_sh, const v
   if (f32part && ((uintptr_t)opart & 15)) return SPMLA_EALIGN;
   if (!fused && attn_wide(T, H, K, S))
     return wide_launch(wide_params(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out,
-                                   o_st, o_sh, lse, lse_st, opart, lsepart, nullptr, 0, 0, nullptr, 0), true, stream);
+                                   o_st, o_sh, lse, lse_st, opart, lsepart, nullptr, 0, 0, nullptr, 0, pg), true, stream);
   return pk::launch_tokens(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st,
                            o_sh, lse, lse_st, opart, lsepart, nullptr, 0, 0, nullptr, 0, fused ? ws : nullptr, stream,
-                           true);
+                           true, pg);
 }
 
 int spmla_attn576(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
@@ -975,6 +988,23 @@ int spmla_attn576_ws(const void* q, long long q_st, long long q_sh, const void* 
                      long long ws_bytes, void* stream) {
   return attn576_launch(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st, o_sh,
                         lse, lse_st, nullptr, nullptr, ws, ws_bytes, stream);
+}
+
+int spmla_attn_paged(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* topk,
+                     long long tk_st, int K, const int* req, const int* block_table, long long bt_st, int bt_cols,
+                     int block_size, long long stride_rows, int T, int H, float sm_scale, float kv_scale, int row_bytes,
+                     int S, void* out, long long o_st, long long o_sh, float* lse, long long lse_st, void* ws,
+                     long long ws_bytes, void* stream) {
+  if (row_bytes != ROW656 && row_bytes != ROW576) return SPMLA_EARG;
+  if (block_size <= 0 || bt_cols <= 0) return SPMLA_EARG;
+  if (block_size & (block_size - 1)) return SPMLA_ELIMIT;
+  if (T > 0 && (!req || !block_table)) return SPMLA_EARG;
+  const Pages pg{req, block_table, bt_st, bt_cols, __builtin_ctz((unsigned)block_size), stride_rows};
+  if (row_bytes == ROW576)
+    return attn576_launch(q, q_st, q_sh, pool, R, topk, tk_st, K, nullptr, T, H, sm_scale, kv_scale, S, out, o_st, o_sh,
+                          lse, lse_st, nullptr, nullptr, S > 1 ? ws : nullptr, ws_bytes, stream, pg);
+  return attn_launch(q, q_st, q_sh, pool, R, topk, tk_st, K, nullptr, T, H, sm_scale, kv_scale, S, out, o_st, o_sh, lse,
+                     lse_st, nullptr, nullptr, nullptr, 0, 0, nullptr, 0, S > 1 ? ws : nullptr, ws_bytes, stream, pg);
 }
 
 int spmla_attn_merge(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,

@@ -165,6 +165,7 @@ struct Params {
   // a token to a word, zero between launches), and per split the lse [32 heads] and the normalized fp32 partial in
   // the lanes' order [16 output blocks][4][64 lanes][4]
   uint32_t* ws_cnt; float* ws_lse; float* ws_o;
+  Pages pg;                                       // attn_kernel<false>: idx holds positions (pg.bt) or rows
 };
 
 // Workspace of the split merge (bytes): counters (4 per token and 128 heads), lse, partials. Each part 256-byte aligned.
@@ -310,8 +311,14 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
     return x;
   };
   auto row_ok = [&](int x) -> int { return (x >= 0 && (long long)x < p.R) ? x : -1; };   // -1: none / invalid
-  int rcur = row_ok(row_raw(w)), rnxt = row_ok(row_raw(w + NW));
-  int rnn = -1;                        // raw entry two tiles ahead: loaded in one iteration, checked in the next
+  // Rows of the first two tiles, entries of later ones: loaded in one iteration, used in the next. With pages the entry is
+  // a position whose table entry is loaded an iteration after it (x2: three tiles ahead, xn / bn: two), so no tile
+  // waits for a round trip; before the first tile the two loads overlap the query's.
+  const int* btrow = nullptr;
+  if (!PK && p.pg.bt) btrow = p.pg.bt + (long long)p.pg.req[t] * p.pg.bt_st;
+  auto table = [&](int x) -> int { return !PK && p.pg.bt ? page_entry(p.pg, btrow, x) : 0; };
+  auto row_of = [&](int x, int b) -> int { return row_ok(!PK && p.pg.bt ? page_row(p.pg, x, b) : x); };
+  int xn = row_raw(w), x1 = row_raw(w + NW), x2 = PK ? -1 : row_raw(w + 2 * NW), bn = 0, b1 = 0;
   uint32_t mcur = mk_raw(w), mnxt = mk_raw(w + NW), mnn = 0u;
   {
     u32x4 qv[HG * QPIECES / 256];
@@ -323,6 +330,8 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
       const uint16_t* src = part < 8 ? qsrc + D_LAT + part * 8 : qsrc + 2 * QGROUP + (part - 8) * 8;
       qv[k] = *(const u32x4*)src & (ok ? 0xffffffffu : 0u);
     }
+    bn = table(xn);
+    b1 = table(x1);
     wait_vm<0>();
 #pragma unroll
     for (int k = 0; k < HG * QPIECES / 256; ++k) {
@@ -330,6 +339,7 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
       *(SPMLA_LDS u32x4*)(qrope + (i / QPIECES) * QRS + (i % QPIECES) * 16) = qv[k];
     }
   }
+  int rcur = row_of(xn, bn), rnxt = row_of(x1, b1);
   const int ntw = ntile > w ? (ntile - w + NW - 1) / NW : 0;   // tiles w, w + 4, ...
   SPMLA_LDS uint8_t* mybuf = lds + L_TILES + w * NBUF * TILE;
   // rope of this lane's row: Row656, dims 16 ks + 8 half .. + 7 of MFMA ks (bf16); Row576, the 32 e4m3 codes of
@@ -417,8 +427,13 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
     const bool more = j + 1 < ntw;
     // the entries loaded one iteration ago are checked only now, after the wait above: checking them where they
     // are loaded would stall every tile on a global-memory round trip
-    if (j > 0) { rnxt = row_ok(rnn); mnxt = mnn; }
-    rnn = j + 2 < ntw ? row_raw(tix + 2 * NW) : -1;
+    if (j > 0) { rnxt = row_of(xn, bn); mnxt = mnn; }
+    if constexpr (PK) xn = j + 2 < ntw ? row_raw(tix + 2 * NW) : -1;
+    else {
+      xn = x2;
+      if (j + 2 < ntw) bn = table(xn);
+      x2 = j + 3 < ntw ? row_raw(tix + 3 * NW) : -1;
+    }
     if (PK) mnn = j + 2 < ntw ? mk_raw(tix + 2 * NW) : 0u;
     __builtin_amdgcn_sched_barrier(0);
 
@@ -799,8 +814,9 @@ int launch_tokens(const void* q, long long q_st, long long q_sh, const void* poo
                   long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                   void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,
                   float* lsepart, const float* prior_o, long long po_st, long long po_sh, const float* prior_lse,
-                  long long pl_st, void* ws, void* stream, bool r576) {
+                  long long pl_st, void* ws, void* stream, bool r576, const Pages& pg) {
   Params p;
+  p.pg = pg;
   p.q = (const uint16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.pool = (const uint8_t*)pool; p.R = R;
   p.idx = idx; p.idx_st = idx_st; p.K = K; p.kcount = kcount;
@@ -851,7 +867,7 @@ int spmla_attn_packed(const void* q, long long q_st, long long q_sh, const void*
   if (f32part ? !lsepart : (S != 1 || !out || !lse)) return SPMLA_EARG;
   if (((uintptr_t)q & 15) || (q_st & 7) || (q_sh & 7) || ((uintptr_t)pool & 15)) return SPMLA_EALIGN;
   if (out && (((uintptr_t)out & 7) || (o_st & 3) || (o_sh & 3))) return SPMLA_EALIGN;
-  pk::Params p;
+  pk::Params p{};
   p.q = (const uint16_t*)q; p.q_st = q_st; p.q_sh = q_sh;
   p.pool = (const uint8_t*)pool; p.R = R;
   p.idx = u; p.idx_st = nmax; p.K = nmax; p.kcount = cnt;

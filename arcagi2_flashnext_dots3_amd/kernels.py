@@ -766,6 +766,33 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
     return out, lse
 
 
+def attend_paged(q, pool, topk_pos, req, block_table, block_size, stride_rows, sm_scale, kv_scale=1.0, R=None,
+                 row_bytes=ROW656):
+    """attend over rows_from_topk(topk_pos, req, block_table, block_size, stride_rows) with the rows formed in the
+    attention kernel (spmla_attn_paged) -> out [T, H, 512] bf16, or None when that kernel does not take the call (the
+    caller then forms the rows): block_size not a power of two, no table columns, more than 65535 tokens, tensors that
+    are not int32 with contiguous columns."""
+    T, H, _ = q.shape
+    K = topk_pos.shape[1]
+    if (block_size <= 0 or block_size & (block_size - 1) or block_table.shape[1] == 0 or not 0 < T <= 65535 or K == 0
+            or not (topk_pos.dtype == req.dtype == block_table.dtype == torch.int32)
+            or topk_pos.stride(1) != 1 or block_table.stride(1) != 1 or not req.is_contiguous() or not query_ok(q)):
+        return None
+    split = auto_split576(T, H, K) if row_bytes == ROW576 else auto_split(T, H, K)
+    out = torch.empty(T, H, D_LAT, dtype=torch.bfloat16, device=q.device)
+    lse = torch.empty(T, H, dtype=torch.float32, device=q.device)
+    wp, wn = None, 0
+    if split > 1:
+        ws = _attn_workspace(q.device, T, H, split, private=row_bytes == ROW576 or T * ((H + 31) // 32) >= 96)
+        wp, wn = ws.data_ptr(), ws.numel()
+    q_st, q_sh, _ = q.stride()
+    _lib.call("spmla_attn_paged", q.data_ptr(), q_st, q_sh, pool.data_ptr(), int(R if R is not None else pool.shape[0]),
+              topk_pos.data_ptr(), topk_pos.stride(0), K, req.data_ptr(), block_table.data_ptr(), block_table.stride(0),
+              block_table.shape[1], block_size, stride_rows, T, H, float(sm_scale), float(kv_scale), row_bytes, split,
+              out.data_ptr(), H * D_LAT, D_LAT, lse.data_ptr(), H, wp, wn, _stream(q))
+    return out
+
+
 def attend_partial(q, pool, idx, sm_scale, kv_scale=1.0, opart=None, lpart=None, split=1, kcount=None, R=None,
                    row_bytes=None):
     """Like attend, but the result stays as `split` normalized fp32 partials (opart [split, T, H, 512], lpart

@@ -344,6 +344,15 @@ int spmla_attn576_ws(const void* q, long long q_st, long long q_sh, const void* 
  * lse_out = ln(e^lse + e^lse'); both -inf -> o = 0, lse = -inf. The host-tier attention of a decode step merges the
  * HBM tier's partial this way, in place of spmla_lse_merge over two partials (the reference's tier combine,
  * dotsnote/engine/arcstats_pkg/arcstats/sparse_offload.py:519-538, fused into the second tier's kernel). */
+/* spmla_attn (row_bytes 656) or spmla_attn576 / spmla_attn576_ws (576) over the pages of a cache: topk[t][k] are positions
+ * of token t's request, formed into rows as spmla_rows_from_topk does (block_size a power of two, else SPMLA_ELIMIT;
+ * bt_cols >= 1), in the attention kernel. ws: as spmla_attn's, for S > 1. */
+int spmla_attn_paged(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* topk,
+                     long long tk_st, int K, const int* req, const int* block_table, long long bt_st, int bt_cols,
+                     int block_size, long long stride_rows, int T, int H, float sm_scale, float kv_scale, int row_bytes,
+                     int S, void* out, long long o_st, long long o_sh, float* lse, long long lse_st, void* ws,
+                     long long ws_bytes, void* stream);
+
 int spmla_attn_merge(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
                      long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale,
                      const float* prior_o, long long po_st, long long po_sh, const float* prior_lse, long long pl_st,

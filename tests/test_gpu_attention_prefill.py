@@ -84,3 +84,38 @@ def test_prefill_kernel_vs_oracle(dev, fmt, T, H, K, form):
     # "rising": outputs up to 1e3; P' rounded to f16 and the bf16 output: 2^-8 of the token's largest value
     tol = 1e-2 if form != "rising" else 2 ** -8 * np.abs(o_ref).max()
     assert attn_excess(o, o_ref, tol) <= 0
+
+
+@pytest.mark.parametrize("fmt", [656, 576])
+@pytest.mark.parametrize("T,H,K,bs,pad", [
+    (3, 32, 2048, 64, 0),              # splits merged in the kernel
+    (5, 128, 40, 1, 0),                # one tile and eight rows, one row per block
+    (130, 64, 200, 16, 3),             # unsplit, a padded block stride
+    (256, 128, 300, 128, 0),           # the 128-head kernel
+    (256, 128, 2048, 64, 1),
+])
+def test_paged_rows_formed_in_the_kernel(dev, fmt, T, H, K, bs, pad):
+    """attend_paged against attend over rows_from_topk: the same bits, with entries of -1, positions past the table and
+    negative table entries, from strided views."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    print(f"[paged attention] fmt={fmt} T={T} H={H} K={K} bs={bs} pad={pad}", flush=True)
+    g = torch.Generator().manual_seed(T + K + bs)
+    nreq, cols, stride = 3, max(2, 1024 // bs), bs + pad
+    nblk = nreq * cols
+    pool = torch.from_numpy(_pool(fmt, nblk * stride, 1.0)).to(dev)
+    table = torch.randperm(nblk, generator=g).view(nreq, cols).to(torch.int32)
+    table[1, cols // 2] = -1
+    table = torch.nn.functional.pad(table, (0, 5), value=-7).to(dev)[:, :cols]
+    pos = torch.randint(0, cols * bs, (T, K + 9), generator=g).to(torch.int32)
+    pos[torch.rand(T, K + 9, generator=g) < 0.05] = -1
+    pos[0, :3] = torch.tensor([cols * bs, cols * bs + bs, 2 ** 31 - 1], dtype=torch.int32)
+    pos[min(2, T - 1), :] = -1
+    pos = pos.to(dev)[:, :K]
+    req = torch.randint(0, nreq, (T,), generator=g).to(torch.int32).to(dev)
+    q = make_q(T, H, seed=K).to(dev)
+    rows = kernels.rows_from_topk(pos, req, table, bs, stride_rows=stride)
+    a, _ = kernels.attend(q, pool, rows, SM, 0.7)
+    b = kernels.attend_paged(q, pool, pos, req, table, bs, stride, SM, 0.7, row_bytes=fmt)
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+    assert kernels.attend_paged(q, pool, pos, req, table, 48, 48, SM, row_bytes=fmt) is None
