@@ -81,3 +81,44 @@ def test_index_key_write(dev, ue8m0):
     exp = np.zeros((R, 132), dtype=np.uint8)
     ref.index_key_write(bf16_bits(k), slots.numpy(), exp, ue8m0=ue8m0)
     assert np.array_equal(store.cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("bs", [64, 48, 0])
+def test_encoding_of_every_bf16_value(dev, bs):
+    """All finite bf16 values as latent and index-key values, in groups of neighbouring and of mixed magnitudes: the
+    oracle's bytes (block sizes with and without a power of two). A token that holds a NaN or an infinity leaves its
+    neighbours alone."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    bits = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    n = 1024
+    kv = torch.empty(n, 512, dtype=torch.bfloat16)
+    kv.view(-1)[: 1 << 16] = torch.where(torch.isfinite(bits.float()), bits, torch.zeros_like(bits))
+    g = torch.Generator().manual_seed(3)
+    fin = bits[torch.isfinite(bits.float())]
+    rest = fin[torch.randint(0, fin.numel(), (n - 128, 512), generator=g)]     # finite groups of mixed magnitudes
+    rest[:, ::128] = torch.exp2(torch.randint(-60, 60, (n - 128, 4), generator=g).float()).to(torch.bfloat16)
+    rest = torch.where(rest.float().abs() > rest[:, ::128].float().abs().repeat_interleave(128, 1), rest[:, ::128].repeat_interleave(128, 1), rest)
+    kv[128:] = rest
+    kv[500:508, ::100] = torch.tensor([float("nan"), float("inf")] * 3)
+    odd = torch.zeros(n, dtype=torch.bool)
+    odd[500:508] = True
+    pe = fin[torch.randint(0, fin.numel(), (n, 64), generator=g)]
+    R = 64 * 48
+    slots = torch.randperm(R, generator=g)[:n].to(torch.int64)
+    shape = (R // bs, bs) if bs else (R,)
+    for fmt, rowb, write in ((0, 656, lambda c: ref.cache_write_656(bf16_bits(kv), bf16_bits(pe), slots.numpy(), c)),
+                             (1, 576, lambda c: ref.cache_write_576(bf16_bits(kv), bf16_bits(pe), slots.numpy(), c, 0.3))):
+        cache = torch.zeros(*shape, rowb, dtype=torch.uint8, device=dev)
+        kernels.cache_write(kv.to(dev), pe.to(dev), slots.to(dev), cache, fmt=fmt, kv_scale=0.3 if fmt else 1.0)
+        exp = np.zeros((R, rowb), dtype=np.uint8)
+        write(exp)
+        got = cache.cpu().numpy().reshape(R, rowb)
+        got[slots[odd]] = exp[slots[odd]]
+        assert np.array_equal(got, exp), f"fmt {fmt}: {(got != exp).sum()} bytes"
+    k = kv.view(-1, 128)[:2000]                            # (of the tokens without NaNs)
+    sl = torch.randperm(R, generator=g)[: k.shape[0]].to(torch.int64)
+    store = torch.zeros(*shape, 132, dtype=torch.uint8, device=dev)
+    kernels.index_key_write(k.to(dev), sl.to(dev), store)
+    exp = np.zeros((R, 132), dtype=np.uint8)
+    ref.index_key_write(bf16_bits(k), sl.numpy(), exp)
+    assert np.array_equal(store.cpu().numpy().reshape(R, 132), exp)
