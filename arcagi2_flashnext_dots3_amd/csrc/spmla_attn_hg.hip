@@ -807,9 +807,8 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
 }
 
 // Per-token launch of attn_kernel<false> (r576: attn_kernel<false, true> over Row576 rows): the arguments of
-// spmla_attn_splitk / spmla_attn_merge / spmla_attn576, already checked by the caller (spmla_attn.hip, which chooses
-// this kernel for launches with few tokens, and for every Row576 launch). Any K: row ids are read from global memory
-// a tile ahead, not staged.
+// spmla_attn_splitk / spmla_attn_merge / spmla_attn576 / spmla_attn_paged, already checked by the caller (spmla_attn.hip,
+// which chooses the kernel). Any K: row ids are read from global memory a tile ahead, not staged.
 int launch_tokens(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
                   long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale, int S,
                   void* out, long long o_st, long long o_sh, float* lse, long long lse_st, float* opart,

@@ -490,8 +490,7 @@ def run_config4(a, dev):
         # the reference's fp16 logits mode (ARC_SHARD_F16OUT): fp16 logits, top-k on fp16 keys
         ms_l16 = _graph_ms(lambda: logits(lg16), a.steps, a.warmup, reps=20)
         ms_t16 = _graph_ms(lambda: kernels.topk(lg16, ctx, K, out=out), a.steps, a.warmup, reps=20)
-        # the step as ShardStore.logits_topk runs it at P = 1: the top-k's first histogram built in the logits
-        # epilogue (spmla_index_logits_hist), then the top-k without its histogram pass (spmla_topk_ws_prehist)
+        # the step as ShardStore.logits_topk runs it at P = 1: spmla_index_logits_hist, then spmla_topk_ws_prehist
         ws = torch.empty(int(kernels._lib.lib().spmla_topk_ws_bytes(B, L, K)), dtype=torch.uint8, device=dev)
 
         def fused(dst=lg):
@@ -623,7 +622,7 @@ def run_config5(a, dev):
     roof = {"bound": "mfma", "achieved": round(tf, 1), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(tf / BF16_PEAK_TFLOPS, 4), "traffic": None, "kernel": "spmla::attn::fwd_kernel"}
     res = _line("chunked prefill attention ms (8192 queries x 128 heads x top-2048) + cache write us", ms_a, "ms", a,
-                ms_a + ms_w, "f16 MFMA (QK latent and PV), bf16 MFMA (rope), fp32 accumulate",
+                ms_a + ms_w, "bf16 MFMA (QK), f16 MFMA (PV), fp32 accumulate",
                 {"workload": "BASELINE config 5: 8192 queries, 128 heads, top-2048 of <= 65536 prior rows; write "
                              "8192 rows at random slots of a paged cache (block 64)"}, roof, cpu, hib=False,
                 cache_write_us=round(ms_w * 1e3, 2),

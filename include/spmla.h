@@ -289,9 +289,8 @@ int spmla_compact_stage(const long long* rows, int tot, const int* sidx, long lo
  * opart != NULL (required for S > 1): the K entries are cut into S splits; opart [S][T][H][512] fp32 (normalized)
  * and lsepart [S][T][H] receive per-split partials for spmla_lse_merge (S = 1: one fp32 partial, e.g. per tier);
  * out / lse are not written then. Any K. Two kernels serve it with the same results up to fp32 summation order:
- * launches of at most 512 (token, split, 32-head group) work items run 32 heads per workgroup (decode batches),
- * longer ones 128 heads per workgroup (prefill chunks; there ceil(ceil(K / S) / 32) * 32 > 2048 falls back to the
- * first kernel).
+ * decode batches and launches with few heads run 32 heads per workgroup, prefill chunks 128 heads per workgroup (there
+ * ceil(ceil(K / S) / 32) * 32 > 2048 falls back to the first kernel).
  * Replaces LayerOffload.attend's decode kernels (oa2_v2_launch dotsnote/engine/arcstats_pkg/arcstats/csrc/
  * offload_attn2.cu:2021-2104, offload_split_launch csrc/offload_attn.cu:1155-1200, _sparse_mla_offload_split_kernel
  * sparse_offload.py:419-516) and triton_bf16_mla_sparse_interface (vllm_patch/.../ops/xpu_mla_sparse.py:182-278),
@@ -304,7 +303,7 @@ int spmla_attn_splitk(const void* q, long long q_st, long long q_sh, const void*
 /* spmla_attn_splitk over Row576 rows, the plugin's per-tensor "fp8" cache: pool [R] rows of 512 latent + 64 rope
  * e4m3 codes (no per-group scales), every code times the tensor's kv_scale. Same arguments, outputs and results
  * (o = kv_scale * softmax(s) codes_latent, s = sm_scale * kv_scale * q . codes); S > 1 needs opart / lsepart (the
- * fp32 partials for spmla_lse_merge). Any K; one kernel (32 heads per workgroup) serves every launch.
+ * fp32 partials for spmla_lse_merge). Any K; the kernel is chosen as for spmla_attn_splitk.
  * Replaces triton_bf16_mla_sparse_interface over the fp8 per-tensor rows (PortableSparseImpl._run,
  * dotsnote/engine/arcstats_pkg/arcstats/dsa_sm89.py:379-391, kernel vllm_patch/.../ops/xpu_mla_sparse.py:77-161). */
 int spmla_attn576(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
