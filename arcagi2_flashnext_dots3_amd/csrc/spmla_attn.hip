@@ -28,8 +28,8 @@
 // tile j with the softmax of tile j + 1), one barrier after each, and written in slices: every MFMA is followed by a
 // fence and carries the side work that fits under its 32 cycles. What bounds it is issue: one wave per SIMD (512
 // registers) issues about one instruction per 4 cycles (8-byte ones 4.6, scalar ones 8: measured), 620 (Row656) or 480
-// per tile next to 68 MFMAs; matrix cores are busy 41 - 45 % of the time, LDS 30 %. Hence addresses that are a register
-// plus immediates, no wait states where none are needed, no scalar work per slice.
+// per tile, 68 of them MFMAs; matrix cores are busy 39 % (Row656) and 44 % (Row576) of the time, LDS 28 and 26 %. Hence
+// addresses that are a register plus immediates, no wait states where none are needed, no scalar work per slice.
 // T = 2048, H = 128, K = 2048: Row656 1304 us (896 TFLOP/s), before (heads split over the waves) 1580 us; Row576 1160 us,
 // before (head-group kernel) 1440 us; back to back for a second the card lowers its clock: 1400 us against 1545, Row576
 // T = 1455 900 us against 1050.
