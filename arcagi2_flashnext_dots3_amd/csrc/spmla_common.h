@@ -112,16 +112,18 @@ __device__ inline int remap_xcd(int i, int n) {
 }
 
 // ---- paged rows: position x of a token's request -> row bt[req[t]][x >> sh] * stride + (x & (2^sh - 1)), -1 for x < 0,
-// past the table's columns or a negative entry (spmla_rows_from_topk's rule). bt null: no pages, x is the row.
+// past the table's columns or a negative entry (spmla_rows_from_topk's rule: a token without a position in the table may
+// have any request, its table row is not read). bt null: no pages, x is the row.
 struct Pages {
   const int* req; const int* bt; long long bt_st; int cols, sh; long long stride;
 };
-__device__ inline int page_entry(const Pages& g, const int* btrow, int x) {      // (cols >= 1)
-  const uint32_t b = (uint32_t)x >> g.sh;
-  return btrow[b < (uint32_t)g.cols ? b : 0u];
+__host__ __device__ inline int page_entry(const Pages& g, const int* btrow, int x) {   // -1: x has none
+  int b = -1;
+  if (x >= 0 && (x >> g.sh) < g.cols) b = btrow[x >> g.sh];
+  return b;
 }
-__device__ inline int page_row(const Pages& g, int x, int blk) {
-  return x >= 0 && (x >> g.sh) < g.cols && blk >= 0 ? (int)(blk * g.stride + (x & ((1 << g.sh) - 1))) : -1;
+__host__ __device__ inline int page_row(const Pages& g, int x, int blk) {              // blk: x's entry
+  return blk >= 0 ? (int)(blk * g.stride + (x & ((1 << g.sh) - 1))) : -1;
 }
 
 // ---- launch error codes ----------------------------------------------------------------------------------

@@ -119,3 +119,24 @@ def test_paged_rows_formed_in_the_kernel(dev, fmt, T, H, K, bs, pad):
     torch.cuda.synchronize()
     assert torch.equal(a, b)
     assert kernels.attend_paged(q, pool, pos, req, table, 48, 48, SM, row_bytes=fmt) is None
+
+
+@pytest.mark.parametrize("fmt", [656, 576])
+@pytest.mark.parametrize("T,K", [(3, 2048), (5, 40), (256, 300)])    # merged splits, unsplit, the 128-head kernel
+def test_paged_padding_tokens_of_no_request(dev, fmt, T, K):
+    """Tokens without a position in the table may have any request id: the same bits as attend over rows_from_topk."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    print(f"[paged attention] padding fmt={fmt} T={T} K={K}", flush=True)
+    g = torch.Generator().manual_seed(T + K)
+    bs, nreq, cols, H = 64, 2, 12, 128
+    pool = torch.from_numpy(_pool(fmt, nreq * cols * bs, 1.0)).to(dev)
+    table = torch.randperm(nreq * cols, generator=g).view(nreq, cols).to(torch.int32).to(dev)
+    pos = torch.randint(0, cols * bs, (T, K), generator=g).to(torch.int32)
+    req = torch.randint(0, nreq, (T,), generator=g).to(torch.int32)
+    pos[1], req[1] = -1, -1
+    pos[T - 1], req[T - 1] = cols * bs, 2 ** 31 - 1
+    pos, req, q = pos.to(dev), req.to(dev), make_q(T, H, seed=K).to(dev)
+    a, _ = kernels.attend(q, pool, kernels.rows_from_topk(pos, req, table, bs), SM, 0.7)
+    b = kernels.attend_paged(q, pool, pos, req, table, bs, bs, SM, 0.7, row_bytes=fmt)
+    torch.cuda.synchronize()
+    assert torch.equal(a, b) and not a[1].any() and not a[T - 1].any()
