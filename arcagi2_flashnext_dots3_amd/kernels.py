@@ -770,11 +770,13 @@ def attend_paged(q, pool, topk_pos, req, block_table, block_size, stride_rows, s
                  row_bytes=ROW656):
     """attend over rows_from_topk(topk_pos, req, block_table, block_size, stride_rows) with the rows formed in the
     attention kernel (spmla_attn_paged) -> out [T, H, 512] bf16, or None when that kernel does not take the call (the
-    caller then forms the rows): block_size not a power of two, no table columns, more than 65535 tokens, tensors that
-    are not int32 with contiguous columns."""
+    caller then forms the rows): block_size not a power of two, no table columns, more than 65535 tokens, fewer
+    positions or request ids than tokens (the kernel reads one of each for every token), tensors that are not int32 with
+    contiguous columns."""
     T, H, _ = q.shape
     K = topk_pos.shape[1]
     if (block_size <= 0 or block_size & (block_size - 1) or block_table.shape[1] == 0 or not 0 < T <= 65535 or K == 0
+            or topk_pos.shape[0] < T or req.shape[0] < T
             or not (topk_pos.dtype == req.dtype == block_table.dtype == torch.int32)
             or topk_pos.stride(1) != 1 or block_table.stride(1) != 1 or not req.is_contiguous() or not query_ok(q)):
         return None

@@ -345,7 +345,8 @@ int spmla_attn576_ws(const void* q, long long q_st, long long q_sh, const void* 
  * dotsnote/engine/arcstats_pkg/arcstats/sparse_offload.py:519-538, fused into the second tier's kernel). */
 /* spmla_attn (row_bytes 656) or spmla_attn576 / spmla_attn576_ws (576) over the pages of a cache: topk[t][k] are positions
  * of token t's request, formed into rows as spmla_rows_from_topk does (block_size a power of two, else SPMLA_ELIMIT;
- * bt_cols >= 1), in the attention kernel. ws: as spmla_attn's, for S > 1. */
+ * bt_cols >= 1), in the attention kernel. req[t] is read for every token (any value where the token has no position in
+ * the table). ws: as spmla_attn's, for S > 1. */
 int spmla_attn_paged(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* topk,
                      long long tk_st, int K, const int* req, const int* block_table, long long bt_st, int bt_cols,
                      int block_size, long long stride_rows, int T, int H, float sm_scale, float kv_scale, int row_bytes,

@@ -6,8 +6,9 @@ import sys
 
 import numpy as np
 import pytest
+import torch
 
-from arcagi2_flashnext_dots3_amd import build
+from arcagi2_flashnext_dots3_amd import _lib, build, kernels
 
 SRC = r"""
 #include "spmla_common.h"
@@ -65,3 +66,18 @@ def test_rows_of_positions(lib, sh, cols, stride):
     blk = x >> sh
     entry = np.where((x >= 0) & (blk < cols), bt[np.clip(blk, 0, cols - 1)], -1)
     assert np.array_equal(out, np.where(entry >= 0, entry * stride + (x & ((1 << sh) - 1)), -1))
+
+
+@pytest.mark.parametrize("nreq,npos,taken", [(4, 4, True), (6, 5, True), (3, 4, False), (4, 3, False), (0, 4, False)])
+def test_fewer_request_ids_or_positions_than_tokens(monkeypatch, nreq, npos, taken):
+    """The kernel reads a request id and a list of positions for every token: attend_paged leaves calls with fewer to
+    the separate conversion, which looks up only what a position needs."""
+    calls = []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: calls.append(name))
+    monkeypatch.setattr(kernels, "_stream", lambda t: None)
+    monkeypatch.setattr(kernels, "auto_split", lambda T, H, K: 1)
+    q = torch.zeros(4, 16, 576, dtype=torch.bfloat16)
+    i32 = dict(dtype=torch.int32)
+    out = kernels.attend_paged(q, torch.zeros(64, 656, dtype=torch.uint8), torch.zeros(npos, 64, **i32),
+                               torch.zeros(nreq, **i32), torch.zeros(2, 1, **i32), 64, 64, 0.1)
+    assert (out is not None) == taken and calls == (["spmla_attn_paged"] if taken else [])
