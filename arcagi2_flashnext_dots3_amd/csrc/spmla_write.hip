@@ -14,10 +14,11 @@
 // Index key (dotsnote/engine/arcstats_pkg/arcstats/shard_indexer.py:42-60): s = max(amax, 1e-4) / 448 (optionally
 //   rounded up to a power of two, UE8M0), code = e4m3fn_rne(k / s); 132-byte row [128 codes | fp32 s].
 //
-// One wave per token, 4 tokens per 256-thread block; slot < 0 (padding) and slot >= R are skipped. The encoding bounded these
-// kernels (a branchy software encoder and one division per value): finite groups now use the hardware's conversion, which
-// equals e4m3_rne on every fp32 value except the sign of NaNs (all 2^32 compared), and one reciprocal per group. The value
-// loads do not wait for the slot. 8192 tokens: rows 8.2 -> 4.9 us, index keys 5.0 -> 3.8; 8 tokens: 4.1 -> 2.6 and 2.9 -> 2.7.
+// One wave per token, 4 tokens per 256-thread block; tokens with slot < 0 (padding), slot >= R or another rank's slot are
+// skipped and their values are not read (a padded batch may hold fewer rows of values than slots). The encoding bounded
+// these kernels (a branchy software encoder and one division per value): finite groups now use the hardware's conversion,
+// which equals e4m3_rne on every fp32 value except the sign of NaNs (all 2^32 compared), and one reciprocal per group.
+// 8192 tokens: rows 8.2 -> 4.9 us, index keys 5.0 -> 3.8; 8 tokens: 4.1 -> 2.6 and 2.9 -> 2.7.
 #include "spmla_common.h"
 
 namespace spmla {
@@ -72,10 +73,10 @@ __global__ void __launch_bounds__(256) cache_write_kernel(WriteParams p) {
   const int tok = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
   const int lane = threadIdx.x & 63;
   if (tok >= p.n) return;
-  const u32x4 raw = *(const u32x4*)(p.kv + (long long)tok * p.kv_st + lane * 8);
-  const uint2 rope = *(const uint2*)(p.pe + (long long)tok * p.pe_st + (lane & 15) * 4);
   const long long slot = p.slots[tok];
   if (slot < 0 || slot >= p.R) return;
+  const u32x4 raw = *(const u32x4*)(p.kv + (long long)tok * p.kv_st + lane * 8);
+  const uint2 rope = *(const uint2*)(p.pe + (long long)tok * p.pe_st + (lane & 15) * 4);
   const int rowb = p.fmt == 0 ? ROW656 : (p.fmt == 1 ? ROW576 : ROW400);
   long long blk;
   int off;
@@ -169,11 +170,11 @@ __global__ void __launch_bounds__(256) key_write_kernel(KeyParams p) {
   const int tok = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
   const int lane = threadIdx.x & 63;
   if (tok >= p.n) return;
-  const uint32_t raw = *(const uint32_t*)(p.k + (long long)tok * p.k_st + lane * 2);
   const long long slot = p.slots[tok];
   if (slot < 0 || (p.P > 1 && slot % p.P != p.rank)) return;
   const long long r = p.P > 1 ? slot / p.P : slot;
   if (r >= p.R_local) return;
+  const uint32_t raw = *(const uint32_t*)(p.k + (long long)tok * p.k_st + lane * 2);
   long long b;
   int t;
   div_slot(r, p.rpb, p.sh, b, t);
