@@ -102,7 +102,7 @@ __device__ inline float half_swap(float x) {
 // accumulator (read by the scale FMAs) to VGPRs; the statements are volatile so that they keep their order. Hazards the
 // compiler cannot see inside asm are kept off by that order, not by wait states (each would take an issue slot): an
 // operand is converted a slice before its MFMA (2 wait states after a VALU write), and a chain's result is read three or
-// more MFMAs, or 11 wait states, after its last one (chain_end). Back-to-back MFMAs of one chain have srcC == vdst exactly
+// more MFMAs, or 12 wait states, after its last one (chain_end). Back-to-back MFMAs of one chain have srcC == vdst exactly
 // (forwarded). tests/test_attention_hazards.py checks the compiled order.
 __device__ inline f32x16 qk_first(bf16x8 a, bf16x8 b) {
   f32x16 d;
@@ -113,11 +113,12 @@ __device__ inline f32x16 qk_next(bf16x8 a, bf16x8 b, f32x16 c) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
   return c;
 }
-// after the last MFMA of a chain and N instructions that do not touch c: what is left of 11 wait states
+// after the last MFMA of a chain and N instructions that do not touch c: what is left of 12 wait states (the compiler's
+// s_nop 11 behind this MFMA as a builtin)
 template <int N>
 __device__ inline void chain_end(f32x16& c) {
   __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_nop %1" : "+v"(c) : "n"(N < 11 ? 10 - N : 0));
+  asm volatile("s_nop %1" : "+v"(c) : "n"(N < 12 ? 11 - N : 0));
 }
 // the maximum of x over the two lanes l, l ^ 32
 __device__ inline float half_max(float x) {

@@ -1,7 +1,8 @@
 """The attention kernels' inline-asm MFMA and DPP statements rely on the order of the compiled code instead of wait
-states, which the compiler does not add for asm: in their assembly no MFMA operand and no DPP source is
-written by the VALU in the two instructions before, and no VGPR result of an MFMA is read or overwritten before three
-more MFMAs were issued or 11 wait states passed."""
+states, which the compiler does not add for asm: in their assembly, along every branch too, no MFMA operand and no DPP
+source is written by the VALU in the two instructions before, and no VGPR result of an MFMA is read or overwritten (by a
+load either) before three more MFMAs were issued or 12 wait states passed, which is what the compiler puts behind the
+same MFMA when it comes from a builtin."""
 import os
 import re
 import subprocess
@@ -10,6 +11,8 @@ import pytest
 
 from arcagi2_flashnext_dots3_amd import build
 
+WAIT = 12
+LOADS = ("ds_read", "global_load", "buffer_load", "scratch_load", "flat_load")
 REG = re.compile(r"([av])(?:\[(\d+):(\d+)\]|(\d+))$")
 
 
@@ -43,11 +46,23 @@ def hazards(lines):
         if "mfma" in op:
             mfma.append((dst, now))
         else:
-            touched = {r for r in src | (dst if op.startswith("v_") else set()) if r[0] == "v"}
-            if any(touched & d and now - at - 1 < 11 for d, at in mfma[-3:]):
+            touched = {r for r in src | (dst if op.startswith(("v_", *LOADS)) else set()) if r[0] == "v"}
+            if any(touched & d and now - at - 1 < WAIT for d, at in mfma[-3:]):
                 bad.append((n, l))
         now += 1 + (int(toks[0], 0) if op == "s_nop" else 0)
         hist.append((op, set() if stores else dst, toks[0]))
+    return bad
+
+
+def branch_hazards(body, window=60):
+    """The same over the code before and after every branch of the kernel's assembly."""
+    labels = {l.split(":")[0]: i for i, l in enumerate(body) if re.match(r"\.LBB\w+:", l)}
+    bad = []
+    for i, l in enumerate(body):
+        m = re.match(r"\s*s_c?branch\w*\s+(\.LBB\w+)", l)
+        if m:
+            j = labels[m[1]]
+            bad += [(l.strip(), *b) for b in hazards(body[max(0, i - window):i + 1] + body[j:j + window])]
     return bad
 
 
@@ -59,7 +74,12 @@ def test_scanner_finds_planted_hazards():
     assert hazards(["v_mov_b32_e32 v5, v9", "s_nop 0", m])
     a = "v_mfma_f32_32x32x16_f16 a[0:15], v[40:43], v[44:47], a[0:15]"
     assert hazards([m, a, a, "ds_write_b128 v9, v[16:19] offset:64"])
-    assert hazards([m, "s_nop 9", "v_add_f32_e32 v1, v16, v2"]) and not hazards([m, "s_nop 10", "v_add_f32_e32 v1, v16, v2"])
+    assert hazards([m, "s_nop 10", "v_add_f32_e32 v1, v16, v2"]) and not hazards([m, "s_nop 11", "v_add_f32_e32 v1, v16, v2"])
+    assert hazards([m, "ds_read_b128 v[20:23], v9"]) and not hazards([m, "ds_read_b128 v[32:35], v9"])
+    loop = [".LBB0_1:", "v_add_f32_e32 v1, v16, v2", "s_nop 15", m, "s_cbranch_scc1 .LBB0_1", "s_nop 15"]
+    assert not hazards(loop) and branch_hazards(loop)
+    skip = [m, "s_cbranch_scc1 .LBB0_2", "s_nop 15", ".LBB0_2:", "v_add_f32_e32 v1, v16, v2"]
+    assert not hazards(skip) and branch_hazards(skip)
     assert not hazards([m, a, a, a, "ds_write_b128 v9, v[16:19] offset:64"])
 
 
@@ -77,4 +97,42 @@ def test_compiled_order_of_asm_statements(tmp_path, src, kernel, count):
         end = next(i for i in range(s, len(text)) if ".Lfunc_end" in text[i])
         body = text[s:end]
         assert sum("v_mfma_f32_32x32x16_bf16" in l for l in body) >= 36
-        assert not hazards(body)
+        assert not hazards(body) and not branch_hazards(body)
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no hipcc")
+def test_wait_states_are_the_compilers(tmp_path):
+    src = tmp_path / "m.hip"
+    src.write_text("""#include <hip/hip_runtime.h>
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__global__ void k(const bf16x8* a, const bf16x8* b, f32x16* o) {
+  o[threadIdx.x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[threadIdx.x], b[threadIdx.x], f32x16{}, 0, 0, 0) * 2.0f;
+}
+""")
+    out = tmp_path / "m.s"
+    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", str(src), "-o", str(out)], check=True,
+                   capture_output=True)
+    m = re.search(r"v_mfma_f32_32x32x16_bf16 v.*\n\s*s_nop (\d+)", out.read_text())
+    assert int(m[1]) + 1 <= WAIT
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="no hipcc")
+def test_chain_end_fills_the_wait(tmp_path):
+    """chain_end alone is the whole wait, with nothing else in between."""
+    src = tmp_path / "c.hip"
+    src.write_text("""#include "spmla_attn_hg.hip"
+__global__ void chain_probe(const bf16x8* a, const bf16x8* b, f32x16* o) {
+  f32x16* dst = o + threadIdx.x;
+  f32x16 c = spmla::pk::qk_first(a[threadIdx.x], b[threadIdx.x]);
+  spmla::pk::chain_end<0>(c);
+  *dst = c * 2.0f;
+}
+""")
+    out = tmp_path / "c.s"
+    subprocess.run([build.HIPCC, *build.FLAGS, "-I", build.CSRC, "--cuda-device-only", "-S", str(src), "-o", str(out)],
+                   check=True, capture_output=True)
+    text = out.read_text().split("\n")
+    at = next(i for i, l in enumerate(text) if re.match(r"_Z11chain_probe\S+:", l))
+    nops = re.findall(r"#ASMSTART\n\s*s_nop (\d+)\n", "\n".join(text[at:]))      # (the compiler's own nops not counted)
+    assert int(nops[0]) + 1 >= WAIT
