@@ -5,6 +5,7 @@ offload_cuda.split_partials, fast_topk.local/merge, ShardStore.write/logits, Lay
 RuntimeError on a failed launch and never falls back to a CPU path.
 """
 import functools
+import threading
 
 import torch
 
@@ -259,6 +260,17 @@ def _attn_workspace(device, T, H, split, private=False):
             ws[_WS_CNT[key]:cnt].zero_()
         _WS_CNT[key] = cnt
     return ws
+
+
+_WS_LOCK = threading.Lock()
+
+
+def _merged_call(device, T, H, split, private, stream, name, *args):
+    """Entry point `name` with _attn_workspace's workspace appended. The counters that a launch finds zero and the launch
+    itself are queued together: host threads may share a stream, and so its workspace."""
+    with _WS_LOCK:
+        ws = _attn_workspace(device, T, H, split, private)
+        _lib.call(name, *args, ws.data_ptr(), ws.numel(), stream)
 
 
 def _attn_counter_bytes(T, H):
@@ -744,10 +756,9 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
                       idx.stride(0), K, _ptr(kcount), T, H, float(sm_scale), float(kv_scale), 1, out.data_ptr(),
                       out.stride(0), out.stride(1), lse.data_ptr(), lse.stride(0), None, None, st)
             return out, lse
-        ws = _attn_workspace(q.device, T, H, split, private=True)
-        _lib.call("spmla_attn576_ws", q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(), idx.stride(0),
-                  K, _ptr(kcount), T, H, float(sm_scale), float(kv_scale), split, out.data_ptr(), out.stride(0),
-                  out.stride(1), lse.data_ptr(), lse.stride(0), ws.data_ptr(), ws.numel(), st)
+        _merged_call(q.device, T, H, split, True, st, "spmla_attn576_ws", q.data_ptr(), q.stride(0), q.stride(1), pptr,
+                     Rv, idx.data_ptr(), idx.stride(0), K, _ptr(kcount), T, H, float(sm_scale), float(kv_scale), split,
+                     out.data_ptr(), out.stride(0), out.stride(1), lse.data_ptr(), lse.stride(0))
         return out, lse
     if split == 1:
         _lib.call("spmla_attn_splitk", q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(),
@@ -755,14 +766,15 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
                   out.stride(0), out.stride(1), lse.data_ptr(), lse.stride(0), None, None, st)
         return out, lse
     _need(1 <= split <= 8, "attend: split must be 1 .. 8")
-    nb = attn_ws_bytes(T, H, split)
+    args = (q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(), idx.stride(0), K, _ptr(kcount), T, H,
+            float(sm_scale), float(kv_scale), split, out.data_ptr(), out.stride(0), out.stride(1), lse.data_ptr(),
+            lse.stride(0))
     if ws is None:
         # from 96 workgroups on (3/8 of the compute units) the unsplit launch needs none: a capture brings its own
-        ws = _attn_workspace(q.device, T, H, split, private=T * ((H + 31) // 32) >= 96)
-    _need(ws.dtype == torch.uint8 and ws.numel() >= nb, "attend: workspace too small")
-    _lib.call("spmla_attn", q.data_ptr(), q.stride(0), q.stride(1), pptr, Rv, idx.data_ptr(), idx.stride(0), K,
-              _ptr(kcount), T, H, float(sm_scale), float(kv_scale), split, out.data_ptr(), out.stride(0),
-              out.stride(1), lse.data_ptr(), lse.stride(0), ws.data_ptr(), ws.numel(), st)
+        _merged_call(q.device, T, H, split, T * ((H + 31) // 32) >= 96, st, "spmla_attn", *args)
+    else:
+        _need(ws.dtype == torch.uint8 and ws.numel() >= attn_ws_bytes(T, H, split), "attend: workspace too small")
+        _lib.call("spmla_attn", *args, ws.data_ptr(), ws.numel(), st)
     return out, lse
 
 
@@ -783,15 +795,16 @@ def attend_paged(q, pool, topk_pos, req, block_table, block_size, stride_rows, s
     split = auto_split576(T, H, K) if row_bytes == ROW576 else auto_split(T, H, K)
     out = torch.empty(T, H, D_LAT, dtype=torch.bfloat16, device=q.device)
     lse = torch.empty(T, H, dtype=torch.float32, device=q.device)
-    wp, wn = None, 0
-    if split > 1:
-        ws = _attn_workspace(q.device, T, H, split, private=row_bytes == ROW576 or T * ((H + 31) // 32) >= 96)
-        wp, wn = ws.data_ptr(), ws.numel()
     q_st, q_sh, _ = q.stride()
-    _lib.call("spmla_attn_paged", q.data_ptr(), q_st, q_sh, pool.data_ptr(), int(R if R is not None else pool.shape[0]),
-              topk_pos.data_ptr(), topk_pos.stride(0), K, req.data_ptr(), block_table.data_ptr(), block_table.stride(0),
-              block_table.shape[1], block_size, stride_rows, T, H, float(sm_scale), float(kv_scale), row_bytes, split,
-              out.data_ptr(), H * D_LAT, D_LAT, lse.data_ptr(), H, wp, wn, _stream(q))
+    args = (q.data_ptr(), q_st, q_sh, pool.data_ptr(), int(R if R is not None else pool.shape[0]), topk_pos.data_ptr(),
+            topk_pos.stride(0), K, req.data_ptr(), block_table.data_ptr(), block_table.stride(0), block_table.shape[1],
+            block_size, stride_rows, T, H, float(sm_scale), float(kv_scale), row_bytes, split, out.data_ptr(), H * D_LAT,
+            D_LAT, lse.data_ptr(), H)
+    if split > 1:
+        _merged_call(q.device, T, H, split, row_bytes == ROW576 or T * ((H + 31) // 32) >= 96, _stream(q),
+                     "spmla_attn_paged", *args)
+    else:
+        _lib.call("spmla_attn_paged", *args, None, 0, _stream(q))
     return out
 
 

@@ -260,3 +260,42 @@ def test_workspace_under_capture_reuses_the_eager_one(monkeypatch):
     assert b is big and key is None
     with pytest.raises(ValueError, match="graph capture"):
         kernels._workspace("attn", d0, 5000)
+
+
+def test_merged_launches_of_two_threads_on_one_stream(monkeypatch):
+    """Two host threads share a stream's attention workspace. A launch of few counters uses the bytes behind them as
+    scratch: it must not come between the clearing of another's counters and that launch."""
+    import ctypes
+    import threading
+    import time
+    from arcagi2_flashnext_dots3_amd import _lib, kernels
+    monkeypatch.setattr(kernels, "_WS", {})
+    monkeypatch.setattr(kernels, "_stream", lambda t: 0)
+    monkeypatch.setattr(kernels, "_device_stream", lambda d: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    H, big, small = 16, 100, 8
+    assert kernels._attn_counter_bytes(big, H) > kernels._attn_counter_bytes(small, H)
+    small_done, dirty = threading.Event(), []
+
+    def launch(name, *a):                       # what the kernel needs and leaves of its workspace
+        T = a[9]
+        ws, n = a[-3], kernels._attn_counter_bytes(T, H)
+        if T == big:
+            small_done.wait(1.0)
+            dirty.append(any(ctypes.string_at(ws, n)))
+        else:
+            ctypes.memset(ws + n, 7, 4096)
+            small_done.set()
+    monkeypatch.setattr(_lib, "call", launch)
+    pool = torch.zeros(64, 576, dtype=torch.uint8)
+
+    def attend(T):
+        kernels.attend(torch.zeros(T, H, 576, dtype=torch.bfloat16), pool, torch.zeros(T, 64, dtype=torch.int32), 0.1, split=2)
+    first = threading.Thread(target=attend, args=(big,))
+    second = threading.Thread(target=attend, args=(small,))
+    first.start()
+    time.sleep(0.2)
+    second.start()
+    first.join()
+    second.join()
+    assert dirty == [False] and small_done.is_set()
