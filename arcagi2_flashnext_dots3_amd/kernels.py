@@ -689,7 +689,7 @@ def attention_ok(q, idx):
     return query_ok(q) and idx.dtype == torch.int32 and idx.stride(1) == 1
 
 
-ATTN_SPLIT_ROWS = 2048      # rows of one (token, split) in spmla_attn's split merge, rounded up to 32-row tiles
+ATTN_SPLIT_ROWS = 2048      # most rows of one (token, split), in tiles of 32, that spmla_attn merges
 
 
 def _split_cost(n, K, s, cus):
@@ -702,21 +702,26 @@ def _split_cost(n, K, s, cus):
 
 
 @functools.lru_cache(maxsize=4096)
+def _best_split(T, H, K, limit, cus):
+    n = T * ((H + 31) // 32)
+    if 2 * n > cus or n == 0:
+        return 1
+    fits = [s for s in range(1, 9) if s == 1 or limit is None or -(-(-(-K // s)) // 32) * 32 <= limit]
+    return min(fits, key=lambda s: (_split_cost(n, K, s, cus), s))
+
+
 def auto_split576(T, H, K, cus=256):
     """Row splits per token (merged in the kernel, at most 8). 1 when the unsplit launch has more than half as many
     workgroups of 32 heads as there are compute units: a second round would cost what the shorter lists save. Else the
     split of least _split_cost."""
-    n = T * ((H + 31) // 32)
-    if 2 * n > cus or n == 0:
-        return 1
-    return min(range(1, 9), key=lambda s: (_split_cost(n, K, s, cus), s))
+    return _best_split(T, H, K, None, cus)
 
 
 def auto_split(T, H, K, cus=256):
-    """auto_split576 for Row656 pools: 1 as well when a split would hold more than ATTN_SPLIT_ROWS rows (the limit of
-    spmla_attn; the unsplit kernel takes any K)."""
-    s = auto_split576(T, H, K, cus)
-    return 1 if -(-(-(-K // s)) // 32) * 32 > ATTN_SPLIT_ROWS else s
+    """auto_split576 for Row656 pools: of the splits of at most ATTN_SPLIT_ROWS rows each (spmla_attn takes no longer
+    ones; unsplit any K). 128 heads, us: K = 8192, 20 tokens 85 (6 splits), unsplit 144; K = 12000, 12 / 23 tokens 86 /
+    129 (8 splits), unsplit 197 / 205."""
+    return _best_split(T, H, K, ATTN_SPLIT_ROWS, cus)
 
 
 @functools.lru_cache(maxsize=4096)

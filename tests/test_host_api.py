@@ -240,6 +240,17 @@ def test_auto_split_respects_the_split_kernel_row_limit():
         assert kernels.auto_split(Tm, H, 4096) > 1 and kernels.auto_split(Tm + 1, H, 4096) == 1
 
 
+@pytest.mark.parametrize("T,K,least", [(20, 8192, 4), (23, 8192, 4), (12, 12000, 6), (23, 12000, 6), (25, 12000, 6)])
+def test_auto_split_takes_a_permitted_split_of_long_lists(T, K, least):
+    """Where the cheapest split is beyond the row limit, the cheapest of the permitted ones is taken and not the unsplit
+    launch, unless that costs less."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    s = kernels.auto_split(T, 128, K)
+    assert least <= s <= 8 and kernels.auto_split576(T, 128, K) < least
+    cost = [kernels._split_cost(4 * T, K, i, 256) for i in range(1, 9)]
+    assert cost[s - 1] == min(cost[0], *cost[least - 1:])
+
+
 def test_workspace_under_capture_reuses_the_eager_one(monkeypatch):
     """Under HIP graph capture the workspace cache allocates nothing: it hands out the device's largest eager
     workspace of the kind and raises when there is none or it is too small (a buffer allocated inside a capture holds
