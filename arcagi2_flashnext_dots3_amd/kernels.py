@@ -694,11 +694,12 @@ ATTN_SPLIT_ROWS = 2048      # most rows of one (token, split), in tiles of 32, t
 
 def _split_cost(n, K, s, cus):
     """Model of a launch of n * s workgroups over K / s rows each (us): rounds of one workgroup per compute unit, each a
-    fixed part and the longest wave's 32-row tiles; the merge of the splits on top. Fitted to graphed launches at
-    K = 512 .. 2048 (128 heads, K = 2048, T = 1 / 8 / 16 / 32: 1 split 48 / 50 / 50 / 51 us, 2 splits 34 / 36 / 36 / 39,
-    4 splits 25 / 27 / 29 / 54, 8 splits 24 / 26 / 49 / 85)."""
+    fixed part and the longest wave's 32-row tiles; the merge of the splits on top. Fitted to graphed launches of 128
+    heads at K = 384 .. 2048 (1 / 2 / 4 / 8 splits; K = 2048, T = 1 42 / 32 / 26 / 24 us, 16 46 / 35 / 29 / 49, 32 47 / 38 / 51 /
+    79; K = 1024, T = 16 29 / 26 / 25 / 44; K = 512, T = 1 18.5 / 19.2 / 18.7 / 20.9, 16 20.4 / 21.1 / 22.2 / 41.5). Up to 512
+    rows the merge costs what the shorter lists save: the launch stays whole and needs no workspace."""
     tiles = -(-(-(-K // s)) // 32)
-    return -(-n * s // cus) * (12.7 + 2.2 * -(-tiles // 4)) + (3.0 + 0.6 * s if s > 1 else 0.0)
+    return -(-n * s // cus) * (12.7 + 2.2 * -(-tiles // 4)) + (4.5 + 1.0 * s if s > 1 else 0.0)
 
 
 @functools.lru_cache(maxsize=4096)

@@ -251,6 +251,16 @@ def test_auto_split_takes_a_permitted_split_of_long_lists(T, K, least):
     assert cost[s - 1] == min(cost[0], *cost[least - 1:])
 
 
+def test_short_lists_are_not_split():
+    """Launches of up to 512 rows stay whole: shorter ones never needed a workspace (nor a capture of them one reserved
+    before)."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    for K in (1, 40, 256, 385, 416, 480, 511, 512):
+        for H in (16, 32, 64, 128, 160):
+            assert all(f(T, H, K) == 1 for T in range(130) for f in (kernels.auto_split, kernels.auto_split576)), (H, K)
+    assert kernels.auto_split(1, 128, 2048) == 8 and kernels.auto_split(32, 128, 1024) == 2
+
+
 def test_workspace_under_capture_reuses_the_eager_one(monkeypatch):
     """Under HIP graph capture the workspace cache allocates nothing: it hands out the device's largest eager
     workspace of the kind and raises when there is none or it is too small (a buffer allocated inside a capture holds
