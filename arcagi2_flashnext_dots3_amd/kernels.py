@@ -230,26 +230,43 @@ def _workspace(kind, device, nbytes, zero=False):
     return b, key
 
 
+def _has_workspace(kind, device, nbytes):
+    dev = torch.device(device)
+    return any(k == kind and d == dev and b.numel() >= nbytes for (k, d, _), b in _WS.items())
+
+
 def fused_max_tokens(H, cus=256):
     """The most tokens for which auto_split picks the in-kernel split merge (H heads): up to it attend needs a
     workspace."""
     return cus // (2 * ((H + 31) // 32))
 
 
-def reserve_workspace(device, H, T=None, split=8):
+@functools.lru_cache(maxsize=4096)
+def attn_reserve_bytes(H, K=None, cus=256):
+    """Bytes of a workspace that serves every merged launch of H heads over up to K rows (None: any) that auto_split /
+    auto_split576 choose. Lists of up to 2048 rows never take a second round of workgroups: the splits of all tokens are
+    at most one round (128 heads 17 MB); longer ones may."""
+    hg = (H + 31) // 32
+    n = cus // (2 * hg) * hg                                       # workgroups of an unsplit launch, at most
+    wgs = min(8 * n, cus) if K is not None and K <= 2048 else 8 * n
+    return sum((b + 255) // 256 * 256 for b in (4 * n, 128 * wgs)) + 65536 * wgs   # counters, lse, partials
+
+
+def reserve_workspace(device, H, T=None, split=8, K=None):
     """Allocate now (eagerly) the attention workspace that attend's split merge needs for up to T tokens of H heads
-    (default: every size auto_split sends there), so that later HIP graph captures find it. No-op when present."""
-    T = fused_max_tokens(H) if T is None else T
-    if T > 0:
-        _workspace("attn", device, attn_ws_bytes(T, H, split), zero=True)
+    (default: every size auto_split sends there, lists of up to K rows), so that later HIP graph captures share it.
+    No-op when present."""
+    nb = attn_reserve_bytes(H, K) if T is None else attn_ws_bytes(T, H, split) if T > 0 else 0
+    if nb > 0:
+        _workspace("attn", device, nb, zero=True)
 
 
 def _attn_workspace(device, T, H, split, private=False):
     """A workspace for a merged launch with its leading counter bytes zero (queued on the current stream): the cached
-    one, or, with private under graph capture, a temporary of the graph itself, so that graphs may replay beside each
-    other and beside eager calls."""
+    one. Under graph capture the device's largest cached one; with private, or where none is large enough, a temporary
+    of the graph itself, so that graphs may replay beside each other and beside eager calls."""
     nb, cnt = attn_ws_bytes(T, H, split), _attn_counter_bytes(T, H)
-    if private and torch.cuda.is_current_stream_capturing():
+    if torch.cuda.is_current_stream_capturing() and (private or not _has_workspace("attn", device, nb)):
         ws, key = torch.empty(nb, dtype=torch.uint8, device=device), None
     else:
         ws, key = _workspace("attn", device, nb, zero=True)
@@ -739,8 +756,8 @@ def attend(q, pool, idx, sm_scale, kv_scale=1.0, out=None, lse=None, split=None,
     split > 1 (at most 8) cuts K into partials that the kernel merges in a workspace: a cached one per stream, under
     HIP graph capture one of the graph's own. For Row656 (spmla_attn; split None: auto_split) ws may be given, a uint8
     workspace of attn_ws_bytes whose leading counter bytes are zero -- the kernel leaves them so --, and captured
-    launches of fewer than 96 workgroups (token, 32 heads) take either ws or a workspace reserved by an earlier eager
-    call, see reserve_workspace."""
+    launches of fewer than 96 workgroups (token, 32 heads) share the largest workspace of an earlier eager call where it
+    is large enough (see reserve_workspace); graphs that share one are replayed one at a time."""
     T, H, _ = q.shape
     K = idx.shape[1]
     rb = int(row_bytes) if row_bytes is not None else (int(pool.shape[-1]) if torch.is_tensor(pool) else ROW656)

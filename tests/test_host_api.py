@@ -283,6 +283,38 @@ def test_workspace_under_capture_reuses_the_eager_one(monkeypatch):
         kernels._workspace("attn", d0, 5000)
 
 
+def test_attention_workspace_under_capture(monkeypatch):
+    """A captured merged launch takes the workspace of an earlier eager call when that is large enough, else one of the
+    graph's own: the splits of fewer tokens may need more than those of the eager call did."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    H, K = 128, 2048
+    need = [kernels.attn_ws_bytes(T, H, kernels.auto_split(T, H, K)) for T in (12, 8)]
+    assert need[1] > need[0]
+    d = torch.device("cpu")
+    eager = torch.full((need[0],), 7, dtype=torch.uint8)
+    monkeypatch.setattr(kernels, "_WS", {("attn", d, 1): eager})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    ws = kernels._attn_workspace(d, 8, H, kernels.auto_split(8, H, K))
+    assert ws is not eager and ws.numel() >= need[1] and not ws[:kernels._attn_counter_bytes(8, H)].any()
+    assert kernels._attn_workspace(d, 12, H, kernels.auto_split(12, H, K)) is eager
+    assert not eager[:kernels._attn_counter_bytes(12, H)].any()
+
+
+@pytest.mark.parametrize("H", [16, 32, 64, 100, 128, 160])
+def test_reserved_attention_workspace_serves_every_split(H):
+    """attn_reserve_bytes covers what auto_split chooses for every number of tokens, and no more than one round of
+    workgroups (128 heads: 17 MB) for lists of up to 2048 rows."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    for K, Ks in ((2048, (544, 640, 1000, 1024, 1504, 2048)), (None, (4096, 8192, 12000, 16384, 60000))):
+        have = kernels.attn_reserve_bytes(H, K)
+        for T in range(1, kernels.fused_max_tokens(H) + 2):
+            for k in Ks:
+                for f in (kernels.auto_split, kernels.auto_split576):
+                    s = f(T, H, k)
+                    assert s == 1 or kernels.attn_ws_bytes(T, H, s) <= have, (T, k, s)
+    assert kernels.attn_reserve_bytes(H, 2048) < 17.5e6
+
+
 def test_merged_launches_of_two_threads_on_one_stream(monkeypatch):
     """Two host threads share a stream's attention workspace. A launch of few counters uses the bytes behind them as
     scratch: it must not come between the clearing of another's counters and that launch."""
