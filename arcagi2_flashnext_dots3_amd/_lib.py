@@ -98,13 +98,18 @@ def lib():
     return _L
 
 
-def call(name, *args):
-    """Invoke entry point `name`; a nonzero return code raises RuntimeError naming the entry point."""
+def status(name, *args):
+    """Invoke entry point `name` and return its value."""
     f = _FN.get(name) or getattr(lib(), name)
     try:
-        rc = f(*args)
-    except TypeError:            # not ints, floats and None: ctypes takes it or refuses it
-        rc = getattr(lib(), name)(*args)
+        return f(*args)
+    except TypeError:            # not ints, floats and None (numpy integers): ctypes takes it or refuses it
+        return getattr(lib(), name)(*args)
+
+
+def call(name, *args):
+    """Invoke entry point `name`; a nonzero return code raises RuntimeError naming the entry point."""
+    rc = status(name, *args)
     if rc != 0:
         raise RuntimeError(f"{name} failed: {rc} ({ERRORS.get(rc, 'hip error')})")
     return rc

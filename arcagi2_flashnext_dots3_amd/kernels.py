@@ -343,12 +343,11 @@ def logits_hist(q, w, base, R, rpb, bstride, block_table, block_size, req, ctx, 
     min(ctx, Lc) written. Returns False without a launch above 258048 columns; the caller then runs the logits and topk
     separately."""
     rows = q.shape[0]
-    _lib.lib()
-    rc = _lib._FN["spmla_index_logits_hist"](
-        q.data_ptr(), q.stride(0), q.stride(1), w.data_ptr(), w.stride(0), base.data_ptr(), R, rpb, bstride,
-        block_table.data_ptr(), block_table.stride(0), block_size, req.data_ptr(), ctx.data_ptr(), rows, q.shape[1],
-        q.shape[2], Lc, int(bool(noinf)), lg.data_ptr(), lg.stride(0), _LG_DT[lg.dtype], ws.data_ptr(), ws.numel(),
-        K, _stream(q))
+    rc = _lib.status(
+        "spmla_index_logits_hist", q.data_ptr(), q.stride(0), q.stride(1), w.data_ptr(), w.stride(0), base.data_ptr(), R,
+        rpb, bstride, block_table.data_ptr(), block_table.stride(0), block_size, req.data_ptr(), ctx.data_ptr(), rows,
+        q.shape[1], q.shape[2], Lc, int(bool(noinf)), lg.data_ptr(), lg.stride(0), _LG_DT[lg.dtype], ws.data_ptr(),
+        ws.numel(), K, _stream(q))
     if rc == -5:
         return False
     if rc != 0:

@@ -44,6 +44,19 @@ def test_other_argument_types_go_through_ctypes():
         _lib.call("spmla_cache_write", ctypes.c_void_p(256), 0, None, 0, None, -1, None, 0, 1, 0, 0, 1.0, None)
 
 
+def test_logits_hist_takes_numpy_integers(monkeypatch):
+    import numpy as np
+    from arcagi2_flashnext_dots3_amd import kernels
+    monkeypatch.setattr(kernels, "_stream", lambda t: 0)
+    f32, i32, K, Lc, bs = dict(dtype=torch.float32), dict(dtype=torch.int32), *map(np.int64, (16, 1000, 64))
+    args = (torch.zeros(0, 64, 128, dtype=torch.bfloat16), torch.zeros(0, 64, **f32), torch.zeros(64, 132), 64, 64, 8448,
+            torch.zeros(1, 16, **i32), bs, torch.zeros(0, **i32), torch.zeros(0, **i32), Lc, K, torch.zeros(0, 1000, **f32),
+            torch.zeros(64, dtype=torch.uint8))
+    assert kernels.logits_hist(*args)                          # no rows: nothing is launched
+    with pytest.raises(RuntimeError, match="-2"):
+        kernels.logits_hist(*args[:11], np.int64(0), *args[12:])
+
+
 @pytest.mark.gpu
 def test_stream_handle(dev):
     from arcagi2_flashnext_dots3_amd import kernels
