@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "spmla_common.h"
+#include "spmla_rules.h"
 
 namespace spmla {
 namespace attn {
@@ -849,18 +850,9 @@ long long ws_bytes(int T, int H, int S);
 
 extern "C" {
 
-// Whether a launch without the split merge takes fwd_kernel (128 heads per workgroup, one workgroup per compute unit)
-// or the head-group kernel (spmla_attn_hg.hip: 32 heads per workgroup, one per compute unit as well, any K). fwd_kernel
-// pays for whole groups of 128 heads and for whole rounds of 256 workgroups; a round costs as much as 3.1 times 256
-// head-group workgroups at K = 2048, 2.5 times at K <= 512 (their prologue and merge weigh more). Measured (us, head-group
-// / fwd_kernel), Row656, K = 2048: H = 128: T = 192 169 / 163, 224 206 / 163, 256 198 / 169, 400 326 / 306, 640 475 / 459,
-// 900 688 / 616, 2048 1559 / 1304; T = 2048: H = 32 417 / 1140, 64 798 / 1186, 96 1199 / 1242; T = 512, H = 160 477 / 598;
-// T = 700, H = 72 406 / 435. H = 128: T = 300, K = 512 100 / 101, T = 400, K = 1024 199 / 172, T = 256, K = 64 45 / 26.
-// Row576 lies the same way (H = 128, K = 2048: T = 192 134 / 140, 224 166 / 146, 400 288 / 279, 2048 1386 / 1168).
-static bool attn_wide(int T, int H, int K, int S) {
-  const int rows = ((K + S - 1) / S + attn::TR - 1) / attn::TR * attn::TR;     // of a split
-  const long long n32 = (long long)T * S * ((H + 31) / 32), n128 = (long long)T * S * ((H + attn::HGW - 1) / attn::HGW);
-  return rows <= attn::KMAX && 10 * n32 > (rows <= 512 ? 25 : 31) * ((n128 + 255) / 256 * 256);
+static bool attn_wide(int T, int H, int K, int S) {       // fwd_kernel and not the head-group kernel
+  static_assert(attn::KMAX == rules::WIDE_ROWS && attn::HGW == 128 && attn::TR == 32, "what the rule was measured with");
+  return rules::attn_wide(T, H, K, S);
 }
 
 static attn::Params wide_params(const void* q, long long q_st, long long q_sh, const void* pool, long long R,

@@ -1,0 +1,36 @@
+"""The launchers' rules of sizes (csrc/spmla_rules.h), compiled for the host, against measured points on both sides."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from arcagi2_flashnext_dots3_amd import build
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no host compiler")
+    d = tmp_path_factory.mktemp("rules")
+    (d / "r.cpp").write_text('#include "spmla_rules.h"\n'
+                             'extern "C" int wide(int T, int H, int K, int S) { return spmla::rules::attn_wide(T, H, K, S); }\n')
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", build.CSRC, str(d / "r.cpp"), "-o",
+                    str(d / "r.so")], check=True, capture_output=True)
+    return ctypes.CDLL(str(d / "r.so"))
+
+
+@pytest.mark.parametrize("T,H,K,hg,fwd", [                          # us of the head-group kernel and of fwd_kernel
+    (129, 128, 2048, 142, 169), (224, 128, 2048, 195, 172), (300, 128, 2048, 253, 319), (400, 128, 2048, 345, 325),
+    (2048, 128, 2048, 1618, 1406), (1500, 32, 2048, 384, 874), (512, 160, 2048, 523, 645), (129, 128, 1024, 86, 94),
+    (300, 128, 512, 100, 108), (400, 128, 1024, 209, 187),
+    (129, 128, 128, 39, 31), (129, 128, 40, 34, 22), (300, 128, 128, 65, 54), (2000, 64, 128, 233, 184),
+    (512, 64, 32, 45, 34), (512, 160, 256, 160, 144), (1000, 160, 40, 228, 160)])
+def test_attention_kernel_choice(lib, T, H, K, hg, fwd):
+    assert bool(lib.wide(T, H, K, 1)) == (fwd < hg)
+
+
+def test_lists_beyond_the_prefill_kernel(lib):
+    assert lib.wide(4096, 128, 2048, 1) and not lib.wide(4096, 128, 2049, 1) and lib.wide(4096, 128, 4096, 2)
+    assert not lib.wide(0, 128, 2048, 1)
