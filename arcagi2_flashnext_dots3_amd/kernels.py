@@ -710,12 +710,14 @@ ATTN_SPLIT_ROWS = 2048      # most rows of one (token, split), in tiles of 32, t
 
 def _split_cost(n, K, s, cus):
     """Model of a launch of n * s workgroups over K / s rows each (us): rounds of one workgroup per compute unit, each a
-    fixed part and the longest wave's 32-row tiles; the merge of the splits on top. Fitted to graphed launches of 128
-    heads at K = 384 .. 2048 (1 / 2 / 4 / 8 splits; K = 2048, T = 1 42 / 32 / 26 / 24 us, 16 46 / 35 / 29 / 49, 32 47 / 38 / 51 /
-    79; K = 1024, T = 16 29 / 26 / 25 / 44; K = 512, T = 1 18.5 / 19.2 / 18.7 / 20.9, 16 20.4 / 21.1 / 22.2 / 41.5). Up to 512
-    rows the merge costs what the shorter lists save: the launch stays whole and needs no workspace."""
+    fixed part and the longest wave's 32-row tiles; the merge of the splits on top (its kernel is built for 2, 4 and 8).
+    Fitted to graphed launches (1 / 2 / 4 / 8 splits; 128 heads: K = 2048, T = 1 42 / 32 / 26 / 24 us, 16 46 / 35 / 29 / 49, 32
+    47 / 38 / 51 / 79; K = 1024, T = 16 29 / 26 / 25 / 44; K = 512, T = 8 20.0 / 20.6 / 19.7 / 23.7, T = 16 20.4 / 21.1 / 22.2 /
+    41.5; K = 640, T = 8 21.9 / 22.5 / 21.8 / 23.4; 32 heads, K = 512, T = 32 20.4 / 21.1 / 19.5 / 23.0; K = 384 16.2 / 18.5 /
+    17.9 / 20.1 and less for one launch at any T)."""
     tiles = -(-(-(-K // s)) // 32)
-    return -(-n * s // cus) * (12.7 + 2.2 * -(-tiles // 4)) + (4.5 + 1.0 * s if s > 1 else 0.0)
+    merge = 0.0 if s == 1 else (5.7 if s == 2 else 6.2 if s <= 4 else 9.2) + 0.003 * max(0, n * s - 128)
+    return -(-n * s // cus) * (10.4 + 2.15 * -(-tiles // 4)) + merge
 
 
 @functools.lru_cache(maxsize=4096)
