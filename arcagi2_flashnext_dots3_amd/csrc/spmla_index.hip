@@ -23,6 +23,8 @@
 //   remaining levels run on those candidates alone; ties on the final key take the lowest columns. The K winners are
 //   bitonic-sorted in LDS (only the stages whose pairs cross waves take a workgroup barrier); on the several-
 //   workgroup path, whose lists arrive in column order, fp16 winners are ordered by a stable radix sort instead.
+#include <type_traits>
+
 #include "spmla_common.h"
 #include <limits.h>
 #include <algorithm>
@@ -530,20 +532,29 @@ __device__ inline uint32_t wave_incl_scan(uint32_t x) {
   x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);   // row_bcast:31, rows 2, 3
   return x;
 }
-// Minimum / maximum over the wave (uniform result): quad permutations and row mirrors within each 16-lane row,
-// then the four rows' results through readlane.
+// op over the 16 lanes of a row, in every lane of it: quad permutations and row mirrors
+template <class T, class Op>
+__device__ inline T row_reduce(T x, Op op) {
+  auto dpp = [](T y, auto ctrl) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, y), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  x = op(x, dpp(x, std::integral_constant<int, 0xb1>()));      // quad_perm [1, 0, 3, 2]
+  x = op(x, dpp(x, std::integral_constant<int, 0x4e>()));      // quad_perm [2, 3, 0, 1]
+  x = op(x, dpp(x, std::integral_constant<int, 0x141>()));     // row_half_mirror
+  return op(x, dpp(x, std::integral_constant<int, 0x140>()));  // row_mirror
+}
+template <bool MAX>
+__device__ inline uint32_t row_minmax(uint32_t x) {
+  return row_reduce(x, [](uint32_t a, uint32_t b) { return MAX ? (a > b ? a : b) : (a < b ? a : b); });
+}
+__device__ inline uint32_t lane_of(uint32_t x, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)x, l); }
+// Minimum / maximum over the wave (uniform): the four rows' results through readlane
 template <bool MAX>
 __device__ inline uint32_t wave_minmax(uint32_t x) {
-  auto op = [](uint32_t a, uint32_t b) { return MAX ? (a > b ? a : b) : (a < b ? a : b); };
-  x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, false));   // quad_perm [1, 0, 3, 2]
-  x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x4e, 0xf, 0xf, false));   // quad_perm [2, 3, 0, 1]
-  x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xf, 0xf, false));  // row_half_mirror
-  x = op(x, (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x140, 0xf, 0xf, false));  // row_mirror
-  const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)x, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)x, 16);
-  const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)x, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)x, 48);
-  return op(op(a, b), op(c, d));
+  x = row_minmax<MAX>(x);
+  const uint32_t a = lane_of(x, 0), b = lane_of(x, 16), c = lane_of(x, 32), d = lane_of(x, 48);
+  return MAX ? max(max(a, b), max(c, d)) : min(min(a, b), min(c, d));
 }
-
 // block-wide exclusive scan of a per-thread count (1024 threads = 16 waves): wave scans on the VALU, the 16 wave
 // totals through LDS (wsum: 16-byte aligned, 16 words); every thread sums the totals of the waves before its own
 __device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t* wsum, uint32_t* total) {
@@ -1124,9 +1135,10 @@ __global__ void __launch_bounds__(TK_NT) topk_kernel(TopkParams p) {
 // indexer logits (a few entries each at the K-th key, where the 11-bit radix digits of the key put a fifth of the row
 // into one bin), so there is no second level and no sort of the winners. A row is a chain of barriers, LDS atomics and
 // one read of the row; in graphs, against a radix level over several workgroups, a second on its bin and a finishing
-// sort: 4 rows of 16000 columns 9.6 us (32.7), 64 of 32768 15.0 us (39.0), 2048 of 16384 55.6 us (356).
-// A row whose bins from the K-th key's on hold more than BK_LIM entries somewhere (heavy ties, far outliers, no finite
-// value) goes through a radix select over (key, column) instead.
+// sort: 4 rows of 16000 columns 9.8 us (32.7), 64 of 32768 15.3 us (39.0), 2048 of 16384 55.6 us (356).
+// Values that crowd at the low end of their range (far outliers, skewed distributions) are binned by the key's integer
+// instead, which spaces bins by magnitude. A row whose bins from the K-th key's on still hold more than
+// BK_LIM entries somewhere (heavy ties, outliers below, no finite value) has the K-th key's bin cut further (bk_refine).
 constexpr int BK_BINS = 4096;
 constexpr int BK_LIM = 256;                  // entries of a bin that are ranked by counting
 constexpr int BK_LIST = TK_KMAX + BK_LIM;    // entries from the K-th key's bin on
@@ -1137,19 +1149,26 @@ struct BkLds {
   __attribute__((aligned(16))) uint32_t off[BK_BINS];   // counts, then first slots, then ends
   unsigned long long list[BK_LIST];
   __attribute__((aligned(16))) uint32_t wsum[16];
-  __attribute__((aligned(16))) uint32_t red[32];        // per wave: smallest, largest finite key
+  __attribute__((aligned(16))) uint32_t red[48];        // per wave: smallest, largest finite key, smallest of its threads' largest
   uint32_t sh[8];
 };
 
 __device__ inline float unkey(uint32_t k) { return u2f((k & 0x80000000u) ? k & 0x7fffffffu : ~k); }   // okey's inverse
-__device__ inline int bk_bin(float v, float vmin, float scale) {
-  const float t = fminf(fmaxf((v - vmin) * scale, 0.f), (float)(BK_BINS - 1));   // -inf: 0; +inf: the last bin
-  return v != v ? BK_BINS - 1 : (int)t;                                            // NaN is the largest key
+// vmin, scale: bins of the value; kmin, sh (by_key): of the key. bin of the K-th key (-1: none), entries from it on, in it
+struct BkRange { float vmin, scale; uint32_t kmin; int sh; bool by_key; int bin; uint32_t n, c; };
+template <bool KEY>
+__device__ inline int bk_bin(float v, const BkRange& r) {
+  if constexpr (KEY) {
+    const uint32_t k = okey(v);
+    return k < r.kmin ? 0 : (int)min((k - r.kmin) >> r.sh, (uint32_t)(BK_BINS - 1));
+  }
+  const float t = fminf(fmaxf((v - r.vmin) * r.scale, 0.f), (float)(BK_BINS - 1));   // -inf: 0; +inf: the last bin
+  return v != v ? BK_BINS - 1 : (int)t;                                                // NaN is the largest key
 }
-struct BkRange { float vmin, scale; int bin; uint32_t n; };   // bin of the K-th key, entries from it on
+__device__ inline int bk_bin(float v, const BkRange& r) { return r.by_key ? bk_bin<true>(v, r) : bk_bin<false>(v, r); }
 
 // Bins of the keys v (bit i of vm: v[i] is one), K of them wanted (0 < K <= their number): L.off = every bin's first slot.
-// False (uniform) when the radix select has to do it.
+// False (uniform) when bk_refine has to do it.
 template <int EPT>
 __device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uint32_t K, BkRange& r) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -1161,23 +1180,29 @@ __device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uin
     mx = fin ? fmaxf(mx, v[i]) : mx;
   }
   const uint32_t kn = wave_minmax<false>(okey(mn)), kx = wave_minmax<true>(okey(mx));
-  if (lane == 0) { L.red[wv] = kn; L.red[16 + wv] = kx; }
+  const uint32_t kq = wave_minmax<false>(okey(mx));
+  if (lane == 0) { L.red[wv] = kn; L.red[16 + wv] = kx; L.red[32 + wv] = kq; }
   ((u32x4*)L.off)[tid] = u32x4{0u, 0u, 0u, 0u};
   if (tid < 8) L.sh[tid] = 0u;
   __syncthreads();
-  uint32_t an = 0xffffffffu, ax = 0u;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const u32x4 a = ((const u32x4*)L.red)[q], b = ((const u32x4*)L.red)[4 + q];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { an = min(an, a[e]); ax = max(ax, b[e]); }
-  }
+  const uint32_t x = L.red[min(lane, 47)];                // a 16-lane row each of minima, maxima and smallest thread maxima
+  const uint32_t xx = row_minmax<true>(x), an = lane_of(row_minmax<false>(x), 0), ax = lane_of(xx, 16);
+  const float q = unkey(lane_of(xx, 32));                 // (of a wave's 64 threads with EPT values each: a high quantile)
+  r.bin = -1;
   r.vmin = unkey(an);
-  r.scale = ((float)BK_BINS - 0.01f) / (unkey(ax) - r.vmin);
+  r.kmin = an;
+  const float span = unkey(ax) - r.vmin;
+  r.scale = ((float)BK_BINS - 0.01f) / span;
   if (!(r.scale > 0.f && r.scale < __builtin_inff())) return false;   // no finite value, one value, or an overflow
+  r.sh = max(0, 20 - (int)__builtin_clz((ax - an) | 1u));             // (ax - an) >> sh < 4096
+  // by key when the high values lie that low in the range: bins of equal width would hold hundreds of them each
+  r.by_key = q >= r.vmin && (q - r.vmin) * 2048.f < (float)EPT * span;
+  auto count = [&](auto key) {
 #pragma unroll
-  for (int i = 0; i < EPT; ++i)
-    if ((vm >> i) & 1u) atomicAdd(&L.off[bk_bin(v[i], r.vmin, r.scale)], 1u);
+    for (int i = 0; i < EPT; ++i)
+      if ((vm >> i) & 1u) atomicAdd(&L.off[bk_bin<decltype(key)::value>(v[i], r)], 1u);
+  };
+  if (r.by_key) count(std::true_type()); else count(std::false_type());
   __syncthreads();
   u32x4* own = (u32x4*)L.off + (TK_NT - 1 - tid);      // bins 4095 - 4 t (element 3) down to 4092 - 4 t
   u32x4 h = *own;
@@ -1188,7 +1213,7 @@ __device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uin
   for (int e = 3; e >= 0; --e) {
     const uint32_t c = h[e];
     if (run < K) big = max(big, c);
-    if (run < K && run + c >= K) { L.sh[1] = (uint32_t)(BK_BINS - 4 - 4 * tid + e); L.sh[2] = run + c; }
+    if (run < K && run + c >= K) { L.sh[1] = (uint32_t)(BK_BINS - 4 - 4 * tid + e); L.sh[2] = run + c; L.sh[3] = c; }
     h[e] = run;
     run += c;
   }
@@ -1198,49 +1223,148 @@ __device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uin
   __syncthreads();
   r.bin = (int)L.sh[1];
   r.n = L.sh[2];
+  r.c = L.sh[3];
   return L.sh[0] <= (uint32_t)BK_LIM;
 }
 
-// The K best of the entries src.ent(j), j < n ((key, ~column) packed, 0: none), into L.list in no order: radix select
-// over the 64 bits (all entries differ), then an append.
-template <class Src>
-__device__ inline void bk_radix(BkLds& L, const Src& src, int n, uint32_t K) {
-  const int tid = threadIdx.x;
-  unsigned long long prefix = 0, mask = 0;
-  uint32_t need = K;
-  for (int level = 0; level < 6; ++level) {
-    const int shift = level == 0 ? 53 : level == 1 ? 42 : level == 2 ? 32 : level == 3 ? 21 : level == 4 ? 10 : 0;
-    const unsigned long long dm = level == 2 || level == 5 ? 0x3ffu : 0x7ffu;
+// Entries in registers: (key, ~column) of entry i as key(i), low(i), its value val(i). fence: what follows is computed from the registers
+// again (the compiler would keep keys and columns of all entries beside them, and spill).
+template <int EPT>
+struct RowRegs {                                           // columns c + 4096 (i / 4) + i % 4 of a row
+  float (&v)[EPT];
+  int c;
+  __device__ float val(int i) const { return v[i]; }
+  __device__ uint32_t key(int i) const { return okey(v[i]); }
+  __device__ uint32_t low(int i) const { return ~(uint32_t)(c + 4 * TK_NT * (i >> 2) + (i & 3)); }
+  __device__ void fence() {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) asm volatile("" : "+v"(v[i]));
+    asm volatile("" : "+v"(c));
+  }
+};
+template <int EPT>
+struct ListRegs {
+  unsigned long long (&e)[EPT];
+  __device__ float val(int i) const { return unkey(key(i)); }
+  __device__ uint32_t key(int i) const { return (uint32_t)(e[i] >> 32); }
+  __device__ uint32_t low(int i) const { return (uint32_t)e[i]; }
+  __device__ void fence() {
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) asm volatile("" : "+v"(e[i]));
+  }
+};
+
+// The K best of the n entries ent (bit i of vm: entry i is one; all different) into L.list in no order, after bk_bins gave
+// up: the bin of the K-th key (r.bin; -1: all) is cut by its keys' range into 4096 bins of a power of two, then that bin
+// again, then, between equal keys, by column (lo .. hi: the range of ~column), until the bin is taken whole or its entries
+// can be ranked by counting. A chain of barriers and of same-bin atomics of the equal values. us, several workgroups' radix
+// passes / a radix select over (key, column) that re-read the row / bins by key or this: 64 rows of 32768: one far outlier
+// 35 / 67 / 23, lognormal 30 / 68 / 17, 25 distinct values 39 / 85 / 45, 1 % of the values not zero 107 / 196 / 59, one
+// value 107 / 161 / 26; 64 of 131072: 50 / 90 / 38, 47 / 96 / 47, 59 / 124 / 63, 477 / 254 / 84, 478 / 214 / 45.
+template <int EPT, class Ent>
+__device__ inline void bk_refine(BkLds& L, Ent ent, uint32_t vm, uint32_t n, const BkRange& r, uint32_t K, uint32_t lo,
+                                 uint32_t hi) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  uint32_t sm = 0u, cm = vm, above = 0u, c = n;            // selected entries, candidates; their numbers
+  auto fence = [&]() { ent.fence(); asm volatile("" : "+v"(sm), "+v"(cm)); };
+  auto above_bin = [&](auto key) {
+    fence();
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const int b = bk_bin<decltype(key)::value>(ent.val(i), r);
+      const uint32_t bit = cm & (1u << i);
+      sm |= b > r.bin ? bit : 0u;
+      cm &= b != r.bin ? ~bit : ~0u;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (r.bin >= 0) {
+    above = r.n - r.c;
+    c = r.c;
+    if (r.by_key) above_bin(std::true_type()); else above_bin(std::false_type());
+  }
+  bool col = false;
+  uint32_t rl = 0u, rw = 0u;                               // the candidates' keys (or ~columns): rl .. rl + rw
+  // a cut leaves 12 bits less of the range: at most 3 by key and 2 by column, after which one entry is left
+#pragma unroll 1
+  for (int cut = 0; cut < 5 && c > (uint32_t)BK_LIM && above + c != K; ++cut) {       // uniform
+    __syncthreads();                                       // L.red, L.sh are read
+    if (!col) {
+      uint32_t mn = 0xffffffffu, mx = 0u;
+      fence();
+#pragma unroll
+      for (int i = 0; i < EPT; ++i) {
+        const uint32_t k = ent.key(i);
+        mn = min(mn, (cm >> i) & 1u ? k : 0xffffffffu);
+        mx = max(mx, (cm >> i) & 1u ? k : 0u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      mn = wave_minmax<false>(mn);
+      mx = wave_minmax<true>(mx);
+      if (lane == 0) { L.red[wv] = mn; L.red[16 + wv] = mx; }
+      __syncthreads();
+      rl = wave_minmax<false>(L.red[lane & 15]);
+      rw = wave_minmax<true>(L.red[16 + (lane & 15)]) - rl;
+      if (rw == 0u) { col = true; rl = lo; rw = hi - lo; }
+    }
+    const int s = max(0, 20 - (int)__builtin_clz(rw | 1u));            // rw >> s < 4096
+    auto digit = [&](int i) -> uint32_t { return ((col ? ent.low(i) : ent.key(i)) - rl) >> s; };
+    ((u32x4*)L.off)[tid] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
-    L.off[tid] = 0u;
-    L.off[tid + TK_NT] = 0u;
+    fence();
+#pragma unroll
+    for (int i = 0; i < EPT; ++i)
+      if ((cm >> i) & 1u) atomicAdd(&L.off[digit(i)], 1u);
     __syncthreads();
-    for (int j = tid; j < n; j += TK_NT) {
-      const unsigned long long e = src.ent(j);
-      if (e && (e & mask) == prefix) atomicAdd(&L.off[(e >> shift) & dm], 1u);
+    const u32x4 h = ((u32x4*)L.off)[TK_NT - 1 - tid];      // bins 4095 - 4 t (element 3) down to 4092 - 4 t
+    uint32_t tot;
+    uint32_t run = above + block_excl_scan(h[0] + h[1] + h[2] + h[3], L.wsum, &tot);
+#pragma unroll
+    for (int e = 3; e >= 0; --e) {
+      if (run < K && run + h[e] >= K) { L.sh[1] = (uint32_t)(BK_BINS - 4 - 4 * tid + e); L.sh[2] = run; L.sh[3] = h[e]; }
+      run += h[e];
     }
     __syncthreads();
-    const int b0 = 2047 - 2 * tid;
-    const uint32_t h0 = L.off[b0], h1 = L.off[b0 - 1];
-    uint32_t tot;
-    const uint32_t before = block_excl_scan(h0 + h1, L.wsum, &tot);
-    if (before < need && before + h0 >= need) { L.sh[1] = (uint32_t)b0; L.sh[2] = before; L.sh[3] = h0; }
-    if (before + h0 < need && before + h0 + h1 >= need) { L.sh[1] = (uint32_t)b0 - 1; L.sh[2] = before + h0; L.sh[3] = h1; }
-    __syncthreads();
-    prefix |= (unsigned long long)L.sh[1] << shift;
-    mask |= dm << shift;
-    need -= L.sh[2];
-    if (L.sh[3] == need) break;                        // uniform: the bin is taken whole
+    const uint32_t b = L.sh[1];
+    above = L.sh[2];
+    c = L.sh[3];
+    fence();
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const uint32_t d = digit(i), bit = cm & (1u << i);
+      sm |= d > b ? bit : 0u;
+      cm &= d != b ? ~bit : ~0u;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    rl += b << s;
+    rw = min(rw - (b << s), (1u << s) - 1u);
+  }
+  // the selected, and the candidates (at most BK_LIM, unless they are all taken)
+  const bool whole = above + c == K;
+  if (whole) { sm |= cm; cm = 0u; }
+  unsigned long long* cand = (unsigned long long*)L.off;
+  __syncthreads();                                         // L.off is read
+  uint32_t tot;
+  const uint32_t at = block_excl_scan((uint32_t)__popc(sm) | ((uint32_t)__popc(cm) << 16), L.wsum, &tot);
+  uint32_t so = at & 0xffffu, co = at >> 16;
+  fence();
+#pragma unroll
+  for (int i = 0; i < EPT; ++i) {
+    const unsigned long long e = ((unsigned long long)ent.key(i) << 32) | ent.low(i);
+    if ((sm >> i) & 1u) { if (so < (uint32_t)BK_LIST) L.list[so] = e; ++so; }
+    if ((cm >> i) & 1u) { if (co < (uint32_t)BK_LIM) cand[co] = e; ++co; }
+    __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
-  if (tid == 0) L.sh[4] = 0u;
-  __syncthreads();
-  for (int j = tid; j < n; j += TK_NT) {
-    const unsigned long long e = src.ent(j);
-    if (e && (e & mask) >= prefix) {
-      const uint32_t s = atomicAdd(&L.sh[4], 1u);
-      if (s < (uint32_t)BK_LIST) L.list[s] = e;
-    }
+  if (!whole) {                                            // four lanes rank a candidate
+    const uint32_t i = (uint32_t)tid >> 2, nc = min(c, (uint32_t)BK_LIM);
+    const unsigned long long e = i < nc ? cand[i] : 0ull;
+    uint32_t rank = 0u;
+#pragma unroll 4
+    for (uint32_t j = (uint32_t)tid & 3u; j < nc; j += 4u) rank += (uint32_t)(cand[j] > e);
+    rank += (uint32_t)__builtin_amdgcn_mov_dpp((int)rank, 0xb1, 0xf, 0xf, false);
+    rank += (uint32_t)__builtin_amdgcn_mov_dpp((int)rank, 0x4e, 0xf, 0xf, false);
+    if ((tid & 3) == 0 && i < nc && rank < K - above) L.list[above + rank] = e;
   }
   __syncthreads();
 }
@@ -1292,26 +1416,18 @@ __device__ inline uint32_t bk_load(const void* row, int c0, int c1, float (&v)[E
     for (int i = 0; i < EPT; ++i) v[i] = one(4 * (tid + TK_NT * (i >> 2)) + (i & 3));
   }
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) vm |= (uint32_t)(4 * (tid + TK_NT * (i >> 2)) + (i & 3) < n) << i;
+  for (int i = 0; i < EPT; ++i) {
+    vm |= (uint32_t)(4 * (tid + TK_NT * (i >> 2)) + (i & 3) < n) << i;
+    if constexpr (F16) asm volatile("" : "+v"(v[i]));     // (the fp16 values would be kept beside them)
+  }
   return vm;
 }
-
-template <bool F16>
-struct RowEnts {     // columns c0 .. of a logits row as (key, ~column)
-  const void* x; int c0;
-  __device__ unsigned long long ent(int j) const {
-    float v;
-    if constexpr (F16) v = (float)((const _Float16*)x)[c0 + j];
-    else v = ((const float*)x)[c0 + j];
-    return tk_pack(okey(v), c0 + j);
-  }
-};
 
 // The entries of L.list from the K-th key's bin on, in final order, to o[0, K) (column, -1 for +-inf), and -1 to kout.
 __device__ inline void bk_emit(BkLds& L, const BkRange& r, uint32_t K, int kout, int* o) {
   for (uint32_t i = threadIdx.x; i < r.n; i += TK_NT) {
     const unsigned long long e = L.list[i];
-    const int b = bk_bin(unkey((uint32_t)(e >> 32)), r.vmin, r.scale);
+    const int b = bk_bin(unkey((uint32_t)(e >> 32)), r);
     const uint32_t end = L.off[b];                        // the appends moved a bin's first slot to its end
     uint32_t at = b + 1 < BK_BINS ? L.off[b + 1] : 0u, first = at;
     for (uint32_t j = first; j < end; ++j) at += (uint32_t)(L.list[j] > e);
@@ -1319,7 +1435,7 @@ __device__ inline void bk_emit(BkLds& L, const BkRange& r, uint32_t K, int kout,
   }
   for (int s = (int)K + (int)threadIdx.x; s < kout; s += TK_NT) o[s] = -1;
 }
-__device__ inline void bk_emit_sorted(BkLds& L, uint32_t K, int kout, int* o) {   // after bk_radix
+__device__ inline void bk_emit_sorted(BkLds& L, uint32_t K, int kout, int* o) {   // after bk_refine
   tk_sort_desc(L.list, (int)K);
   for (int s = threadIdx.x; s < kout; s += TK_NT) {
     int c = -1;
@@ -1349,15 +1465,18 @@ __global__ void __launch_bounds__(TK_NT, EPT <= 16 ? 8 : 4) topk_row_kernel(Topk
   const uint32_t vm = bk_load<F16, EPT>(x, 0, n, v);
   BkRange r;
   if (!bk_bins<EPT>(L, v, vm, K, r)) {
-    bk_radix(L, RowEnts<F16>{x, 0}, n, K);
+    bk_refine<EPT>(L, RowRegs<EPT>{v, 4 * tid}, vm, (uint32_t)n, r, K, ~(uint32_t)(n - 1), ~0u);
     bk_emit_sorted(L, K, p.K, o);
     return;
   }
+  auto append = [&](auto key) {
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    const int b = bk_bin(v[i], r.vmin, r.scale);
-    if (((vm >> i) & 1u) && b >= r.bin) L.list[atomicAdd(&L.off[b], 1u)] = tk_pack(okey(v[i]), 4 * (tid + TK_NT * (i >> 2)) + (i & 3));
-  }
+    for (int i = 0; i < EPT; ++i) {
+      const int b = bk_bin<decltype(key)::value>(v[i], r);
+      if (((vm >> i) & 1u) && b >= r.bin) L.list[atomicAdd(&L.off[b], 1u)] = tk_pack(okey(v[i]), 4 * (tid + TK_NT * (i >> 2)) + (i & 3));
+    }
+  };
+  if (r.by_key) append(std::true_type()); else append(std::false_type());
   __syncthreads();
   bk_emit(L, r, K, p.K, o);
 }
@@ -1397,26 +1516,21 @@ __global__ void __launch_bounds__(TK_NT) topk_chunk_kernel(TopkChunkParams p) {
   const uint32_t vm = bk_load<F16, EPT>(x, c0, c1, v);
   BkRange r;
   if (!bk_bins<EPT>(L, v, vm, K, r)) {
-    bk_radix(L, RowEnts<F16>{x, c0}, c1 - c0, K);
+    bk_refine<EPT>(L, RowRegs<EPT>{v, c0 + 4 * tid}, vm, (uint32_t)(c1 - c0), r, K, ~(uint32_t)(c1 - 1), ~(uint32_t)c0);
     for (uint32_t i = tid; i < K; i += TK_NT) list[i] = L.list[i];
     if (tid == 0) ((uint32_t*)wr)[g] = K;
     return;
   }
+  auto append = [&](auto key) {
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    const int b = bk_bin(v[i], r.vmin, r.scale);
-    if (((vm >> i) & 1u) && b >= r.bin) list[atomicAdd(&L.off[b], 1u)] = tk_pack(okey(v[i]), c0 + 4 * (tid + TK_NT * (i >> 2)) + (i & 3));
-  }
+    for (int i = 0; i < EPT; ++i) {
+      const int b = bk_bin<decltype(key)::value>(v[i], r);
+      if (((vm >> i) & 1u) && b >= r.bin) list[atomicAdd(&L.off[b], 1u)] = tk_pack(okey(v[i]), c0 + 4 * (tid + TK_NT * (i >> 2)) + (i & 3));
+    }
+  };
+  if (r.by_key) append(std::true_type()); else append(std::false_type());
   if (tid == 0) ((uint32_t*)wr)[g] = r.n;
 }
-
-struct ListEnts {     // the lists of a row one after another, BK_LIST places each (0: no entry)
-  const uint8_t* wr;
-  __device__ unsigned long long ent(int j) const {
-    const int g = j / BK_LIST;
-    return (uint32_t)(j - g * BK_LIST) < ((const uint32_t*)wr)[g] ? ((const unsigned long long*)(wr + BkWs::LISTS))[j] : 0ull;
-  }
-};
 
 template <int G>                                          // lists per row, rounded up
 __global__ void __launch_bounds__(TK_NT) topk_lists_kernel(TopkChunkParams p) {
@@ -1431,16 +1545,16 @@ __global__ void __launch_bounds__(TK_NT) topk_lists_kernel(TopkChunkParams p) {
     for (int s = tid; s < p.K; s += TK_NT) o[s] = -1;
     return;
   }
-  const ListEnts src{p.ws + (long long)row * p.row_bytes};
-  const int m = p.G * BK_LIST;
+  const uint8_t* wr = p.ws + (long long)row * p.row_bytes;
+  const int m = p.G * BK_LIST;                            // places of the row's lists one after another
   unsigned long long e[EPT];
   float v[EPT];
   uint32_t vm = 0, cnt[EPT];
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {                         // every place is read, the unused ones dropped
     const int j = min(tid + TK_NT * i, m - 1);
-    e[i] = ((const unsigned long long*)(src.wr + BkWs::LISTS))[j];
-    cnt[i] = ((const uint32_t*)src.wr)[j / BK_LIST];
+    e[i] = ((const unsigned long long*)(wr + BkWs::LISTS))[j];
+    cnt[i] = ((const uint32_t*)wr)[j / BK_LIST];
   }
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
@@ -1454,15 +1568,20 @@ __global__ void __launch_bounds__(TK_NT) topk_lists_kernel(TopkChunkParams p) {
   }
   BkRange r;
   if (!bk_bins<EPT>(L, v, vm, K, r)) {
-    bk_radix(L, src, m, K);
+    uint32_t have = 0u;
+    for (int g = 0; g < p.G; ++g) have += ((const uint32_t*)wr)[g];
+    bk_refine<EPT>(L, ListRegs<EPT>{e}, vm, have, r, K, ~(uint32_t)(n - 1), ~0u);
     bk_emit_sorted(L, K, p.K, o);
     return;
   }
+  auto append = [&](auto key) {
 #pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    const int b = bk_bin(v[i], r.vmin, r.scale);
-    if (((vm >> i) & 1u) && b >= r.bin) L.list[atomicAdd(&L.off[b], 1u)] = e[i];
-  }
+    for (int i = 0; i < EPT; ++i) {
+      const int b = bk_bin<decltype(key)::value>(v[i], r);
+      if (((vm >> i) & 1u) && b >= r.bin) L.list[atomicAdd(&L.off[b], 1u)] = e[i];
+    }
+  };
+  if (r.by_key) append(std::true_type()); else append(std::false_type());
   __syncthreads();
   bk_emit(L, r, K, p.K, o);
 }

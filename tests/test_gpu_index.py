@@ -419,3 +419,34 @@ def test_topk_bucket_selection(dev, L, dtype):
         wide = torch.full((lg.shape[0], L + 5), 9.0, dtype=dtype, device=dev)      # rows at odd strides and offsets
         wide[:, 3:3 + L] = torch.from_numpy(lg).to(dev)
         assert np.array_equal(kernels.topk(wide[:, 3:3 + L], dctx, K).cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("L", [300, 2500, 9000, 16001, 32768, 40000, 131072, 200001, 262144])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_topk_skewed_and_tied_rows(dev, L, dtype):
+    """Rows whose values crowd at an end of their range (bins by key), or in few values (the K-th key's bin cut by key range
+    and by column): bit-exact against the oracle, at the edges of the keys per thread and of the chunks."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    g = np.random.RandomState(L)
+    x = (280 + 56 * g.randn(12, L)).astype(np.float32)
+    x[0, L // 3] = 5e4                                           # one far above, one far below, both, several
+    x[1, L // 3] = -5e4
+    x[2, L // 5], x[2, L // 7] = 5e4, -5e4
+    x[3, g.permutation(L)[: min(L, 40)]] = 3e4
+    x[4] = np.exp(2.4 * g.randn(L))
+    x[5] = -np.exp(2.4 * g.randn(L))
+    x[6] = np.round(x[6] / 16) * 16
+    x[7] = np.where(g.rand(L) < 0.99, 0, x[7])
+    x[8] = np.where(g.rand(L) < 0.9, -np.inf, x[8])
+    x[9] = np.where(g.rand(L) < 0.3, np.nan, np.where(g.rand(L) < 0.3, np.inf, 7))
+    x[10] = np.where(g.rand(L) < 0.5, -0.0, 0.0)
+    x[11] = np.where(np.arange(L) % 3 == 0, 2 ** -20, 2 ** -21) * (1 if L % 2 else -1)
+    lg = torch.from_numpy(x).to(dtype)
+    ctx = np.full(12, L, dtype=np.int32)
+    dlg, dctx = lg.to(dev), torch.from_numpy(ctx).to(dev)
+    for K in (1, 257, 2048):
+        print(f"[skewed] L={L} K={K} {dtype}", flush=True)
+        exp = ref.topk(lg.numpy(), ctx, K)
+        for single in (False, True):
+            got = kernels.topk(dlg, dctx, K, single_pass=single).cpu().numpy()
+            assert np.array_equal(got, exp), f"rows {np.where((got != exp).any(1))[0]} (single_pass={single})"
