@@ -44,6 +44,29 @@ __device__ inline uint32_t okey16(uint32_t h) {
   return ((h & 0x8000u) ? (~h & 0xffffu) : (h | 0x8000u)) << 16;
 }
 
+// op over the 16 lanes of a row, in every lane of it: quad permutations and row mirrors
+template <class T, class Op>
+__device__ inline T row_reduce(T x, Op op) {
+  auto dpp = [](T y, auto ctrl) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, y), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  x = op(x, dpp(x, std::integral_constant<int, 0xb1>()));      // quad_perm [1, 0, 3, 2]
+  x = op(x, dpp(x, std::integral_constant<int, 0x4e>()));      // quad_perm [2, 3, 0, 1]
+  x = op(x, dpp(x, std::integral_constant<int, 0x141>()));     // row_half_mirror
+  return op(x, dpp(x, std::integral_constant<int, 0x140>()));  // row_mirror
+}
+template <bool MAX>
+__device__ inline uint32_t row_minmax(uint32_t x) {
+  return row_reduce(x, [](uint32_t a, uint32_t b) { return MAX ? (a > b ? a : b) : (a < b ? a : b); });
+}
+__device__ inline uint32_t lane_of(uint32_t x, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)x, l); }
+// Minimum / maximum over the wave (uniform): the four rows' results through readlane
+template <bool MAX>
+__device__ inline uint32_t wave_minmax(uint32_t x) {
+  x = row_minmax<MAX>(x);
+  const uint32_t a = lane_of(x, 0), b = lane_of(x, 16), c = lane_of(x, 32), d = lane_of(x, 48);
+  return MAX ? max(max(a, b), max(c, d)) : min(min(a, b), min(c, d));
+}
 // ------------------------------------------------------------------------------------------------ logits
 constexpr int LG_NWV = 8;                 // waves per logits workgroup (2 per SIMD: 256 registers each)
 constexpr int LG_TPW = 16;                // 32-key tiles per wave and workgroup when the rows overfill the device
@@ -315,7 +338,9 @@ __global__ void __launch_bounds__(LG_NWV * 64) logits_kernel(LogitParams p) {
 // LDS ring by LDS DMA, every wave reads them as the A operand (chunk c of head h at c ^ (h & 7): no bank conflicts) and
 // does 32 MFMAs a row, two head blocks by two key blocks; the ReLU and weighting of one product run under the
 // MFMAs of the next. Same products and sums in the same order as above. Rows whose range misses the 512 keys are only
-// filled. Bound by the matrix cores (32 x 32 cycles a row and wave) and, at 60%, the LDS reads; measured: 2048 rows of 16384
+// filled; where the ranges of a workgroup's rows (a few requests' keys among many) leave tiles out, the workgroups of those
+// take part of the rows of the others (256 rows that each see an eighth of 16384 keys: 48 -> 16 us, row at a time 21).
+// Bound by the matrix cores (32 x 32 cycles a row and wave) and, at 60%, the LDS reads; measured: 2048 rows of 16384
 // keys (15360 valid on average) 417 us.
 constexpr int FL_NWV = 8, FL_KEYS = 64 * FL_NWV;   // waves, keys of a workgroup
 constexpr int FL_RING = 3;
@@ -338,14 +363,14 @@ __global__ void __launch_bounds__(FL_NWV * 64, 2) flat_logits_kernel(FlatParams 
   if (f < 0) return;
   const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int m0 = f / ntile * p.rw, n0 = f % ntile * FL_KEYS;
-  const int key = n0 + 64 * wv + lane;                      // this lane's output column
+  const int m0 = f / ntile * p.rw, own = f % ntile;
+  int n0 = own * FL_KEYS, key = n0 + 64 * wv + lane;        // this lane's output column
   // rows of the chunk: lane r holds row m0 + r's range
   const int mr = m0 + lane;
   const bool rok = lane < p.rw && mr < p.M;
   const int lo_l = rok ? p.lo[mr] : 0, hi_l = rok ? p.hi[mr] : 0;
-  const bool act = rok && max(lo_l, n0) < min(hi_l, min(n0 + FL_KEYS, p.N));
-  uint64_t todo = __ballot(act), fill = __ballot(rok && !act);
+  auto meets = [&]() -> bool { return rok && max(lo_l, n0) < min(hi_l, min(n0 + FL_KEYS, p.N)); };
+  uint64_t fill = __ballot(rok && !meets());
   auto put = [&](int r, float v) {                          // column `key` of row m0 + r (beyond N, r < 0: dropped)
     const uint64_t a = (uint64_t)(uintptr_t)(p.out + (long long)(m0 + max(r, 0)) * p.out_st);
     const uint32_t alo = __builtin_amdgcn_readfirstlane((uint32_t)a), ahi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
@@ -354,7 +379,23 @@ __global__ void __launch_bounds__(FL_NWV * 64, 2) flat_logits_kernel(FlatParams 
     __builtin_amdgcn_raw_buffer_store_b32(f2u(v), rs, 4 * key, 0, 0);
   };
   for (; fill; fill &= fill - 1) put(__builtin_ctzll(fill), -__builtin_inff());
-  if (!todo) return;                                        // uniform over the workgroup
+  // The chunk's ranges lie in tiles t0 .. t1: its ntile workgroups share them, n / tiles on one, part of the rows each
+  const int lc = max(lo_l, 0), hc = min(hi_l, p.N);
+  const bool some = rok && lc < hc;
+  const int t0 = (int)wave_minmax<false>(some ? (uint32_t)lc / FL_KEYS : 0x7fffffffu);
+  const int nt = (int)wave_minmax<true>(some ? (uint32_t)(hc - 1) / FL_KEYS + 1u : 0u) - t0;
+  if (nt <= 0) return;                                      // uniform over the workgroup, as the returns below
+  int r0 = 0, r1 = 64;                                      // this workgroup's part of the rows
+  if (nt < ntile) {
+    const int nsub = ntile / nt, sub = own / nt, per = (p.rw + nsub - 1) / nsub;
+    if (sub >= nsub) return;
+    n0 = (t0 + own - sub * nt) * FL_KEYS;
+    key = n0 + 64 * wv + lane;
+    r0 = sub * per;
+    r1 = r0 + per;
+  }
+  uint64_t todo = __ballot(meets() && lane >= r0 && lane < r1);
+  if (!todo) return;
 
   // copies of query row m0 + r into ring slot s: 64 heads, 2 KiB a wave, then 8 weights a wave (3 instructions)
   auto issue = [&](int r, int s) {
@@ -531,29 +572,6 @@ __device__ inline uint32_t wave_incl_scan(uint32_t x) {
   x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);   // row_bcast:15, rows 1, 3
   x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);   // row_bcast:31, rows 2, 3
   return x;
-}
-// op over the 16 lanes of a row, in every lane of it: quad permutations and row mirrors
-template <class T, class Op>
-__device__ inline T row_reduce(T x, Op op) {
-  auto dpp = [](T y, auto ctrl) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, y), decltype(ctrl)::value, 0xf, 0xf, false));
-  };
-  x = op(x, dpp(x, std::integral_constant<int, 0xb1>()));      // quad_perm [1, 0, 3, 2]
-  x = op(x, dpp(x, std::integral_constant<int, 0x4e>()));      // quad_perm [2, 3, 0, 1]
-  x = op(x, dpp(x, std::integral_constant<int, 0x141>()));     // row_half_mirror
-  return op(x, dpp(x, std::integral_constant<int, 0x140>()));  // row_mirror
-}
-template <bool MAX>
-__device__ inline uint32_t row_minmax(uint32_t x) {
-  return row_reduce(x, [](uint32_t a, uint32_t b) { return MAX ? (a > b ? a : b) : (a < b ? a : b); });
-}
-__device__ inline uint32_t lane_of(uint32_t x, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)x, l); }
-// Minimum / maximum over the wave (uniform): the four rows' results through readlane
-template <bool MAX>
-__device__ inline uint32_t wave_minmax(uint32_t x) {
-  x = row_minmax<MAX>(x);
-  const uint32_t a = lane_of(x, 0), b = lane_of(x, 16), c = lane_of(x, 32), d = lane_of(x, 48);
-  return MAX ? max(max(a, b), max(c, d)) : min(min(a, b), min(c, d));
 }
 // block-wide exclusive scan of a per-thread count (1024 threads = 16 waves): wave scans on the VALU, the 16 wave
 // totals through LDS (wsum: 16-byte aligned, 16 words); every thread sums the totals of the waves before its own

@@ -150,6 +150,28 @@ def test_mqa_logits_many_rows(dev, M, N):
     assert np.all(np.abs(got[t].cpu().numpy()[fin] - exp[fin]) <= 2e-5 * scale[fin])
 
 
+@pytest.mark.parametrize("M,N,nreq", [(64, 16384, 8), (256, 9000, 5), (100, 40000, 64), (40, 20000, 1)])
+def test_mqa_logits_short_ranges(dev, M, N, nreq):
+    """Rows of several requests, each over its own keys, a small part of all: the workgroups of keys that no row of a chunk
+    sees share the others' rows. The same bits as the row-at-a-time kernel, -inf everywhere else."""
+    from arcagi2_flashnext_dots3_amd import kernels
+    g = torch.Generator().manual_seed(M + N)
+    codes = torch.randint(0, 120, (N, 128), generator=g, dtype=torch.uint8).to(dev)
+    scales = torch.rand(N, generator=g).to(dev)
+    q = torch.randn(M, 64, 128, generator=g).to(torch.bfloat16).to(dev)
+    w = torch.randn(M, 64, generator=g).to(dev)
+    r = torch.arange(M) * nreq // M
+    ks = (r * (N // max(nreq, 8))).to(torch.int32)
+    ke = (ks + 1 + torch.randint(0, N // max(nreq, 8), (M,), generator=g)).to(torch.int32)
+    ke[M // 2] = ks[M // 2]
+    ks, ke = ks.to(dev), ke.to(dev)
+    print(f"[mqa logits] short ranges M={M} N={N} nreq={nreq}", flush=True)
+    got = kernels.mqa_logits(q, (codes, scales), w, ks, ke)
+    exp = torch.cat([kernels.mqa_logits(q[i:i + 4], (codes, scales), w[i:i + 4], ks[i:i + 4], ke[i:i + 4]) for i in range(0, M, 4)])
+    assert torch.equal(got, exp) and int((got > -float("inf")).sum()) == int((ke - ks).sum())
+
+
+
 @pytest.mark.parametrize("B,nn,two_d,dtype", [(3, 2, False, torch.int64), (3, 4, True, torch.int32), (5, 1, False, torch.int32)])
 def test_paged_logits_rows_formed_in_the_kernel(dev, B, nn, two_d, dtype):
     """spmla_paged_mqa_logits_seq (the wrapper) against spmla_paged_mqa_logits with explicit per-row requests and
