@@ -1505,8 +1505,9 @@ __global__ void __launch_bounds__(TK_NT, EPT <= 16 ? 8 : 4) topk_row_kernel(Topk
 struct BkWs {                                             // workspace of a row: G list lengths, then G lists
   static constexpr int GMAX = 8;
   static constexpr long long LISTS = 64;                  // bytes before the lists
-  static constexpr long long NEED = LISTS + (long long)GMAX * BK_LIST * 8;
+  static constexpr long long row_bytes(int G) { return LISTS + (long long)G * BK_LIST * 8; }
 };
+static_assert(BkWs::GMAX * 4 <= BkWs::LISTS && BkWs::row_bytes(1) % 64 == 0, "lengths before the lists, rows 64-byte aligned");
 struct TopkChunkParams {
   const void* lg; long long lg_st;
   const int* ctx; int rows, Lc, K;
@@ -1614,15 +1615,13 @@ __global__ void __launch_bounds__(TK_NT) topk_lists_kernel(TopkChunkParams p) {
 //            takes its slots from a block scan per pass over 8 consecutive columns per thread, so every list is
 //            in column order (the finishing pass's stable radix sort of fp16 keys relies on it). Otherwise the
 //            next level narrows the prefix to b, and this pass also builds its chunk's histogram of that level
-//            (into the other half of the histogram buffer, which no workgroup of the row is reading) and, when the
-//            workspace has the overflow area, writes its chunk's keys in b there (at the offset the level-0
-//            histograms give), so that the next level's collect pass reads those keys instead of the row.
+//            (into the other half of the histogram buffer, which no workgroup of the row is reading).
 // A finishing pass (one workgroup per row) resolves the candidates' remaining levels, sorts the K winners and
 // writes the positions. Rows with n <= K, and rows whose bin is still too large after two levels (heavy ties), run
 // the one-workgroup selection there. Per-row state lives in the workspace, one header per level (the collect pass
 // of level L reads header L and its first workgroup writes header L + 1).
 enum : int { TKW_SELECT = 0, TKW_WHOLE = 1, TKW_CANDS = 2, TKW_FALLBACK = 3 };
-struct TkwHdr { int state, prefix, mask, need, sb, binc, lvl, ovf; };   // 32 bytes; ovf: next level reads the overflow list
+struct __attribute__((aligned(32))) TkwHdr { int state, prefix, mask, need, sb, binc, lvl; };
 
 struct TopkWs {
   int G, CL;                                      // chunks per row, columns per chunk (multiple of 1024)
@@ -1655,7 +1654,6 @@ struct TopkWsParams {
   const int* ctx; int rows, Lc, K;
   int* out; long long out_st;
   uint8_t* ws; TopkWs w;
-  unsigned long long* ovf;                        // optional overflow lists, G * CL entries per row (or null)
   int level;
 };
 
@@ -1666,7 +1664,7 @@ __device__ inline int tkw_n(const TopkWsParams& p, int row) {
 
 // the row's state entering level p.level (level 0: select everything, need K)
 __device__ inline TkwHdr tkw_state(const TopkWsParams& p, int row) {
-  if (p.level == 0) return TkwHdr{TKW_SELECT, 0, 0, p.K, 0, 0, 0, 0};
+  if (p.level == 0) return TkwHdr{TKW_SELECT, 0, 0, p.K, 0, 0, 0};
   return p.w.hdr(p.ws, row)[p.level];
 }
 
@@ -1753,10 +1751,6 @@ __global__ void __launch_bounds__(TK_NT) topk_collect_kernel(TopkWsParams p) {
   const uint32_t sb = (uint32_t)st.sb + sum, cb = sh[4];   // this chunk's first winner / candidate slot
   const bool narrow = !whole && !fits && p.level + 1 < 2;   // uniform per row: the next level runs on bin b
   const int nshift = tk_shift(p.level + 1);
-  // level 0 narrowing with an overflow area: the chunk's keys in b go to the row's overflow list (at cb, like the
-  // candidates), where level 1 reads them
-  const bool to_ovf = narrow && p.ovf != nullptr;
-  unsigned long long* ovf_row = p.ovf ? p.ovf + (long long)row * p.w.G * p.w.CL : nullptr;
   if (narrow) {
     for (int i = tid; i < TK_HCOPY * TK_HSTR; i += TK_NT) nh[i] = 0;
     __syncthreads();
@@ -1769,47 +1763,24 @@ __global__ void __launch_bounds__(TK_NT) topk_collect_kernel(TopkWsParams p) {
     h.sb = st.sb + (int)above;
     h.binc = (int)binc;
     h.lvl = p.level + 1;
-    h.ovf = 0;
     if (whole) { h.state = TKW_WHOLE; h.sb = st.sb + (int)need; }
     else if (fits) h.state = TKW_CANDS;
-    else { h.state = p.level + 1 < 2 ? TKW_SELECT : TKW_FALLBACK; h.ovf = to_ovf ? 1 : 0; }
+    else h.state = p.level + 1 < 2 ? TKW_SELECT : TKW_FALLBACK;
     *next = h;
   }
   unsigned long long* sel = p.w.sel(p.ws, row);
-  unsigned long long* cand = to_ovf ? ovf_row : p.w.cand(p.ws, row);
-  const uint32_t clim = to_ovf ? (uint32_t)(p.w.G * p.w.CL) : (uint32_t)TK_CAP;   // entries of the candidate list
+  unsigned long long* cand = p.w.cand(p.ws, row);
   const void* x = lrow<F16>(p.lg, row, p.lg_st);
-  // the keys this workgroup visits: logits columns c0 .. c1, or (a level narrowed with an overflow list) entries
-  // c0 .. c1 of the overflow list: the previous level's bin keys of chunk g, at the offset its histograms give
-  int c0 = g * p.w.CL, c1 = min(c0 + p.w.CL, n);
-  const bool from_ovf = st.ovf != 0 && p.ovf != nullptr;
-  if (from_ovf) {
-    const uint32_t* h0 = p.w.hist(p.ws, row) + (long long)((p.level - 1) & 1) * p.w.G * 2048;
-    const uint32_t pb = ((uint32_t)prefix >> tk_shift(p.level - 1)) & 0x7ffu;
-    const uint32_t lim = (uint32_t)(p.w.G * p.w.CL);   // entries of the row's overflow list
-    uint32_t o = 0;
-    for (int c = 0; c < g; ++c) o += h0[(long long)c * 2048 + pb];
-    const uint32_t e = o + h0[(long long)g * 2048 + pb];
-    c0 = (int)min(o, lim);
-    c1 = (int)min(max(e, o), lim);
-  }
+  const int c0 = g * p.w.CL, c1 = min(c0 + p.w.CL, n);      // the columns this workgroup visits
   // thread t visits the 8 consecutive entries 8t .. 8t + 7 of each 8192-entry pass, and the slots of a pass come
   // from one block scan of the per-thread counts: every list the pass appends to stays in column order (the
   // finishing pass's stable sort relies on it to order equal keys by column)
-  const bool vec = !from_ovf && ((uintptr_t)x & 15u) == 0u;   // 16-byte aligned row: vector loads
+  const bool vec = ((uintptr_t)x & 15u) == 0u;              // 16-byte aligned row: vector loads
   uint32_t sbase = sb, cbase = cb;                  // running slot bases of this chunk's lists
   for (int base = c0; base < c1; base += 8 * TK_NT) {
     uint32_t k[8];
-    int jj[8];
     const int j0 = base + 8 * tid;
-    if (from_ovf) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const unsigned long long e = j0 + i < c1 ? ovf_row[j0 + i] : 0ull;
-        k[i] = (uint32_t)(e >> 32);
-        jj[i] = (int)~(uint32_t)e;
-      }
-    } else if (vec && j0 + 8 <= c1) {
+    if (vec && j0 + 8 <= c1) {
       if constexpr (F16) {
         const u32x4 v = *(const u32x4*)((const uint16_t*)x + j0);
 #pragma unroll
@@ -1819,14 +1790,9 @@ __global__ void __launch_bounds__(TK_NT) topk_collect_kernel(TopkWsParams p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) { k[i] = okey(a[i]); k[4 + i] = okey(b[i]); }
       }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) jj[i] = j0 + i;
     } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        k[i] = j0 + i < c1 ? lkey<F16>(x, j0 + i) : 0u;
-        jj[i] = j0 + i;
-      }
+      for (int i = 0; i < 8; ++i) k[i] = j0 + i < c1 ? lkey<F16>(x, j0 + i) : 0u;
     }
     uint32_t selm = 0, candm = 0, binm = 0;
 #pragma unroll
@@ -1834,7 +1800,7 @@ __global__ void __launch_bounds__(TK_NT) topk_collect_kernel(TopkWsParams p) {
       const bool in = j0 + i < c1 && (k[i] & mask) == prefix;
       const uint32_t d = (k[i] >> shift) & 0x7ffu;
       selm |= (uint32_t)(in && (d > b || (whole && d == b))) << i;
-      candm |= (uint32_t)(in && (fits || to_ovf) && d == b) << i;
+      candm |= (uint32_t)(in && fits && d == b) << i;
       binm |= (uint32_t)(in && d == b) << i;
     }
     // both counts stay below 2^16: a pass holds 8192 entries
@@ -1845,8 +1811,8 @@ __global__ void __launch_bounds__(TK_NT) topk_collect_kernel(TopkWsParams p) {
     cbase += tot >> 16;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      if ((selm >> i) & 1u) { if (so < (uint32_t)TK_KMAX) sel[so] = tk_pack(k[i], jj[i]); ++so; }
-      if ((candm >> i) & 1u) { if (co < clim) cand[co] = tk_pack(k[i], jj[i]); ++co; }
+      if ((selm >> i) & 1u) { if (so < (uint32_t)TK_KMAX) sel[so] = tk_pack(k[i], j0 + i); ++so; }
+      if ((candm >> i) & 1u) { if (co < (uint32_t)TK_CAP) cand[co] = tk_pack(k[i], j0 + i); ++co; }
       if (narrow && ((binm >> i) & 1u))
         atomicAdd(&nh[(tid & (TK_HCOPY - 1)) * TK_HSTR + ((k[i] >> nshift) & 0x7ffu)], 1u);
     }
@@ -2098,6 +2064,13 @@ inline int flat_rows(int M, int N) {
   return best;
 }
 
+// Workspace bytes of a row by its route: none up to BK_COLS columns, the chunks' lists up to GMAX chunks, the radix state
+static int topk_chunks_of(int Lc) { return (Lc + idx::BK_COLS - 1) / idx::BK_COLS; }
+static long long topk_ws_row(int Lc) {
+  if (Lc <= idx::BK_COLS) return 0;
+  return topk_chunks_of(Lc) <= idx::BkWs::GMAX ? idx::BkWs::row_bytes(topk_chunks_of(Lc)) : idx::topk_ws_layout(Lc).row_bytes;
+}
+
 extern "C" {
 
 static int logits_row(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
@@ -2154,7 +2127,7 @@ int spmla_index_logits_hist(const void* q, long long q_st, long long q_sh, const
   if (K > idx::TK_KMAX) return SPMLA_ELIMIT;
   if (rows == 0 || Lc == 0) return SPMLA_OK;
   const idx::TopkWs tw = idx::topk_ws_layout(Lc);
-  if (!topk_ws || ((uintptr_t)topk_ws & 15) || ws_bytes < (long long)rows * tw.row_bytes) return SPMLA_EARG;
+  if (!topk_ws || ((uintptr_t)topk_ws & 15) || ws_bytes < rows * topk_ws_row(Lc)) return SPMLA_EARG;
   if (tw.CL >= 65536) return SPMLA_ELIMIT;                  // longer rows: use the separate calls
   return logits_row(q, q_st, q_sh, w, w_st, store, R_local, rows_per_block, block_stride, block_table, bt_st,
                     block_size, req, ctx, rows, H, D, Lc, 1, 0, noinf, out, out_st, out_dtype, stream, 1);
@@ -2255,17 +2228,10 @@ int spmla_topk(const void* logits, long long lg_st, const int* ctx, int rows, in
   return (int)hipGetLastError();
 }
 
-// Workspace: the rows' headers, lists and histograms, then (optional) the rows' overflow lists of G * CL entries,
-// used when a chunk's bin count fits the collect pass's 16-bit slot counters (CL < 2^16).
-static long long topk_ws_base(int rows, int Lc) { return (long long)rows * idx::topk_ws_layout(Lc).row_bytes; }
-static long long topk_ws_ovf(int rows, int Lc) {
-  const idx::TopkWs w = idx::topk_ws_layout(Lc);
-  return w.CL < 65536 ? (long long)rows * w.G * w.CL * 8 : 0;
-}
-
+// (never 0 for a row, so that a buffer of this size has an address: 64 bytes more a row)
 long long spmla_topk_ws_bytes(int rows, int Lc, int K) {
   if (rows < 0 || Lc < 0 || K <= 0) return 0;
-  return topk_ws_base(rows, Lc) + topk_ws_ovf(rows, Lc);
+  return (long long)rows * (topk_ws_row(Lc) + 64);
 }
 
 int spmla_topk_ws(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
@@ -2274,24 +2240,21 @@ int spmla_topk_ws(const void* logits, long long lg_st, const int* ctx, int rows,
   if (K > idx::TK_KMAX) return SPMLA_ELIMIT;
   if (rows == 0) return SPMLA_OK;
   if (!logits || !ctx || !out || !ws) return SPMLA_EARG;
-  const long long base = topk_ws_base(rows, Lc), ovf = topk_ws_ovf(rows, Lc);
-  if (((uintptr_t)ws & 15) || ws_bytes < base) return SPMLA_EARG;
+  if (((uintptr_t)ws & 15) || ws_bytes < rows * topk_ws_row(Lc)) return SPMLA_EARG;
   if (Lc <= idx::BK_COLS) {                         // a row fits one workgroup's registers
     idx::topk_rows(idx::TopkParams{logits, lg_st, ctx, rows, Lc, K, out, out_st}, dtype, (hipStream_t)stream);
     return (int)hipGetLastError();
   }
-  if (Lc <= idx::BkWs::GMAX * idx::BK_COLS) {       // up to 8 chunks, whose lists one workgroup's registers hold
-    const int G = (Lc + idx::BK_COLS - 1) / idx::BK_COLS;
-    idx::topk_chunks(idx::TopkChunkParams{logits, lg_st, ctx, rows, Lc, K, out, out_st, (uint8_t*)ws,
-                                          idx::topk_ws_layout(Lc).row_bytes, G, ((Lc + G - 1) / G + 1023) / 1024 * 1024},
+  const int G = topk_chunks_of(Lc);
+  if (G <= idx::BkWs::GMAX) {                       // the chunks' lists fit one workgroup's registers
+    idx::topk_chunks(idx::TopkChunkParams{logits, lg_st, ctx, rows, Lc, K, out, out_st, (uint8_t*)ws, topk_ws_row(Lc), G,
+                                          ((Lc + G - 1) / G + 1023) / 1024 * 1024},
                      dtype, (hipStream_t)stream);
     return (int)hipGetLastError();
   }
   idx::TopkWsParams p;
   p.lg = logits; p.lg_st = lg_st; p.ctx = ctx; p.rows = rows; p.Lc = Lc; p.K = K; p.out = out; p.out_st = out_st;
   p.ws = (uint8_t*)ws; p.w = idx::topk_ws_layout(Lc);
-  // with room for the overflow lists, a level that narrows hands its bin's keys to the next level in a list
-  p.ovf = ovf > 0 && ws_bytes >= base + ovf ? (unsigned long long*)((uint8_t*)ws + base) : nullptr;
   if (dtype == 1) idx::topk_ws_passes<true>(p, (hipStream_t)stream);
   else idx::topk_ws_passes<false>(p, (hipStream_t)stream);
   return (int)hipGetLastError();
@@ -2310,10 +2273,8 @@ int spmla_topk_scratch(const void* logits, long long lg_st, const int* ctx, int 
   if (K > idx::TK_KMAX) return SPMLA_ELIMIT;
   if (rows == 0) return SPMLA_OK;
   if (!logits || !ctx || !out) return SPMLA_EARG;
-  const long long full = spmla_topk_ws_bytes(rows, Lc, K), base = topk_ws_base(rows, Lc);
-  if (full <= 0) return SPMLA_EARG;
-  if (base > idx::TOPK_SCRATCH_BYTES) return SPMLA_ELIMIT;   // beyond the fixed scratch: use spmla_topk_ws
-  const long long need = full <= idx::TOPK_SCRATCH_BYTES ? full : base;   // the overflow lists when they fit
+  const long long radix = (long long)rows * idx::topk_ws_layout(Lc).row_bytes, need = rows * topk_ws_row(Lc);
+  if (max(radix, need) > idx::TOPK_SCRATCH_BYTES) return SPMLA_ELIMIT;   // (as long as every row took the radix state)
   void* ws = nullptr;
   const int rc = scratch_ptr(&ws);
   if (rc != SPMLA_OK) return rc;

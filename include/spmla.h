@@ -70,18 +70,16 @@ int spmla_index_logits(const void* q, long long q_st, long long q_sh, const floa
 int spmla_topk(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
                long long out_st, int dtype, void* stream);
 
-/* Bytes of workspace spmla_topk_ws uses for rows x Lc (0 for invalid sizes): the per-row state, lists and histograms,
- * then the overflow lists (8 bytes per column) through which a narrowing level of rows above 262144 columns hands its
- * boundary bin's keys to the next level instead of that level reading the row again. */
+/* Bytes of workspace for spmla_topk_ws over rows x Lc (0 for invalid sizes), per row: nothing is used up to 32768 columns
+ * (64 bytes, so that a buffer has an address), a list of 18 KiB per chunk up to 262144, 144 KiB of state above. */
 long long spmla_topk_ws_bytes(int rows, int Lc, int K);
 
 /* spmla_topk with the same result, long rows spread over several workgroups: rows of at most 32768 columns take
  * spmla_topk's one workgroup, up to 262144 columns a workgroup per chunk of at most 32768 columns and one that selects
  * among their lists, above that a histogram pass and two collect passes over 4 chunks and a finishing workgroup.
- * ws: device memory of spmla_topk_ws_bytes(rows, Lc, K) bytes (a smaller one without the overflow lists is accepted),
- * 16-byte aligned, any contents (every pass writes what the next reads); calls that share a workspace must not
- * overlap. Same replacement as spmla_topk (fast_topk.local + merge at P = 1, dotsnote/engine/arcstats_pkg/arcstats/
- * fast_topk.py:52-78; csrc/topk_select.cu:251-286; shard_indexer.py:194-221). */
+ * ws: device memory of spmla_topk_ws_bytes(rows, Lc, K) bytes, 16-byte aligned, any contents (every pass writes what the
+ * next reads); calls that share a workspace must not overlap. Same replacement as spmla_topk (fast_topk.local + merge at
+ * P = 1, dotsnote/engine/arcstats_pkg/arcstats/fast_topk.py:52-78; csrc/topk_select.cu:251-286; shard_indexer.py:194-221). */
 int spmla_topk_ws(const void* logits, long long lg_st, const int* ctx, int rows, int Lc, int K, int* out,
                   long long out_st, void* ws, long long ws_bytes, int dtype, void* stream);
 
@@ -104,9 +102,9 @@ int spmla_topk_ws_prehist(const void* logits, long long lg_st, const int* ctx, i
 /* spmla_topk_ws without a caller workspace and without any allocation: the passes use the library's own
  * fixed device scratch (a file-scope array of spmla_topk_scratch_bytes() = 16 MiB per GPU, held from library load
  * until the process ends; its device address is looked up once per device on the first call there). Same result
- * as spmla_topk_ws (the overflow lists included when they fit the scratch). Sizes whose workspace without the
- * overflow lists exceeds the scratch return SPMLA_ELIMIT (e.g. 64 rows fit at any Lc up to 2^31). All calls on one GPU share the scratch: calls that overlap on one GPU (other streams,
- * other threads) race and must not be issued. The scratch keeps the last call's contents; the passes need no
+ * as spmla_topk_ws. Sizes whose state in the passes of the longest rows exceeds the scratch return SPMLA_ELIMIT (64 rows
+ * fit at any Lc up to 2^31). All calls on one GPU share the scratch: calls that overlap on one GPU (other streams, other
+ * threads) race and must not be issued. The scratch keeps the last call's contents; the passes need no
  * particular initial contents. No counterpart in the reference: for callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc). */
 long long spmla_topk_scratch_bytes(void);

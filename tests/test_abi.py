@@ -156,6 +156,20 @@ def test_topk_workspace_size():
     assert L.spmla_topk_ws_bytes(1, 131072, 2048) > one          # more chunks per row, more histograms
 
 
+@pytest.mark.parametrize("rows,Lc,lists", [(2048, 16384, 0), (64, 32768, 0), (64, 32769, 2), (2048, 131072, 4), (3, 262144, 8)])
+def test_topk_workspace_holds_what_the_route_writes(rows, Lc, lists):
+    """No state for rows that one workgroup selects, a list per chunk of 32768 columns up to eight (2304 entries of 8 bytes
+    after 64 bytes of lengths), nothing per column; a workspace that is too small for it is refused."""
+    from arcagi2_flashnext_dots3_amd import _lib
+    L = _lib.lib()
+    need = rows * (64 + lists * 2304 * 8) if lists else 0
+    assert need < L.spmla_topk_ws_bytes(rows, Lc, 2048) <= need + 128 * rows
+    if lists:      # (placeholder pointers 256: refused before a launch)
+        assert L.spmla_topk_ws(256, Lc, 256, rows, Lc, 2048, 256, 2048, 256, need - 16, 0, None) == -2
+        assert L.spmla_index_logits_hist(256, 8192, 128, 256, 64, 256, 64, 64, 8448, 256, 512, 64, 256, 256, rows, 64, 128,
+                                         Lc, 0, 256, Lc, 0, 256, need - 16, 2048, None) == -2
+
+
 def test_zero_sized_calls_are_noops():
     from arcagi2_flashnext_dots3_amd import _lib
     L = _lib.lib()

@@ -51,9 +51,8 @@ def test_index_logits(dev, rows, L, seed):
 
 
 def _topk_check(dev, lg, ctx, K):
-    """The top-k paths against the oracle: several workgroups per row with the full workspace (a narrowing level
-    hands its bin's keys to the next in the overflow lists), the same with a workspace too small for those lists (the
-    next level reads the row again), and one workgroup per row."""
+    """The top-k paths against the oracle: with a workspace of its own size, with a smaller one that still holds the lists,
+    and without one (one workgroup per row)."""
     from arcagi2_flashnext_dots3_amd import _lib, kernels
     exp = ref.topk(lg, ctx, K)
     nb = int(_lib.lib().spmla_topk_ws_bytes(lg.shape[0], lg.shape[1], K))
@@ -450,3 +449,17 @@ def test_topk_skewed_and_tied_rows(dev, L, dtype):
         for single in (False, True):
             got = kernels.topk(dlg, dctx, K, single_pass=single).cpu().numpy()
             assert np.array_equal(got, exp), f"rows {np.where((got != exp).any(1))[0]} (single_pass={single})"
+
+
+@pytest.mark.parametrize("rows,L", [(3, 32768), (5, 32769), (3, 100003), (2, 262144), (2, 262145), (1, 600000)])
+def test_topk_writes_inside_its_workspace(dev, rows, L):
+    """The selection with a workspace of exactly spmla_topk_ws_bytes, the bytes behind it untouched."""
+    from arcagi2_flashnext_dots3_amd import _lib, kernels
+    lg = torch.randn(rows, L, generator=torch.Generator().manual_seed(L))
+    lg[:, ::5] = lg[:, :1]                                       # ties: full lists
+    ctx = np.full(rows, L, dtype=np.int32)
+    nb = int(_lib.lib().spmla_topk_ws_bytes(rows, L, 2048))
+    print(f"[topk ws] rows={rows} L={L} {nb} bytes", flush=True)
+    ws = torch.full((nb + 4096,), 0xA5, dtype=torch.uint8, device=dev)
+    got = kernels.topk(lg.to(dev), torch.from_numpy(ctx).to(dev), 2048, ws=ws[:nb]).cpu().numpy()
+    assert np.array_equal(got, ref.topk(lg.numpy(), ctx, 2048)) and bool((ws[nb:] == 0xA5).all())
