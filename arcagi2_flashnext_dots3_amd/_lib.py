@@ -109,7 +109,11 @@ def status(name, *args):
 
 def call(name, *args):
     """Invoke entry point `name`; a nonzero return code raises RuntimeError naming the entry point."""
-    rc = status(name, *args)
+    f = _FN.get(name)
+    try:
+        rc = f(*args) if f else status(name, *args)
+    except TypeError:
+        rc = status(name, *args)
     if rc != 0:
         raise RuntimeError(f"{name} failed: {rc} ({ERRORS.get(rc, 'hip error')})")
     return rc

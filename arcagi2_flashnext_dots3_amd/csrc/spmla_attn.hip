@@ -897,7 +897,7 @@ static int attn_launch(const void* q, long long q_st, long long q_sh, const void
   if (T == 0) return SPMLA_OK;
   if (!q || !idx || (R > 0 && !pool)) return SPMLA_EARG;
   const bool f32part = opart != nullptr;   // fp32 partials (any S) instead of the bf16 output
-  const bool fused = !f32part && S > 1;    // bf16 output of S splits merged in the kernel (workspace ws)
+  bool fused = !f32part && S > 1;          // bf16 output of S splits merged in the kernel (workspace ws)
   if (f32part ? !lsepart : (!out || !lse)) return SPMLA_EARG;
   if (fused) {
     if (!ws || prior_o) return SPMLA_EARG;
@@ -908,7 +908,12 @@ static int attn_launch(const void* q, long long q_st, long long q_sh, const void
   if (((uintptr_t)q & 15) || (q_st & 7) || (q_sh & 7) || ((uintptr_t)pool & 15)) return SPMLA_EALIGN;
   if (out && (((uintptr_t)out & 7) || (o_st & 3) || (o_sh & 3))) return SPMLA_EALIGN;
   if (f32part && ((uintptr_t)opart & 15)) return SPMLA_EALIGN;
-  if (fused && ((K + S - 1) / S + attn::TR - 1) / attn::TR * attn::TR > attn::KMAX) return SPMLA_ELIMIT;
+  if (fused && ((K + S - 1) / S + attn::TR - 1) / attn::TR * attn::TR > attn::KMAX) return SPMLA_ELIMIT;   // (a limit kept
+  // from the kernel that merged before; the head-group kernel has none)
+  if (fused) {
+    S = rules::merged_splits(T, H, K, S);
+    fused = S > 1;
+  }
   if (fused || !attn_wide(T, H, K, S))
     return pk::launch_tokens(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out, o_st,
                              o_sh, lse, lse_st, opart, lsepart, prior_o, po_st, po_sh, prior_lse, pl_st,
@@ -948,7 +953,7 @@ static int attn576_launch(const void* q, long long q_st, long long q_sh, const v
   if (T == 0) return SPMLA_OK;
   if (!q || !idx || (R > 0 && !pool)) return SPMLA_EARG;
   const bool f32part = opart != nullptr;
-  const bool fused = !f32part && S > 1;
+  bool fused = !f32part && S > 1;
   if (f32part ? !lsepart : (!out || !lse || (fused && !ws))) return SPMLA_EARG;
   if (fused) {
     if (S > 8) return SPMLA_ELIMIT;
@@ -958,6 +963,10 @@ static int attn576_launch(const void* q, long long q_st, long long q_sh, const v
   if (((uintptr_t)q & 15) || (q_st & 7) || (q_sh & 7) || ((uintptr_t)pool & 15)) return SPMLA_EALIGN;
   if (out && (((uintptr_t)out & 7) || (o_st & 3) || (o_sh & 3))) return SPMLA_EALIGN;
   if (f32part && ((uintptr_t)opart & 15)) return SPMLA_EALIGN;
+  if (fused) {
+    S = rules::merged_splits(T, H, K, S);
+    fused = S > 1;
+  }
   if (!fused && attn_wide(T, H, K, S))
     return wide_launch(wide_params(q, q_st, q_sh, pool, R, idx, idx_st, K, kcount, T, H, sm_scale, kv_scale, S, out,
                                    o_st, o_sh, lse, lse_st, opart, lsepart, nullptr, 0, 0, nullptr, 0, pg), true, stream);

@@ -738,8 +738,8 @@ def auto_split576(T, H, K, cus=256):
 
 def auto_split(T, H, K, cus=256):
     """auto_split576 for Row656 pools: of the splits of at most ATTN_SPLIT_ROWS rows each (spmla_attn takes no longer
-    ones; unsplit any K). 128 heads, us: K = 8192, 20 tokens 85 (6 splits), unsplit 144; K = 12000, 12 / 23 tokens 86 /
-    129 (8 splits), unsplit 197 / 205."""
+    ones; unsplit any K, and it takes fewer splits where those are faster). 128 heads, us: K = 8192, 20 tokens 75, unsplit
+    144; K = 12000, 12 / 23 tokens 70 / 121, unsplit 197 / 205."""
     return _best_split(T, H, K, ATTN_SPLIT_ROWS, cus)
 
 

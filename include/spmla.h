@@ -312,9 +312,10 @@ int spmla_attn576(const void* q, long long q_st, long long q_sh, const void* poo
 /* Bytes of the workspace spmla_attn needs for T tokens, H heads and S splits (0 for S = 1; -1 for bad sizes). */
 long long spmla_attn_ws_bytes(int T, int H, int S);
 
-/* spmla_attn_splitk with the bf16 out + lse for any S in 1 .. 8: the S splits of a (token, group of 32 heads), which
+/* spmla_attn_splitk with the bf16 out + lse for any S in 1 .. 8: the splits of a (token, group of 32 heads), which
  * share the token's min(K, kcount) entries, merge in the kernel -- each writes its normalized fp32 partial and lse to
- * ws, and the last split to finish merges all of them in order (weights e^(lse_s - M) / Z) into out / lse.
+ * ws, and the last split to finish merges all of them in order (weights e^(lse_s - M) / Z) into out / lse. S splits where
+ * they are one round of workgroups (T * ceil(H / 32) * S <= 256), beyond that as many of up to S as are fastest.
  * ws: spmla_attn_ws_bytes(T, H, S) bytes, 256-byte aligned. Its first C = 4 * T * ceil(H / 128) bytes (rounded up
  * to a multiple of 256) are the launch's counters and must be zero when it starts; the kernel leaves them zero, and
  * the bytes past them are scratch. So a workspace zero-filled once serves launches that run one after another,
