@@ -200,6 +200,7 @@ def index_logits(q, w, store, block_table, block_size, req, ctx, Lc, out=None, P
 
 _WS = {}
 _WS_CNT = {}      # attention workspaces: counter bytes of the last launch (the bytes known to be zero)
+_WS_LOCK = threading.Lock()      # held from the look-up of an attention workspace until its launch is queued
 _WS_KEEP = []     # every workspace ever handed out: a HIP graph captured with one keeps its address for good
 
 
@@ -213,7 +214,7 @@ def _workspace(kind, device, nbytes, zero=False):
     key is None under capture."""
     dev = torch.device(device)
     if torch.cuda.is_current_stream_capturing():
-        have = [b for (k, d, _), b in _WS.items() if k == kind and d == dev]
+        have = [b for (k, d, _), b in list(_WS.items()) if k == kind and d == dev]
         b = max(have, key=lambda t: t.numel(), default=None)
         _need(b is not None and b.numel() >= nbytes,
               f"{kind} workspace of {nbytes} bytes needed under HIP graph capture: pass one explicitly, or make an "
@@ -232,7 +233,7 @@ def _workspace(kind, device, nbytes, zero=False):
 
 def _has_workspace(kind, device, nbytes):
     dev = torch.device(device)
-    return any(k == kind and d == dev and b.numel() >= nbytes for (k, d, _), b in _WS.items())
+    return any(k == kind and d == dev and b.numel() >= nbytes for (k, d, _), b in list(_WS.items()))
 
 
 def fused_max_tokens(H, cus=256):
@@ -258,7 +259,8 @@ def reserve_workspace(device, H, T=None, split=8, K=None):
     No-op when present."""
     nb = attn_reserve_bytes(H, K) if T is None else attn_ws_bytes(T, H, split) if T > 0 else 0
     if nb > 0:
-        _workspace("attn", device, nb, zero=True)
+        with _WS_LOCK:
+            _workspace("attn", device, nb, zero=True)
 
 
 def _attn_workspace(device, T, H, split, private=False):
@@ -277,9 +279,6 @@ def _attn_workspace(device, T, H, split, private=False):
             ws[_WS_CNT[key]:cnt].zero_()
         _WS_CNT[key] = cnt
     return ws
-
-
-_WS_LOCK = threading.Lock()
 
 
 def _merged_call(device, T, H, split, private, stream, name, *args):

@@ -354,3 +354,35 @@ def test_merged_launches_of_two_threads_on_one_stream(monkeypatch):
     first.join()
     second.join()
     assert dirty == [False] and small_done.is_set()
+
+
+def test_reservation_beside_a_merged_launch(monkeypatch):
+    """A reservation by another host thread replaces a stream's attention workspace by a larger one, zero throughout. A
+    launch that already has the old one must still clear that one's counters."""
+    import ctypes
+    import threading
+    from arcagi2_flashnext_dots3_amd import _lib, kernels
+    T, H, K, key = 100, 16, 64, ("attn", torch.device("cpu"), 0)
+    old = torch.full((kernels.attn_ws_bytes(T, H, 2),), 7, dtype=torch.uint8)        # the last launch's scratch
+    monkeypatch.setattr(kernels, "_WS", {key: old})
+    monkeypatch.setattr(kernels, "_WS_CNT", {key: 0})
+    monkeypatch.setattr(kernels, "_WS_KEEP", [old])
+    monkeypatch.setattr(kernels, "_stream", lambda t: 0)
+    monkeypatch.setattr(kernels, "_device_stream", lambda d: 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    workspace, dirty = kernels._workspace, []
+    other = threading.Thread(target=kernels.reserve_workspace, args=(key[1], 128, 64))
+
+    def beside(*a, **kw):                       # the launch has its workspace, then the reservation comes
+        got = workspace(*a, **kw)
+        if threading.current_thread() is not other:
+            other.start()
+            other.join(0.5)
+        return got
+    monkeypatch.setattr(kernels, "_workspace", beside)
+    monkeypatch.setattr(_lib, "call", lambda name, *a: dirty.append(
+        a[-3] != old.data_ptr() or any(ctypes.string_at(a[-3], kernels._attn_counter_bytes(T, H)))))
+    kernels.attend(torch.zeros(T, H, 576, dtype=torch.bfloat16), torch.zeros(64, 576, dtype=torch.uint8),
+                   torch.zeros(T, K, dtype=torch.int32), 0.1, split=2)
+    other.join()
+    assert dirty == [False] and kernels._WS[key].numel() > old.numel()
