@@ -292,7 +292,7 @@ __global__ void __launch_bounds__(256, 1) fwd_kernel(Params p) {
     const int* btrow = p.pg.bt + (long long)p.pg.req[t] * p.pg.bt_st;
     int b[KMAX / 256];
 #pragma unroll
-    for (int k = 0; k < KMAX / 256; ++k) b[k] = page_entry(p.pg, btrow, xs[k]);
+    for (int k = 0; k < KMAX / 256; ++k) b[k] = page_entry(p.pg, btrow, xs[k], p.pg.req + t);
 #pragma unroll
     for (int k = 0; k < KMAX / 256; ++k) xs[k] = page_row(p.pg, xs[k], b[k]);
   }

@@ -317,7 +317,7 @@ __global__ void __launch_bounds__(256, 1) attn_kernel(Params p) {
   // waits for a round trip; before the first tile the two loads overlap the query's.
   const int* btrow = nullptr;
   if (!PK && p.pg.bt) btrow = p.pg.bt + (long long)p.pg.req[t] * p.pg.bt_st;
-  auto table = [&](int x) -> int { return !PK && p.pg.bt ? page_entry(p.pg, btrow, x) : 0; };
+  auto table = [&](int x) -> int { return !PK && p.pg.bt ? page_entry(p.pg, btrow, x, p.pg.req + t) : 0; };
   auto row_of = [&](int x, int b) -> int { return row_ok(!PK && p.pg.bt ? page_row(p.pg, x, b) : x); };
   int xn = row_raw(w), x1 = row_raw(w + NW), x2 = PK ? -1 : row_raw(w + 2 * NW), bn = 0, b1 = 0;
   uint32_t mcur = mk_raw(w), mnxt = mk_raw(w + NW), mnn = 0u;

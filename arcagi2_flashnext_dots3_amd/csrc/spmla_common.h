@@ -117,13 +117,14 @@ __device__ inline int remap_xcd(int i, int n) {
 struct Pages {
   const int* req; const int* bt; long long bt_st; int cols, sh; long long stride;
 };
-__host__ __device__ inline int page_entry(const Pages& g, const int* btrow, int x) {   // -1: x has none
-  int b = -1;
-  if (x >= 0 && (x >> g.sh) < g.cols) b = btrow[x >> g.sh];
-  return b;
+__host__ __device__ inline bool page_has(const Pages& g, int x) { return x >= 0 && (x >> g.sh) < g.cols; }
+// x's entry; where x has none any readable word is read in its place, so that no lookup stands under a branch (Row656
+// prefill, against one that always reads the table: 1.3 % longer under branches, 0.5 % so)
+__host__ __device__ inline int page_entry(const Pages& g, const int* btrow, int x, const int* any) {
+  return *(page_has(g, x) ? btrow + (x >> g.sh) : any);
 }
 __host__ __device__ inline int page_row(const Pages& g, int x, int blk) {              // blk: x's entry
-  return blk >= 0 ? (int)(blk * g.stride + (x & ((1 << g.sh) - 1))) : -1;
+  return page_has(g, x) && blk >= 0 ? (int)(blk * g.stride + (x & ((1 << g.sh) - 1))) : -1;
 }
 
 // ---- launch error codes ----------------------------------------------------------------------------------

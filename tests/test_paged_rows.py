@@ -14,7 +14,7 @@ SRC = r"""
 #include "spmla_common.h"
 extern "C" void rows(const int* btrow, int cols, int sh, long long stride, const int* x, int n, int* out) {
   const spmla::Pages g{nullptr, btrow, 0, cols, sh, stride};
-  for (int i = 0; i < n; ++i) out[i] = spmla::page_row(g, x[i], spmla::page_entry(g, btrow, x[i]));
+  for (int i = 0; i < n; ++i) out[i] = spmla::page_row(g, x[i], spmla::page_entry(g, btrow, x[i], x));
 }
 """
 CHILD = r"""
