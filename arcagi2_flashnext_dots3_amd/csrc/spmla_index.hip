@@ -1154,9 +1154,10 @@ __global__ void __launch_bounds__(TK_NT) topk_kernel(TopkParams p) {
 // into one bin), so there is no second level and no sort of the winners. A row is a chain of barriers, LDS atomics and
 // one read of the row; in graphs, against a radix level over several workgroups, a second on its bin and a finishing
 // sort: 4 rows of 16000 columns 9.8 us (32.7), 64 of 32768 15.3 us (39.0), 2048 of 16384 55.6 us (356).
-// Values that crowd at the low end of their range (far outliers, skewed distributions) are binned by the key's integer
-// instead, which spaces bins by magnitude. A row whose bins from the K-th key's on still hold more than
-// BK_LIM entries somewhere (heavy ties, outliers below, no finite value) has the K-th key's bin cut further (bk_refine).
+// Where the high values crowd at the low end of the range (far outliers, skewed distributions) the bins are of the key's
+// integer instead, which spaces them by magnitude. A row whose bins from the K-th key's on still hold more than BK_LIM
+// entries somewhere (heavy ties, no finite value) has the K-th key's bin cut further (bk_refine). Below 128 entries a bin
+// is ranked by counting faster than a whole row (K = n) is sorted, and above slower (2048 of 25 distinct values 19 / 25 us).
 constexpr int BK_BINS = 4096;
 constexpr int BK_LIM = 256;                  // entries of a bin that are ranked by counting
 constexpr int BK_LIST = TK_KMAX + BK_LIM;    // entries from the K-th key's bin on
@@ -1167,7 +1168,7 @@ struct BkLds {
   __attribute__((aligned(16))) uint32_t off[BK_BINS];   // counts, then first slots, then ends
   unsigned long long list[BK_LIST];
   __attribute__((aligned(16))) uint32_t wsum[16];
-  __attribute__((aligned(16))) uint32_t red[48];        // per wave: smallest, largest finite key, smallest of its threads' largest
+  __attribute__((aligned(16))) uint32_t red[64];        // per wave: smallest, largest finite key, smallest of its threads' largest (twice)
   uint32_t sh[8];
 };
 
@@ -1185,10 +1186,16 @@ __device__ inline int bk_bin(float v, const BkRange& r) {
 }
 __device__ inline int bk_bin(float v, const BkRange& r) { return r.by_key ? bk_bin<true>(v, r) : bk_bin<false>(v, r); }
 
-// Bins of the keys v (bit i of vm: v[i] is one), K of them wanted (0 < K <= their number): L.off = every bin's first slot.
-// False (uniform) when bk_refine has to do it.
+// Bins of the n keys v (bit i of vm: v[i] is one), K of them wanted (0 < K <= n): L.off = every bin's first slot. False
+// (uniform) when bk_refine has to do it. upper: the range starts at the smallest of the threads' largest values instead of
+// the smallest value (2 K <= n, columns dealt to the threads: 1024 values at least and of independent ones a fifth to
+// four fifths of the row lie above it; where the K-th does not, bk_refine finds it in bin 0), so that values far below
+// cost no resolution. The lowest bin is not counted but is what the others leave: a floor of equal values, -inf and
+// everything below the range would queue at its counter. us, 64 rows of 32768, K = 2048, radix passes / range from
+// the smallest value, all bins counted / this: half the row at a floor 32 / 27 / 15.5, Cauchy 31 / 62 / 17, far outlier above 31
+// / 37 / 18, Gaussian 31 / 15.8 / 15.5.
 template <int EPT>
-__device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uint32_t K, BkRange& r) {
+__device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uint32_t n, uint32_t K, bool upper, BkRange& r) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   float mn = __builtin_inff(), mx = -__builtin_inff();
 #pragma unroll
@@ -1198,27 +1205,32 @@ __device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uin
     mx = fin ? fmaxf(mx, v[i]) : mx;
   }
   const uint32_t kn = wave_minmax<false>(okey(mn)), kx = wave_minmax<true>(okey(mx));
-  const uint32_t kq = wave_minmax<false>(okey(mx));
-  if (lane == 0) { L.red[wv] = kn; L.red[16 + wv] = kx; L.red[32 + wv] = kq; }
+  const uint32_t kq = wave_minmax<false>(mx == -__builtin_inff() ? ~0u : okey(mx));        // (~0: no finite key)
+  if (lane == 0) { L.red[wv] = kn; L.red[16 + wv] = kx; L.red[32 + wv] = kq; L.red[48 + wv] = kq == ~0u ? 0u : kq; }
   ((u32x4*)L.off)[tid] = u32x4{0u, 0u, 0u, 0u};
   if (tid < 8) L.sh[tid] = 0u;
   __syncthreads();
-  const uint32_t x = L.red[min(lane, 47)];                // a 16-lane row each of minima, maxima and smallest thread maxima
-  const uint32_t xx = row_minmax<true>(x), an = lane_of(row_minmax<false>(x), 0), ax = lane_of(xx, 16);
-  const float q = unkey(lane_of(xx, 32));                 // (of a wave's 64 threads with EPT values each: a high quantile)
+  const uint32_t x = L.red[lane];                         // a 16-lane row each
+  const uint32_t xx = row_minmax<true>(x), xn = row_minmax<false>(x);
+  const uint32_t an = lane_of(xn, 0), ax = lane_of(xx, 16), aq = lane_of(xn, 32);
+  const float q = unkey(lane_of(xx, 48));                 // (of a wave's 64 threads with EPT values each: a high quantile)
+  const bool high = upper && aq < ax;
   r.bin = -1;
-  r.vmin = unkey(an);
-  r.kmin = an;
+  r.kmin = high ? aq : an;
+  r.vmin = unkey(r.kmin);
   const float span = unkey(ax) - r.vmin;
   r.scale = ((float)BK_BINS - 0.01f) / span;
   if (!(r.scale > 0.f && r.scale < __builtin_inff())) return false;   // no finite value, one value, or an overflow
-  r.sh = max(0, 20 - (int)__builtin_clz((ax - an) | 1u));             // (ax - an) >> sh < 4096
+  r.sh = max(0, 20 - (int)__builtin_clz((ax - r.kmin) | 1u));         // (ax - kmin) >> sh < 4096
   // by key when the high values lie that low in the range: bins of equal width would hold hundreds of them each
-  r.by_key = q >= r.vmin && (q - r.vmin) * 2048.f < (float)EPT * span;
+  r.by_key = q >= r.vmin && (q - r.vmin) * (high ? 128.f : 2048.f / (float)EPT) < span;
   auto count = [&](auto key) {
 #pragma unroll
     for (int i = 0; i < EPT; ++i)
-      if ((vm >> i) & 1u) atomicAdd(&L.off[bk_bin<decltype(key)::value>(v[i], r)], 1u);
+      if ((vm >> i) & 1u) {
+        const int b = bk_bin<decltype(key)::value>(v[i], r);
+        if (b) atomicAdd(&L.off[b], 1u);
+      }
   };
   if (r.by_key) count(std::true_type()); else count(std::false_type());
   __syncthreads();
@@ -1229,7 +1241,7 @@ __device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uin
   uint32_t big = 0;
 #pragma unroll
   for (int e = 3; e >= 0; --e) {
-    const uint32_t c = h[e];
+    const uint32_t c = e == 0 && tid == TK_NT - 1 ? n - run : h[e];
     if (run < K) big = max(big, c);
     if (run < K && run + c >= K) { L.sh[1] = (uint32_t)(BK_BINS - 4 - 4 * tid + e); L.sh[2] = run + c; L.sh[3] = c; }
     h[e] = run;
@@ -1242,7 +1254,7 @@ __device__ inline bool bk_bins(BkLds& L, const float (&v)[EPT], uint32_t vm, uin
   r.bin = (int)L.sh[1];
   r.n = L.sh[2];
   r.c = L.sh[3];
-  return L.sh[0] <= (uint32_t)BK_LIM;
+  return L.sh[0] <= (K == n ? (uint32_t)BK_LIM / 2 : (uint32_t)BK_LIM);
 }
 
 // Entries in registers: (key, ~column) of entry i as key(i), low(i), its value val(i). fence: what follows is computed from the registers
@@ -1276,9 +1288,9 @@ struct ListRegs {
 // up: the bin of the K-th key (r.bin; -1: all) is cut by its keys' range into 4096 bins of a power of two, then that bin
 // again, then, between equal keys, by column (lo .. hi: the range of ~column), until the bin is taken whole or its entries
 // can be ranked by counting. A chain of barriers and of same-bin atomics of the equal values. us, several workgroups' radix
-// passes / a radix select over (key, column) that re-read the row / bins by key or this: 64 rows of 32768: one far outlier
-// 35 / 67 / 23, lognormal 30 / 68 / 17, 25 distinct values 39 / 85 / 45, 1 % of the values not zero 107 / 196 / 59, one
-// value 107 / 161 / 26; 64 of 131072: 50 / 90 / 38, 47 / 96 / 47, 59 / 124 / 63, 477 / 254 / 84, 478 / 214 / 45.
+// passes / a radix select over (key, column) that re-read the row / this: 64 rows of 32768: 25 distinct values 35 / 73 / 34
+// (fp16 33 / 75 / 35), 1 % of the values not zero 107 / 196 / 35, one value 107 / 161 / 27; 64 of 131072: 55 / 113 / 52 (fp16
+// 46 / 111 / 50), 477 / 254 / 55, 478 / 214 / 45.
 template <int EPT, class Ent>
 __device__ inline void bk_refine(BkLds& L, Ent ent, uint32_t vm, uint32_t n, const BkRange& r, uint32_t K, uint32_t lo,
                                  uint32_t hi) {
@@ -1482,7 +1494,7 @@ __global__ void __launch_bounds__(TK_NT, EPT <= 16 ? 8 : 4) topk_row_kernel(Topk
   float v[EPT];
   const uint32_t vm = bk_load<F16, EPT>(x, 0, n, v);
   BkRange r;
-  if (!bk_bins<EPT>(L, v, vm, K, r)) {
+  if (!bk_bins<EPT>(L, v, vm, (uint32_t)n, K, 2u * K <= (uint32_t)n, r)) {
     bk_refine<EPT>(L, RowRegs<EPT>{v, 4 * tid}, vm, (uint32_t)n, r, K, ~(uint32_t)(n - 1), ~0u);
     bk_emit_sorted(L, K, p.K, o);
     return;
@@ -1534,7 +1546,7 @@ __global__ void __launch_bounds__(TK_NT) topk_chunk_kernel(TopkChunkParams p) {
   float v[EPT];
   const uint32_t vm = bk_load<F16, EPT>(x, c0, c1, v);
   BkRange r;
-  if (!bk_bins<EPT>(L, v, vm, K, r)) {
+  if (!bk_bins<EPT>(L, v, vm, (uint32_t)(c1 - c0), K, 2u * K <= (uint32_t)(c1 - c0), r)) {
     bk_refine<EPT>(L, RowRegs<EPT>{v, c0 + 4 * tid}, vm, (uint32_t)(c1 - c0), r, K, ~(uint32_t)(c1 - 1), ~(uint32_t)c0);
     for (uint32_t i = tid; i < K; i += TK_NT) list[i] = L.list[i];
     if (tid == 0) ((uint32_t*)wr)[g] = K;
@@ -1586,9 +1598,9 @@ __global__ void __launch_bounds__(TK_NT) topk_lists_kernel(TopkChunkParams p) {
     v[i] = unkey((uint32_t)(e[i] >> 32));
   }
   BkRange r;
-  if (!bk_bins<EPT>(L, v, vm, K, r)) {
-    uint32_t have = 0u;
-    for (int g = 0; g < p.G; ++g) have += ((const uint32_t*)wr)[g];
+  uint32_t have = 0u;
+  for (int g = 0; g < p.G; ++g) have += ((const uint32_t*)wr)[g];
+  if (!bk_bins<EPT>(L, v, vm, have, K, false, r)) {
     bk_refine<EPT>(L, ListRegs<EPT>{e}, vm, have, r, K, ~(uint32_t)(n - 1), ~0u);
     bk_emit_sorted(L, K, p.K, o);
     return;

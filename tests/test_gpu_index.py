@@ -420,11 +420,11 @@ def test_topk_bucket_selection(dev, L, dtype):
         assert np.array_equal(kernels.topk(wide[:, 3:3 + L], dctx, K).cpu().numpy(), exp)
 
 
-@pytest.mark.parametrize("L", [300, 2500, 9000, 16001, 32768, 40000, 131072, 200001, 262144])
+@pytest.mark.parametrize("L", [300, 2500, 4096, 9000, 16001, 32768, 40000, 131072, 200001, 262144])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_topk_skewed_and_tied_rows(dev, L, dtype):
     """Rows whose values crowd at an end of their range (bins by key), or in few values (the K-th key's bin cut by key range
-    and by column): bit-exact against the oracle, at the edges of the keys per thread and of the chunks."""
+    and by column), or whose K-th value lies below the range that is binned: bit-exact against the oracle, at the edges of the keys per thread and of the chunks."""
     from arcagi2_flashnext_dots3_amd import kernels
     g = np.random.RandomState(L)
     x = (280 + 56 * g.randn(12, L)).astype(np.float32)
@@ -440,10 +440,18 @@ def test_topk_skewed_and_tied_rows(dev, L, dtype):
     x[9] = np.where(g.rand(L) < 0.3, np.nan, np.where(g.rand(L) < 0.3, np.inf, 7))
     x[10] = np.where(g.rand(L) < 0.5, -0.0, 0.0)
     x[11] = np.where(np.arange(L) % 3 == 0, 2 ** -20, 2 ** -21) * (1 if L % 2 else -1)
+    x = np.concatenate([x, np.empty((6, L), np.float32)])
+    j = np.arange(L)
+    x[12] = g.randn(L) / g.randn(L)                              # far values at both ends
+    x[13] = np.maximum(g.randn(L), 0) + 3                        # a floor, a cap
+    x[14] = np.minimum(g.randn(L), 0.3)
+    x[15] = g.randn(L) + 50 * (j % 4096 < 8)                     # the high values in few threads: the K-th lies below the
+    x[16] = g.randn(L) + 50 * ((j // 4) % 1024 < 40)             # threads' largest values
+    x[17] = -j
     lg = torch.from_numpy(x).to(dtype)
-    ctx = np.full(12, L, dtype=np.int32)
+    ctx = np.full(18, L, dtype=np.int32)
     dlg, dctx = lg.to(dev), torch.from_numpy(ctx).to(dev)
-    for K in (1, 257, 2048):
+    for K in (1, 257, min(2048, L // 2), 2048):
         print(f"[skewed] L={L} K={K} {dtype}", flush=True)
         exp = ref.topk(lg.numpy(), ctx, K)
         for single in (False, True):
