@@ -911,7 +911,7 @@ static int attn_launch(const void* q, long long q_st, long long q_sh, const void
   if (fused && ((K + S - 1) / S + attn::TR - 1) / attn::TR * attn::TR > attn::KMAX) return SPMLA_ELIMIT;   // (a limit kept
   // from the kernel that merged before; the head-group kernel has none)
   if (fused) {
-    S = rules::merged_splits(T, H, K, S);
+    S = rules::merged_splits(T, H, K, S, false);
     fused = S > 1;
   }
   if (fused || !attn_wide(T, H, K, S))
@@ -964,7 +964,7 @@ static int attn576_launch(const void* q, long long q_st, long long q_sh, const v
   if (out && (((uintptr_t)out & 7) || (o_st & 3) || (o_sh & 3))) return SPMLA_EALIGN;
   if (f32part && ((uintptr_t)opart & 15)) return SPMLA_EALIGN;
   if (fused) {
-    S = rules::merged_splits(T, H, K, S);
+    S = rules::merged_splits(T, H, K, S, true);
     fused = S > 1;
   }
   if (!fused && attn_wide(T, H, K, S))

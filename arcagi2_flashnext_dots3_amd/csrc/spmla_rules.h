@@ -22,25 +22,27 @@ inline bool attn_wide(int T, int H, int K, int S) {
   return 32 * tiles <= WIDE_ROWS && r32 * (102 + 6 * tiles) > 72 + r128 * (100 + 23 * tiles);
 }
 
-// Model (us) of a merged launch of s splits: ts = T * ceil(H / 32) workgroups a split; see the fit in kernels.py, whose
-// _split_cost this is.
-inline double split_cost(long long ts, int K, int s) {
+// Model (us) of a merged launch of s splits over Row656 or Row576 rows: ts = T * ceil(H / 32) workgroups a split; see the
+// fit in kernels.py, whose _split_cost this is.
+inline double split_cost(long long ts, int K, int s, bool r576) {
   const long long tiles = ((K + s - 1) / s + 31) / 32, wgs = ts * s;
-  const double merge = s == 1 ? 0.0 : (s == 2 ? 5.7 : s <= 4 ? 6.2 : 9.2) + 0.003 * (wgs > 128 ? wgs - 128 : 0);
-  return (double)((wgs + 255) / 256) * (10.4 + 2.15 * ((tiles + 3) / 4)) + merge;
+  const double m2 = r576 ? 4.0 : 3.0, m4 = r576 ? 5.0 : 3.6, m8 = r576 ? 7.3 : 6.0;
+  const double round = (r576 ? 10.8 : 11.5) + (r576 ? 1.81 : 2.13) * (double)((tiles + 3) / 4);
+  return (double)((wgs + 255) / 256) * round + (s == 1 ? 0.0 : s == 2 ? m2 : s <= 4 ? m4 : m8) +
+         0.013 * (double)(wgs < 256 ? wgs : 256);
 }
 
 // Splits of a merged launch that may take up to S. Up to one round of workgroups as many as are asked for: more are taken
 // only where they are faster. us of S splits of 128-head workgroups with f16 partials (the merge before this one) / S
 // splits of this kernel / what is chosen, 128 heads: T = 32, K = 2048, S = 8 60 / 79 / 38 (2); T = 64, K = 256, S = 4 34 / 58
 // / 18 (1); T = 200, K = 2048, S = 8 279 / 438 / 150 (1).
-inline int merged_splits(int T, int H, int K, int S) {
+inline int merged_splits(int T, int H, int K, int S, bool r576) {
   const long long ts = (long long)T * ((H + 31) / 32);
   if (ts * S <= 256) return S;
   if (2 * ts > 256) return 1;
   int best = 1;
   for (int s = 2; s <= S; ++s)
-    if (split_cost(ts, K, s) < split_cost(ts, K, best)) best = s;
+    if (split_cost(ts, K, s, r576) < split_cost(ts, K, best, r576)) best = s;
   return best;
 }
 

@@ -707,39 +707,42 @@ def attention_ok(q, idx):
 ATTN_SPLIT_ROWS = 2048      # most rows of one (token, split), in tiles of 32, that spmla_attn merges
 
 
-def _split_cost(n, K, s, cus):
+def _split_cost(n, K, s, cus, row_bytes=ROW656):
     """Model of a launch of n * s workgroups over K / s rows each (us): rounds of one workgroup per compute unit, each a
-    fixed part and the longest wave's 32-row tiles; the merge of the splits on top (its kernel is built for 2, 4 and 8).
-    Fitted to graphed launches (1 / 2 / 4 / 8 splits; 128 heads: K = 2048, T = 1 42 / 32 / 26 / 24 us, 16 46 / 35 / 29 / 49, 32
-    47 / 38 / 51 / 79; K = 1024, T = 16 29 / 26 / 25 / 44; K = 512, T = 8 20.0 / 20.6 / 19.7 / 23.7, T = 16 20.4 / 21.1 / 22.2 /
-    41.5; K = 640, T = 8 21.9 / 22.5 / 21.8 / 23.4; 32 heads, K = 512, T = 32 20.4 / 21.1 / 19.5 / 23.0; K = 384 16.2 / 18.5 /
-    17.9 / 20.1 and less for one launch at any T)."""
+    fixed part and the longest wave's 32-row tiles; the merge of the splits on top (its kernel is built for 2, 4 and 8) and
+    what the workgroups of a round take from each other. Fitted to 3100 graphed launches over rows of a 1M-row pool that no
+    cache holds (1 / 2 / 4 / 8 splits, Row656; 32 heads, K = 512, T = 8 20.4 / 19.2 / 18.2 / 20.4, T = 54 22.5 / 21.5 / 21.1 / -;
+    K = 1024, T = 8 28.6 / 23.8 / 21.4 / 21.9; K = 384, T = 32 19.6 / 20.1 / 18.7 / 21.8; 128 heads, K = 512, T = 16 22.0 / 21.0 /
+    22.3 / -. Row576: 32 heads, K = 512, T = 8 18.5 / 19.9 / 19.1 / 21.7, T = 54 20.1 / 21.9 / 22.1 / -; K = 1024, T = 8 25.4 / 23.9
+    / 21.9 / 23.1), merges half a us longer for the fill of the counters that captured launches add. The choice costs 0.7 % more
+    than the best of each on average, 11 % at most (16 heads, K = 384)."""
+    a, b, m = (10.8, 1.81, (4.0, 5.0, 7.3)) if row_bytes == ROW576 else (11.5, 2.13, (3.0, 3.6, 6.0))
     tiles = -(-(-(-K // s)) // 32)
-    merge = 0.0 if s == 1 else (5.7 if s == 2 else 6.2 if s <= 4 else 9.2) + 0.003 * max(0, n * s - 128)
-    return -(-n * s // cus) * (10.4 + 2.15 * -(-tiles // 4)) + merge
+    merge = 0.0 if s == 1 else m[0] if s == 2 else m[1] if s <= 4 else m[2]
+    return -(-n * s // cus) * (a + b * -(-tiles // 4)) + merge + 0.013 * min(n * s, cus)
 
 
 @functools.lru_cache(maxsize=4096)
-def _best_split(T, H, K, limit, cus):
+def _best_split(T, H, K, limit, cus, row_bytes):
     n = T * ((H + 31) // 32)
-    if 2 * n > cus or n == 0:
+    if 2 * n > cus or n == 0 or K <= 384:       # (3 or 4 splits of 384 rows gain a us where little else runs, or lose one)
         return 1
     fits = [s for s in range(1, 9) if s == 1 or limit is None or -(-(-(-K // s)) // 32) * 32 <= limit]
-    return min(fits, key=lambda s: (_split_cost(n, K, s, cus), s))
+    return min(fits, key=lambda s: (_split_cost(n, K, s, cus, row_bytes), s))
 
 
 def auto_split576(T, H, K, cus=256):
     """Row splits per token (merged in the kernel, at most 8). 1 when the unsplit launch has more than half as many
     workgroups of 32 heads as there are compute units: a second round would cost what the shorter lists save. Else the
     split of least _split_cost."""
-    return _best_split(T, H, K, None, cus)
+    return _best_split(T, H, K, None, cus, ROW576)
 
 
 def auto_split(T, H, K, cus=256):
     """auto_split576 for Row656 pools: of the splits of at most ATTN_SPLIT_ROWS rows each (spmla_attn takes no longer
     ones; unsplit any K, and it takes fewer splits where those are faster). 128 heads, us: K = 8192, 20 tokens 75, unsplit
     144; K = 12000, 12 / 23 tokens 70 / 121, unsplit 197 / 205."""
-    return _best_split(T, H, K, ATTN_SPLIT_ROWS, cus)
+    return _best_split(T, H, K, ATTN_SPLIT_ROWS, cus, ROW656)
 
 
 @functools.lru_cache(maxsize=4096)

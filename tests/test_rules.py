@@ -16,12 +16,12 @@ def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("rules")
     (d / "r.cpp").write_text('#include "spmla_rules.h"\n'
                              'extern "C" int wide(int T, int H, int K, int S) { return spmla::rules::attn_wide(T, H, K, S); }\n'
-                             'extern "C" double cost(long long n, int K, int s) { return spmla::rules::split_cost(n, K, s); }\n'
-                             'extern "C" int splits(int T, int H, int K, int S) { return spmla::rules::merged_splits(T, H, K, S); }\n')
+                             'extern "C" double cost(long long n, int K, int s, bool r) { return spmla::rules::split_cost(n, K, s, r); }\n'
+                             'extern "C" int splits(int T, int H, int K, int S, bool r) { return spmla::rules::merged_splits(T, H, K, S, r); }\n')
     subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", build.CSRC, str(d / "r.cpp"), "-o",
                     str(d / "r.so")], check=True, capture_output=True)
     L = ctypes.CDLL(str(d / "r.so"))
-    L.cost.restype, L.cost.argtypes = ctypes.c_double, [ctypes.c_longlong, ctypes.c_int, ctypes.c_int]
+    L.cost.restype, L.cost.argtypes = ctypes.c_double, [ctypes.c_longlong, ctypes.c_int, ctypes.c_int, ctypes.c_bool]
     return L
 
 
@@ -45,7 +45,8 @@ def test_split_cost_is_the_callers(lib):
     for n in (1, 4, 33, 100, 128):
         for K in (0, 40, 512, 2048, 12000):
             for i in range(1, 9):
-                assert lib.cost(n, K, i) == pytest.approx(kernels._split_cost(n, K, i, 256), abs=1e-9)
+                for rb in (kernels.ROW656, kernels.ROW576):
+                    assert lib.cost(n, K, i, rb == 576) == pytest.approx(kernels._split_cost(n, K, i, 256, rb), abs=1e-9)
 
 
 @pytest.mark.parametrize("T,H,K,S,chosen", [
@@ -55,6 +56,7 @@ def test_merged_splits_beyond_one_round(lib, T, H, K, S, chosen):
     """A merged launch of more than one round of workgroups takes the cheapest of up to S splits, which is what auto_split
     takes too."""
     from arcagi2_flashnext_dots3_amd import kernels
-    assert lib.splits(T, H, K, S) == chosen
+    for r576 in (False, True):
+        assert lib.splits(T, H, K, S, r576) == chosen
     if T * ((H + 31) // 32) * S > 256:
-        assert lib.splits(T, H, K, 8) == kernels.auto_split576(T, H, K)
+        assert lib.splits(T, H, K, 8, True) == kernels.auto_split576(T, H, K)
