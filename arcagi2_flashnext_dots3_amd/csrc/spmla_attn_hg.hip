@@ -1,20 +1,20 @@
 // Head-group attention: one workgroup of 4 waves per (work item, column group of 32, split); each wave streams its
 // own 32-row tiles (codes into a private LDS double buffer by direct global->LDS copies, rope straight into VGPRs)
-// and keeps its own online softmax, so the waves never wait for each other inside the loop. Two instances:
-//   * attn_kernel<false>, the decode kernel of spmla_attn / spmla_attn_splitk / spmla_attn_merge when a launch has
-//     few tokens (spmla_attn.hip chooses): work item = token, columns = 32 of its heads;
+// and keeps its own online softmax, so the waves never wait for each other inside the loop. attn_kernel<PACKED, R5, SP>
+// (request-packed, Row576 rows, splits merged in the kernel) in five instances:
+//   * attn_kernel<false, false>, Row656 launches without the split merge (spmla_rules.h chooses between it and the prefill
+//     kernel): work item = token, columns = 32 of its heads;
+//   * attn_kernel<false, true>, the same over Row576 rows (spmla_attn576: 512 + 64 e4m3 codes, one per-tensor
+//     kv_scale): no per-group scales, so the latent MFMAs run as one chain into S (no scale combine), P' is P itself in
+//     f16 for every group, and the rope codes are widened to bf16 (exact) in registers;
+//   * attn_kernel<false, *, true>, whose splits of a token's rows merge in the kernel (small batches: K = 2048, 128
+//     heads, 1 / 8 / 16 / 32 tokens 22.7 / 25.9 / 27.6 / 36.1 us, against 53 / 54 / 55 / 51 us for 128-head workgroups
+//     with f16 partials at up to 8 splits, or unsplit at 32 tokens). A launch that leaves compute units idle is bound by
+//     the serial chain of a wave (12.7 us of prologue and merge, 2.0 us per tile), so the rows go to more workgroups;
 //   * attn_kernel<true>, request-packed MTP decode (spmla_attn_packed) over the union rows of spmla_mtp_union: work
 //     item = request, columns = tokens x heads; a column's softmax keeps only the rows its token selected (per-row
 //     token masks, ballots). Reference: dotsnote/engine/arcstats_pkg/arcstats/csrc/offload_attn.cu:700-1153
 //     (pk_attn_kernel).
-//   * attn_kernel<false, *, true>, the decode kernel whose S splits of a token's rows merge in the kernel (small
-//     batches: K = 2048, 128 heads, 1 / 8 / 16 / 32 tokens 22.7 / 25.9 / 27.6 / 36.1 us, against 53 / 54 / 55
-//     / 51 us for 128-head workgroups with f16 partials at up to 8 splits, or unsplit at 32 tokens). A launch that
-//     leaves compute units idle is bound by the serial chain of a wave (12.7 us of prologue and merge, 2.0 us per
-//     tile), so the rows go to more workgroups;
-//   * attn_kernel<false, true>, the same decode over Row576 rows (spmla_attn576: 512 + 64 e4m3 codes, one
-//     per-tensor kv_scale): no per-group scales, so the latent MFMAs run as one chain into S (no scale combine), P'
-//     is P itself in f16 for every group, and the rope codes are widened to bf16 (exact) in registers.
 //
 // Math (reference: dotsnote/kaggle/runtime_dataset/bench_offload_attn2.py:77-93 and
 // dotsnote/engine/vllm_patch/vllm/v1/attention/ops/xpu_mla_sparse.py:77-161):

@@ -16,8 +16,8 @@
 //   (-0 < +0, NaN largest); equal keys -> lower column first; output positions sorted by (value desc, column asc),
 //   -1 where the value is +-inf and in slots >= n. fp32 or fp16 logits: an fp16 key is the same order key of the
 //   16-bit pattern placed in the top half of the 32-bit key (low half zero), so one radix code serves both.
-//   gfx950: rows of up to 32768 columns, and up to 8 such chunks of a row, are selected and sorted by bins of equal
-//   width (topk_row_kernel, topk_chunk_kernel). Longer rows, and the two stages of the rank-sharded selection, go
+//   gfx950: rows of up to 32768 columns, and up to 8 such chunks of a row, are selected and sorted by 4096 bins of the
+//   value or the key (topk_row_kernel, topk_chunk_kernel). Longer rows, and the two stages of the rank-sharded selection, go
 //   through 11/11/10-bit radix levels with an LDS histogram; keys above the boundary bin are appended at slots from a
 //   block scan of per-thread counts (wave scans on DPP); once the boundary bin holds at most the candidate cap the
 //   remaining levels run on those candidates alone; ties on the final key take the lowest columns. The K winners are
@@ -1156,8 +1156,8 @@ __global__ void __launch_bounds__(TK_NT) topk_kernel(TopkParams p) {
 // sort: 4 rows of 16000 columns 9.8 us (32.7), 64 of 32768 15.3 us (39.0), 2048 of 16384 55.6 us (356).
 // Where the high values crowd at the low end of the range (far outliers, skewed distributions) the bins are of the key's
 // integer instead, which spaces them by magnitude. A row whose bins from the K-th key's on still hold more than BK_LIM
-// entries somewhere (heavy ties, no finite value) has the K-th key's bin cut further (bk_refine). Below 128 entries a bin
-// is ranked by counting faster than a whole row (K = n) is sorted, and above slower (2048 of 25 distinct values 19 / 25 us).
+// entries somewhere (heavy ties, no finite value) has the K-th key's bin cut further (bk_refine). A whole row (K = n) needs
+// no cut, only the sort, which is faster from 128 entries a bin on (512 rows of 2048 with 25 distinct values 36 -> 23 us).
 constexpr int BK_BINS = 4096;
 constexpr int BK_LIM = 256;                  // entries of a bin that are ranked by counting
 constexpr int BK_LIST = TK_KMAX + BK_LIM;    // entries from the K-th key's bin on
@@ -1649,7 +1649,8 @@ struct TopkWs {
 __host__ inline TopkWs topk_ws_layout(int Lc) {
   TopkWs w;
   // chunks of 8192 columns, at most 4 per row (every collect workgroup reads all G histograms of its row; with
-  // 8 chunks at 131072 columns the passes took 69.6 us against 58.8 with 4, B = 64)
+  // 8 chunks at 131072 columns the passes took 69.6 us against 58.8 with 4, B = 64). The passes run above 262144
+  // columns; below, the layout only gives the limits of spmla_topk_scratch and spmla_index_logits_hist.
   int G = (Lc + 8191) / 8192;
   if (G > 4) G = 4;
   if (G < 1) G = 1;
@@ -2036,7 +2037,7 @@ static void topk_ws_passes(TopkWsParams p, hipStream_t stream) {
 
 using namespace spmla;
 
-// Logits grid: one 12-wave workgroup per CU. With at most as many rows as CUs, each row's tiles are split over
+// Logits grid: one 8-wave workgroup per CU. With at most as many rows as CUs, each row's tiles are split over
 // CUs / rows workgroups, one round of the whole grid (a wave pays its two-round-trip prologue, ~6 us under load,
 // once); with more rows, workgroups of LG_TPW tiles per wave, rounds fine enough for a short tail.
 inline int lg_cus() {
@@ -2140,7 +2141,7 @@ int spmla_index_logits_hist(const void* q, long long q_st, long long q_sh, const
   if (rows == 0 || Lc == 0) return SPMLA_OK;
   const idx::TopkWs tw = idx::topk_ws_layout(Lc);
   if (!topk_ws || ((uintptr_t)topk_ws & 15) || ws_bytes < rows * topk_ws_row(Lc)) return SPMLA_EARG;
-  if (tw.CL >= 65536) return SPMLA_ELIMIT;                  // longer rows: use the separate calls
+  if (tw.CL >= 65536) return SPMLA_ELIMIT;                  // (kept from 16-bit histogram counts, as the workspace check)
   return logits_row(q, q_st, q_sh, w, w_st, store, R_local, rows_per_block, block_stride, block_table, bt_st,
                     block_size, req, ctx, rows, H, D, Lc, 1, 0, noinf, out, out_st, out_dtype, stream, 1);
 }

@@ -482,7 +482,7 @@ def run_config4(a, dev):
                               dst.data_ptr(), dst.stride(0), int(dst.dtype == torch.float16), kernels._stream(q))
 
         # eager (host dispatch from Python included) and from HIP graphs of 20 launches (the launches alone;
-        # the top-k is four kernels per call)
+        # the top-k is two kernels per call above 32768 columns)
         ms_l = _graph_ms(logits, a.steps, a.warmup, reps=20)
         ms_t = _graph_ms(lambda: kernels.topk(lg, ctx, K, out=out), a.steps, a.warmup, reps=20)
         ms_l_eager = _timed(logits, a.steps, a.warmup)      # after the graph timings, at their settled clocks

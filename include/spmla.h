@@ -85,8 +85,9 @@ int spmla_topk_ws(const void* logits, long long lg_st, const int* ctx, int rows,
 
 /* spmla_index_logits (P = 1, rank 0) for a top-k over the same rows, Lc and ctx that follows with workspace topk_ws
  * (spmla_topk_ws_bytes(rows, Lc, K) bytes, 16-byte aligned): columns j < min(ctx[row], Lc) whose key has no block-table
- * entry are written -inf even with noinf != 0 (they are top-k columns). The workspace is left as it is (the selection
- * needs no histogram of the logits). SPMLA_ELIMIT for Lc above 4 x 64512: use spmla_index_logits and spmla_topk_ws.
+ * entry are written -inf even with noinf != 0 (they are top-k columns). The selection needs no histogram of the logits:
+ * the workspace is checked and left as it is, and SPMLA_ELIMIT for Lc above 4 x 64512 (then spmla_index_logits and
+ * spmla_topk_ws) is the contract of the time when histograms of 16-bit counts were built in it.
  * The reference computes the logits and then selects in separate calls (shard_indexer.py:63-91 then
  * fast_topk.py:52-78 / csrc/topk_select.cu:75-201 at P = 1, shard_indexer.py:194-221). */
 int spmla_index_logits_hist(const void* q, long long q_st, long long q_sh, const float* w, long long w_st,
@@ -336,12 +337,6 @@ int spmla_attn576_ws(const void* q, long long q_st, long long q_sh, const void* 
                      void* out, long long o_st, long long o_sh, float* lse, long long lse_st, void* ws,
                      long long ws_bytes, void* stream);
 
-/* spmla_attn_splitk (S = 1) whose result is merged with a prior partial of the same tokens and heads before the bf16
- * write: prior_o [T][H][512] fp32 normalized (strides po_st, po_sh; 16-byte aligned), prior_lse [T][H] (stride
- * pl_st, natural log). out = w o + w' prior_o with w = e^lse / (e^lse + e^lse'), w' = e^lse' / (e^lse + e^lse'),
- * lse_out = ln(e^lse + e^lse'); both -inf -> o = 0, lse = -inf. The host-tier attention of a decode step merges the
- * HBM tier's partial this way, in place of spmla_lse_merge over two partials (the reference's tier combine,
- * dotsnote/engine/arcstats_pkg/arcstats/sparse_offload.py:519-538, fused into the second tier's kernel). */
 /* spmla_attn (row_bytes 656) or spmla_attn576 / spmla_attn576_ws (576) over the pages of a cache: topk[t][k] are positions
  * of token t's request, formed into rows as spmla_rows_from_topk does (block_size a power of two, else SPMLA_ELIMIT;
  * bt_cols >= 1), in the attention kernel. req[t] is read for every token (any value where the token has no position in
@@ -352,6 +347,12 @@ int spmla_attn_paged(const void* q, long long q_st, long long q_sh, const void* 
                      int S, void* out, long long o_st, long long o_sh, float* lse, long long lse_st, void* ws,
                      long long ws_bytes, void* stream);
 
+/* spmla_attn_splitk (S = 1) whose result is merged with a prior partial of the same tokens and heads before the bf16
+ * write: prior_o [T][H][512] fp32 normalized (strides po_st, po_sh; 16-byte aligned), prior_lse [T][H] (stride
+ * pl_st, natural log). out = w o + w' prior_o with w = e^lse / (e^lse + e^lse'), w' = e^lse' / (e^lse + e^lse'),
+ * lse_out = ln(e^lse + e^lse'); both -inf -> o = 0, lse = -inf. The host-tier attention of a decode step merges the
+ * HBM tier's partial this way, in place of spmla_lse_merge over two partials (the reference's tier combine,
+ * dotsnote/engine/arcstats_pkg/arcstats/sparse_offload.py:519-538, fused into the second tier's kernel). */
 int spmla_attn_merge(const void* q, long long q_st, long long q_sh, const void* pool, long long R, const int* idx,
                      long long idx_st, int K, const int* kcount, int T, int H, float sm_scale, float kv_scale,
                      const float* prior_o, long long po_st, long long po_sh, const float* prior_lse, long long pl_st,

@@ -250,8 +250,7 @@ def test_logits_then_topk_end_to_end(dev):
 
 @pytest.mark.parametrize("dtype,noinf", [(torch.float32, False), (torch.float16, False), (torch.float32, True)])
 def test_logits_hist_topk_matches_separate(dev, dtype, noinf):
-    """The first-level top-k histogram built in the logits epilogue (spmla_index_logits_hist, then
-    spmla_topk_ws_prehist) against the separate calls on the same inputs: identical logits bit for bit and identical
+    """The step's pair of calls (spmla_index_logits_hist, then spmla_topk_ws_prehist) against the separate calls on the same inputs: identical logits bit for bit and identical
     positions, which are also the oracle's top-k of those logits. Rows with ctx below Lc (a short last chunk, ctx 0,
     ctx <= K), indexer-like concentrated values on some rows, and (noinf False) a block-table entry missing inside
     ctx, whose keys both paths write as -inf."""
